@@ -1,0 +1,49 @@
+"""Kernels whose launch shape follows the size, at the sizes where the shape
+changes: tile edges, remainders, the smallest and largest of each range."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from conftest import crandn, rel
+from gpu_util import Dev, init
+
+pytestmark = pytest.mark.gpu
+V, I64 = ctypes.c_void_p, ctypes.c_int64
+EPS = 2.2e-16
+
+
+@pytest.fixture(scope="module")
+def L(pkg):
+    return init(pkg)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 15, 16, 17, 32, 33, 48, 49, 63, 64])
+@pytest.mark.parametrize("rank_def", [False, True])
+def test_jacobi_svd_sizes(L, pkg, n, rank_def):
+    """Singular values against numpy, U orthonormal and diagonalising R R^H
+    (a graded spectrum over four decades; with a zero column when rank_def)."""
+    rng = np.random.default_rng(n)
+    nb = 3
+    s = 10.0 ** (-4.0 * (np.arange(n) + 0.3 * rng.random((nb, n))) / n)
+    R = np.stack([np.triu(np.linalg.qr((np.linalg.qr(crandn(rng, n, n))[0] * s[b]) @ crandn(rng, n, n))[1])
+                  for b in range(nb)])
+    if rank_def:
+        R[:, :, n // 2] = 0
+    dR, dU, ds = Dev(pkg, R), Dev(pkg, nbytes=R.nbytes), Dev(pkg, nbytes=nb * n * 8)
+    L.rsvdt_hip_bjacobi_svd.argtypes = [I64, I64, V, V, V, V]
+    assert L.rsvdt_hip_bjacobi_svd(nb, n, dR.p, dU.p, ds.p, None) == 0
+    U, sg = dU.get(np.complex128, R.shape), ds.get(np.float64, (nb, n))
+    tol = 40 * n * EPS
+    for b in range(nb):
+        ref = np.linalg.svd(R[b], compute_uv=False)
+        top = max(ref[0], 1e-300)
+        assert np.max(np.abs(sg[b] - ref)) <= tol * top
+        live = sg[b] > tol * top
+        Ul = U[b][:, live]
+        assert np.max(np.abs(Ul.conj().T @ Ul - np.eye(live.sum())), initial=0.0) <= tol
+        D = Ul.conj().T @ (R[b] @ R[b].conj().T) @ Ul
+        assert np.max(np.abs(D - np.diag(sg[b][live] ** 2)), initial=0.0) <= tol * top * top
+        t = Ul.sum(axis=0)
+        big = np.abs(t) > 1e-7
+        assert np.all(t.real[big] > 0) and np.all(np.abs(t.imag[big]) <= tol * np.sqrt(n))
