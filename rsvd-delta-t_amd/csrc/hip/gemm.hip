@@ -27,6 +27,7 @@ namespace rsvdt {
 // reused for every 64-column tile the workgroup visits (grid-stride), so
 // `in` is streamed from HBM exactly once per row range.
 typedef double dvec4 __attribute__((ext_vector_type(4)));
+typedef double dvec2 __attribute__((ext_vector_type(2)));
 
 template <int T, typename OV>
 __global__ __launch_bounds__(256) void k_coef_gemm(
@@ -184,142 +185,303 @@ __global__ __launch_bounds__(256) void k_bgram_part(
     if (a < na && c < nc) part[((b * nch + blockIdx.x) * na + a) * nc + c] = acc;
 }
 
-__global__ void k_bgram_reduce(int64_t nbatch, int64_t nch, int64_t na, int64_t nc,
-                               const double2 *__restrict__ part, double2 *__restrict__ G)
+// G_b(a, c) = sum over the nch partial matrices of batch b, in a fixed order:
+// 32 entries x 8 slices of the partials per workgroup, the slices' sums
+// combined through LDS.  One thread per entry walking all partials was a
+// serial chain of loads (165 us for 16 batches of 512 partials of 16 x 16).
+// herm: the tiles below the diagonal (and the border row) were not formed and
+// are the conjugates of their mirrors; ntile: the 16-wide tiles (columns from
+// 16 ntile on are the border).
+__global__ __launch_bounds__(256) void k_bgram_reduce(int64_t nch, int na, int nc, int herm, int ntile,
+                                                      const double2 *__restrict__ part, double2 *__restrict__ G)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t per = na * nc;
-    if (i >= nbatch * per) return;
-    const int64_t b = i / per, e = i % per;
+    __shared__ double2 sh[8][32];
+    const int64_t b = blockIdx.y;
+    const int64_t per = (int64_t)na * nc;
+    const int64_t e = (int64_t)blockIdx.x * 32 + (int)(threadIdx.x & 31);
+    const int sl = threadIdx.x >> 5;
     double2 s = make_double2(0, 0);
-    for (int64_t ch = 0; ch < nch; ++ch) {
-        const double2 v = part[(b * nch + ch) * per + e];
-        s.x += v.x; s.y += v.y;
+    bool mir = false;
+    if (e < per) {
+        const int a = (int)(e / nc), c = (int)(e % nc);
+        const int ta = min(a / 16, ntile), tc = min(c / 16, ntile);
+        mir = herm && ta > tc;
+        const double2 *p = part + b * nch * per + (mir ? (int64_t)c * nc + a : e);
+        for (int64_t ch = sl; ch < nch; ch += 8) {
+            const double2 v = p[ch * per];
+            s.x += v.x; s.y += v.y;
+        }
     }
-    G[i] = s;
+    sh[sl][threadIdx.x & 31] = s;
+    __syncthreads();
+    if (sl == 0 && e < per) {
+#pragma unroll
+        for (int q = 1; q < 8; ++q) { s.x += sh[q][threadIdx.x].x; s.y += sh[q][threadIdx.x].y; }
+        G[b * per + e] = make_double2(s.x, mir ? -s.y : s.y);
+    }
 }
 
 // FP64 MFMA Gram for unit column strides (rows of X and Z contiguous, the
-// per-batch row-major layout).  A wave computes a (16 TA) x (16 TC) tile of
-// G = X^H Z over its share of a row chunk, complex as four real products:
+// per-batch row-major layout).  A workgroup forms a (16 TA) x (16 TC) macro
+// tile of G = X^H Z over a row chunk, complex as four real products:
 //   Re G += Xr Zr + Xi Zi,   Im G += Xr Zi - Xi Zr.
 // A(16x4): lane i -> X(r0 + i/16, a0 + i%16); B(4x16): lane i -> Z(r0 + i/16,
 // c0 + i%16); D: lane i holds G(a0 + 4j + i/16, c0 + i%16), j < 4.
-// nsub waves of a workgroup share one tile and split its 4-row steps (small
-// Grams); otherwise the 4 waves take 4 tiles.  Each (chunk, sub) writes a
-// full partial that k_bgram_reduce sums.  The next step's operands are loaded
-// before the current step's MFMAs.
-template <int TA, int TC>
-__global__ __launch_bounds__(256) void k_bgram_mfma(
-    int64_t nrows, int64_t na, int64_t nc, int64_t chunk, int ntc, int ntiles, int nsub,
-    const double2 *__restrict__ X, int64_t xb, int64_t xr, const double2 *__restrict__ Z, int64_t zb, int64_t zr,
-    double2 *__restrict__ part)
+// The four waves take every fourth 4-row step and the whole macro tile each,
+// or, for 4 x 4 tiles (256 accumulator registers would not leave room for the
+// operands), every other step and half of the tile's rows (GA = 2).  Their
+// sums are combined through LDS in a fixed order and the chunk's partial goes
+// to k_bgram_reduce.
+// What bounds it: FP64 MFMA for n above 16, memory for one tile.  Hence
+//   * BORD: n = 16 T + 1 columns (the Nw + 1 snapshots of a removal) keep T
+//     tiles; the one border column and row are plain FMAs on the operands
+//     the lanes hold anyway (for n = 65: 16 MFMA tiles instead of 25);
+//   * HERM: X and Z the same array (CholeskyQR) forms the upper tiles only;
+//   * PF row steps are in flight per wave where the MFMAs of a step do not
+//     cover a load's latency; the loads are branch-free (clamped addresses,
+//     zeros selected afterwards).
+// 8 batches of 98,304 x 65 (V^H X of a removal): 508 us, 52 TFLOP/s (48 x 48
+// tiles per wave, padded to 96 x 96: 1620 us).  16 batches of 393,216 x 16
+// (QR): 329 us, 4.9 TB/s, with nontemporal loads and 8 steps in flight; 351 us
+// without the hint, 377 us with one step in flight.  The launch bound keeps
+// two waves per SIMD for half tiles (742 us with one).
+template <int TA, int TC, bool HERM, bool BORD>
+__global__ __launch_bounds__(256, TA *TC <= 1 ? 4 : (TA == 4 && !HERM ? 2 : 1)) void k_bgram_mfma(
+    int64_t nrows, int na, int nc, int64_t chunk, int ntc, const double2 *X, int64_t xb, int64_t xr,
+    const double2 *Z, int64_t zb, int64_t zr, double2 *__restrict__ part)
 {
+    constexpr int GA = TA == 4 && !HERM ? 2 : 1, WA = TA / GA, NSUB = 4 / GA;
+    constexpr int PF = TA * TC == 1 ? (HERM ? 8 : 4) : (WA * TC <= 4 ? 2 : 1);
+    constexpr int CW = 16 * TC, RS = 4 * NSUB;   // columns of the macro tile; rows of the workgroup's step
+    extern __shared__ double2 gsm[];             // 16 TA x 16 TC, then the borders: 16 TA, 16 TC, 1
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int tile = blockIdx.y * (4 / nsub) + wv / nsub;
-    const int sub = wv % nsub;
-    if (tile >= ntiles) return;
+    const int h = wv % GA, sub = wv / GA;
     const int64_t b = blockIdx.z;
-    const int64_t a0 = (int64_t)(tile / ntc) * (16 * TA), c0 = (int64_t)(tile % ntc) * (16 * TC);
+    const int a0 = (int)(blockIdx.y / ntc) * (16 * TA), c0 = (int)(blockIdx.y % ntc) * CW;
+    const int aw = a0 + 16 * WA * h;             // first row of G of this wave
     const int64_t r_begin = (int64_t)blockIdx.x * chunk;
-    int64_t r_end = r_begin + chunk;
-    if (r_end > nrows) r_end = nrows;
-    const double2 *Xb = X + b * xb;
-    const double2 *Zb = Z + b * zb;
+    const int64_t r_end = r_begin + chunk < nrows ? r_begin + chunk : nrows;
     const int kr = lane >> 4, cl = lane & 15;
-    bool aok[TA], cok[TC];
+    // the macro tiles of the last row and column of tiles carry the border
+    const bool do_a = BORD && !HERM && a0 + 16 * TA >= na - 1, do_c = BORD && c0 + CW >= nc - 1;
+    const int na_t = BORD ? na - 1 : na, nc_t = BORD ? nc - 1 : nc;
+    bool aok[WA], cok[TC];
+    int ao[WA], co[TC];                          // column offsets, clamped
 #pragma unroll
-    for (int t = 0; t < TA; ++t) aok[t] = a0 + 16 * t + cl < na;
+    for (int t = 0; t < WA; ++t) {
+        aok[t] = aw + 16 * t + cl < na_t;
+        ao[t] = aok[t] ? aw + 16 * t + cl : na_t - 1;
+    }
 #pragma unroll
-    for (int u = 0; u < TC; ++u) cok[u] = c0 + 16 * u + cl < nc;
-    dvec4 gr[TA][TC], gi[TA][TC];
+    for (int u = 0; u < TC; ++u) {
+        cok[u] = c0 + 16 * u + cl < nc_t;
+        co[u] = cok[u] ? c0 + 16 * u + cl : nc_t - 1;
+    }
+    dvec4 gr[WA][TC], gi[WA][TC];
 #pragma unroll
-    for (int t = 0; t < TA; ++t)
+    for (int t = 0; t < WA; ++t)
 #pragma unroll
         for (int u = 0; u < TC; ++u) { gr[t][u] = (dvec4){0, 0, 0, 0}; gi[t][u] = (dvec4){0, 0, 0, 0}; }
-    const double2 zero = make_double2(0, 0);
-    double2 xv[TA], zv[TC];
-    int64_t r0 = r_begin + 4 * sub;
-    {
-        const int64_t r = r0 + kr;
-        const bool rok = r < r_end;
+    double2 ba[WA], bc[TC], bb = make_double2(0, 0);   // border column G(a, nc-1), border row G(na-1, c), corner
 #pragma unroll
-        for (int t = 0; t < TA; ++t) xv[t] = (rok && aok[t]) ? Xb[r * xr + a0 + 16 * t + cl] : zero;
+    for (int t = 0; t < WA; ++t) ba[t] = make_double2(0, 0);
 #pragma unroll
-        for (int u = 0; u < TC; ++u) zv[u] = (rok && cok[u]) ? Zb[r * zr + c0 + 16 * u + cl] : zero;
-    }
-    for (; r0 < r_end; r0 += 4 * nsub) {
-        double2 xn[TA], zn[TC];
-        const int64_t r = r0 + 4 * nsub + kr;
-        const bool rok = r < r_end;
+    for (int u = 0; u < TC; ++u) bc[u] = make_double2(0, 0);
+    double2 xv[PF][WA], zv[PF][TC], xe[PF], ze[PF];
+    bool okv[PF];
+    const double2 *Xb = X + b * xb, *Zb = Z + b * zb;
+    auto load = [&](int p, int64_t r0) {
+        int64_t r = r0 + kr;
+        okv[p] = r < r_end;
+        if (!okv[p]) r = r_end - 1;
+        const double2 *xp = Xb + r * xr;
 #pragma unroll
-        for (int t = 0; t < TA; ++t) xn[t] = (rok && aok[t]) ? Xb[r * xr + a0 + 16 * t + cl] : zero;
+        for (int t = 0; t < WA; ++t) {
+            if constexpr (TA * TC == 1 && HERM) {
+                const dvec2 v = __builtin_nontemporal_load((const dvec2 *)(xp + ao[t]));
+                xv[p][t] = make_double2(v.x, v.y);
+            } else xv[p][t] = xp[ao[t]];
+        }
+        if constexpr (!HERM) {
+            const double2 *zp = Zb + r * zr;
 #pragma unroll
-        for (int u = 0; u < TC; ++u) zn[u] = (rok && cok[u]) ? Zb[r * zr + c0 + 16 * u + cl] : zero;
+            for (int u = 0; u < TC; ++u) zv[p][u] = zp[co[u]];
+            if constexpr (BORD) { ze[p] = zp[nc - 1]; xe[p] = xp[na - 1]; }
+        } else if constexpr (BORD) {
+            ze[p] = xp[na - 1];
+        }
+    };
+    const int64_t rw = r_begin + 4 * sub;
 #pragma unroll
-        for (int t = 0; t < TA; ++t)
+    for (int p = 0; p < PF; ++p) load(p, rw + RS * p);
+    for (int64_t r0 = rw; r0 < r_end; r0 += RS * PF) {
+#pragma unroll
+        for (int p = 0; p < PF; ++p) {
+            double2 x[WA], z[TC], xb1 = make_double2(0, 0), zb1 = make_double2(0, 0);
+#pragma unroll
+            for (int t = 0; t < WA; ++t) {
+                const bool ok = okv[p] && aok[t];
+                x[t] = make_double2(ok ? xv[p][t].x : 0.0, ok ? xv[p][t].y : 0.0);
+            }
 #pragma unroll
             for (int u = 0; u < TC; ++u) {
-                gr[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[t].x, zv[u].x, gr[t][u], 0, 0, 0);
-                gr[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[t].y, zv[u].y, gr[t][u], 0, 0, 0);
-                gi[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[t].x, zv[u].y, gi[t][u], 0, 0, 0);
-                gi[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(-xv[t].y, zv[u].x, gi[t][u], 0, 0, 0);
+                if constexpr (HERM) z[u] = x[u];
+                else {
+                    const bool ok = okv[p] && cok[u];
+                    z[u] = make_double2(ok ? zv[p][u].x : 0.0, ok ? zv[p][u].y : 0.0);
+                }
             }
+            if constexpr (BORD) {
+                zb1 = make_double2(okv[p] ? ze[p].x : 0.0, okv[p] ? ze[p].y : 0.0);
+                if constexpr (HERM) xb1 = zb1;
+                else xb1 = make_double2(okv[p] ? xe[p].x : 0.0, okv[p] ? xe[p].y : 0.0);
+            }
+            load(p, r0 + RS * (p + PF));         // rows past the chunk count as zeros
 #pragma unroll
-        for (int t = 0; t < TA; ++t) xv[t] = xn[t];
+            for (int t = 0; t < WA; ++t)
 #pragma unroll
-        for (int u = 0; u < TC; ++u) zv[u] = zn[u];
+                for (int u = HERM ? t : 0; u < TC; ++u) {
+                    gr[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t].x, z[u].x, gr[t][u], 0, 0, 0);
+                    gi[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t].x, z[u].y, gi[t][u], 0, 0, 0);
+                }
+#pragma unroll
+            for (int t = 0; t < WA; ++t)
+#pragma unroll
+                for (int u = HERM ? t : 0; u < TC; ++u) {
+                    gr[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t].y, z[u].y, gr[t][u], 0, 0, 0);
+                    gi[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(-x[t].y, z[u].x, gi[t][u], 0, 0, 0);
+                }
+            if constexpr (BORD) {
+                if (do_c) {
+#pragma unroll
+                    for (int t = 0; t < WA; ++t) ba[t] = zadd(ba[t], zcmul(x[t], zb1));
+                }
+                if (do_a && h == 0) {
+#pragma unroll
+                    for (int u = 0; u < TC; ++u) bc[u] = zadd(bc[u], zcmul(xb1, z[u]));
+                }
+                bb = zadd(bb, zcmul(xb1, zb1));
+            }
+        }
     }
-    const int64_t nchs = (int64_t)gridDim.x * nsub;
-    const int64_t ch = (int64_t)blockIdx.x * nsub + sub;
-    double2 *pb = part + (b * nchs + ch) * na * nc;
+    // the waves' sums, in a fixed order
+    double2 *sba = gsm + 16 * TA * CW, *sbc = sba + 16 * TA;
+    if constexpr (BORD) {                         // sum the four row classes of a step
+        auto rsum = [](double2 v) {
+            v.x += __shfl_xor(v.x, 16, 64); v.y += __shfl_xor(v.y, 16, 64);
+            v.x += __shfl_xor(v.x, 32, 64); v.y += __shfl_xor(v.y, 32, 64);
+            return v;
+        };
 #pragma unroll
-    for (int t = 0; t < TA; ++t)
+        for (int t = 0; t < WA; ++t) ba[t] = rsum(ba[t]);
 #pragma unroll
-        for (int u = 0; u < TC; ++u)
+        for (int u = 0; u < TC; ++u) bc[u] = rsum(bc[u]);
+        bb = rsum(bb);
+    }
+#pragma unroll 1
+    for (int w = 0; w < NSUB; ++w) {
+        if (sub == w) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int64_t a = a0 + 16 * t + 4 * j + kr, c = c0 + 16 * u + cl;
-                if (a < na && c < nc) pb[a * nc + c] = make_double2(gr[t][u][j], gi[t][u][j]);
+            for (int t = 0; t < WA; ++t) {
+#pragma unroll
+                for (int u = HERM ? t : 0; u < TC; ++u)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        double2 *o = gsm + (16 * (WA * h + t) + 4 * j + kr) * CW + 16 * u + cl;
+                        double2 v = make_double2(gr[t][u][j], gi[t][u][j]);
+                        if (w) v = zadd(*o, v);
+                        *o = v;
+                    }
+                __builtin_amdgcn_sched_barrier(0);      // one tile row's sums in registers at a time
             }
+            if constexpr (BORD) {
+                if (kr == 0) {
+#pragma unroll
+                    for (int t = 0; t < WA; ++t) {
+                        double2 *o = sba + 16 * (WA * h + t) + cl;
+                        *o = w ? zadd(*o, ba[t]) : ba[t];
+                    }
+                    if (h == 0) {
+#pragma unroll
+                        for (int u = 0; u < TC; ++u) sbc[16 * u + cl] = w ? zadd(sbc[16 * u + cl], bc[u]) : bc[u];
+                        if (cl == 0) sbc[CW] = w ? zadd(sbc[CW], bb) : bb;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    }
+    double2 *pb = part + (b * gridDim.x + blockIdx.x) * (int64_t)na * nc;
+    for (int e = threadIdx.x; e < 16 * TA * CW; e += 256) {
+        const int a = e / CW, c = e % CW;
+        if (HERM && a / 16 > c / 16) continue;
+        if (a0 + a < na_t && c0 + c < nc_t) pb[(int64_t)(a0 + a) * nc + c0 + c] = gsm[e];
+    }
+    if constexpr (BORD) {
+        const int e = threadIdx.x;
+        if (do_c && e < 16 * TA && a0 + e < na_t) pb[(int64_t)(a0 + e) * nc + nc - 1] = sba[e];
+        if (do_a && e < CW && c0 + e < nc_t) pb[(int64_t)(na - 1) * nc + c0 + e] = sbc[e];
+        if (do_c && (do_a || HERM) && e == 0) pb[(int64_t)(na - 1) * nc + nc - 1] = sbc[CW];
+    }
 }
 
-// Tile shape of the MFMA Gram: 16/32/48 columns per wave side.
-static int bgram_tside(int64_t n) { return n <= 16 ? 1 : (n <= 32 ? 2 : 3); }
-
-struct bgram_mfma_plan {
-    int TA, TC, ntc, ntiles, nsub;
-    int64_t chunk, nch;
-};
-
-static bgram_mfma_plan bgram_mfma_shape(int64_t nbatch, int64_t nrows, int64_t na, int64_t nc)
+// Partials that rsvdt_hip_bgram_work_bytes has room for (the plans below use
+// at most as many): about 2048 workgroups of four tiles of up to 48 x 48.
+static int64_t bgram_work_parts(int64_t nbatch, int64_t nrows, int64_t na, int64_t nc)
 {
-    bgram_mfma_plan p;
-    p.TA = bgram_tside(na);
-    p.TC = bgram_tside(nc);
-    const int64_t nta = (na + 16 * p.TA - 1) / (16 * p.TA);
-    p.ntc = (int)((nc + 16 * p.TC - 1) / (16 * p.TC));
-    p.ntiles = (int)(nta * p.ntc);
-    p.nsub = p.ntiles >= 4 ? 1 : (p.ntiles >= 2 ? 2 : 4);
-    const int64_t wg_per_chunk = ((p.ntiles + (4 / p.nsub) - 1) / (4 / p.nsub)) * nbatch;
-    int64_t nch = (2048 + wg_per_chunk - 1) / wg_per_chunk;
-    if (nch < 1) nch = 1;
+    auto side = [](int64_t n) { return n <= 16 ? 16 : (n <= 32 ? 32 : 48); };
+    const int64_t ntiles = ((na + side(na) - 1) / side(na)) * ((nc + side(nc) - 1) / side(nc));
+    const int64_t nsub = ntiles >= 4 ? 1 : (ntiles >= 2 ? 2 : 4);
+    const int64_t wg_per_chunk = ((ntiles + (4 / nsub) - 1) / (4 / nsub)) * nbatch;
+    const int64_t nch = (2048 + wg_per_chunk - 1) / wg_per_chunk;
     int64_t chunk = (nrows + nch - 1) / nch;
     if (chunk < 64) chunk = 64;
     chunk = (chunk + 3) / 4 * 4;
+    return (nrows + chunk - 1) / chunk * nsub;
+}
+
+struct bgram_mfma_plan {
+    int TA, TC, ntc, ntiles, bord, herm;
+    int64_t chunk, nch;
+};
+
+// Macro tiles of at most 4 x 4 MFMA tiles, as even as the tile counts allow;
+// row chunks so that the grid holds two workgroups per SIMD's worth of waves
+// for the large tiles (one fits at a time) and eight per CU for a single tile,
+// which needs the loads of many waves in flight.
+static bgram_mfma_plan bgram_mfma_shape(int64_t nbatch, int64_t nrows, int64_t na, int64_t nc, bool herm)
+{
+    bgram_mfma_plan p;
+    p.bord = na > 16 && nc > 16 && na % 16 == 1 && nc % 16 == 1;
+    const int ta = (int)(p.bord ? na / 16 : (na + 15) / 16), tc = (int)(p.bord ? nc / 16 : (nc + 15) / 16);
+    const int ma = (ta + 3) / 4, mc = (tc + 3) / 4;
+    p.TA = (ta + ma - 1) / ma;
+    p.TC = (tc + mc - 1) / mc;
+    p.ntc = mc;
+    p.ntiles = ma * mc;
+    p.herm = herm && p.ntiles == 1;
+    const int64_t target = p.TA * p.TC <= 4 ? 1024 : 512;
+    int64_t nch = (target + p.ntiles * nbatch - 1) / (p.ntiles * nbatch);
+    const int64_t room = bgram_work_parts(nbatch, nrows, na, nc);
+    if (nch > room) nch = room;
+    int64_t chunk = (nrows + nch - 1) / nch;
+    if (chunk < 64) chunk = 64;
+    chunk = (chunk + 15) / 16 * 16;
     p.chunk = chunk;
     p.nch = (nrows + chunk - 1) / chunk;
     return p;
 }
 
-template <int TA, int TC>
-static void launch_bgram_mfma(const bgram_mfma_plan &p, int64_t nbatch, int64_t nrows, int64_t na, int64_t nc,
-                              const double2 *X, int64_t xb, int64_t xr, const double2 *Z, int64_t zb, int64_t zr,
-                              double2 *part, hipStream_t s)
+template <int TA, int TC, bool HERM, bool BORD>
+static int launch_bgram_mfma(const bgram_mfma_plan &p, int64_t nbatch, int64_t nrows, int64_t na, int64_t nc,
+                             const double2 *X, int64_t xb, int64_t xr, const double2 *Z, int64_t zb, int64_t zr,
+                             double2 *part, hipStream_t s)
 {
-    const unsigned gy = (unsigned)((p.ntiles + (4 / p.nsub) - 1) / (4 / p.nsub));
-    hipLaunchKernelGGL((k_bgram_mfma<TA, TC>), dim3((unsigned)p.nch, gy, (unsigned)nbatch), dim3(256), 0, s, nrows, na,
-                       nc, p.chunk, p.ntc, p.ntiles, p.nsub, X, xb, xr, Z, zb, zr, part);
+    const size_t lds = (size_t)(256 * TA * TC + 16 * TA + 16 * TC + 1) * 16;
+    hipLaunchKernelGGL((k_bgram_mfma<TA, TC, HERM, BORD>), dim3((unsigned)p.nch, (unsigned)p.ntiles, (unsigned)nbatch),
+                       dim3(256), lds, s, nrows, (int)na, (int)nc, p.chunk, p.ntc, X, xb, xr, Z, zb, zr, part);
+    RSVDT_LAUNCH_CHECK("rsvdt_hip_bgram(mfma)");
+    return RSVDT_HIP_OK;
 }
 
 static int64_t bgram_chunk(int64_t nbatch, int64_t nrows, int64_t na, int64_t nc)
@@ -485,8 +647,7 @@ extern "C" size_t rsvdt_hip_bgram_work_bytes(int64_t nbatch, int64_t nrows, int6
 {
     const int64_t chunk = bgram_chunk(nbatch, nrows, na, nc);
     const int64_t nch = (nrows + chunk - 1) / chunk;
-    const bgram_mfma_plan p = bgram_mfma_shape(nbatch, nrows, na, nc);
-    int64_t parts = p.nch * p.nsub;
+    int64_t parts = bgram_work_parts(nbatch, nrows, na, nc);
     if (nch > parts) parts = nch;
     return (size_t)(nbatch * parts * na * nc) * 16 + 256;
 }
@@ -500,17 +661,33 @@ extern "C" int rsvdt_hip_bgram(int64_t nbatch, int64_t nrows, int64_t na, int64_
     if (nbatch > 65535) { set_error_msg("rsvdt_hip_bgram: nbatch > 65535"); return RSVDT_HIP_ERR_ARG; }
     hipStream_t st = as_stream(s);
     int64_t nparts;
+    int herm = 0, ntile = 0;
     if (xa == 1 && zc == 1) {
-        const bgram_mfma_plan p = bgram_mfma_shape(nbatch, nrows, na, nc);
+        const bgram_mfma_plan p =
+            bgram_mfma_shape(nbatch, nrows, na, nc, X == Z && na == nc && xr == zr && (xb == zb || nbatch == 1));
         const double2 *X2 = (const double2 *)X, *Z2 = (const double2 *)Z;
         double2 *W = (double2 *)work;
-#define RSVDT_BG(A, C) \
-        if (p.TA == A && p.TC == C) launch_bgram_mfma<A, C>(p, nbatch, nrows, na, nc, X2, xb, xr, Z2, zb, zr, W, st);
-        RSVDT_BG(1, 1) RSVDT_BG(1, 2) RSVDT_BG(1, 3) RSVDT_BG(2, 1) RSVDT_BG(2, 2) RSVDT_BG(2, 3)
-        RSVDT_BG(3, 1) RSVDT_BG(3, 2) RSVDT_BG(3, 3)
+        int rc = RSVDT_HIP_ERR_ARG;
+#define RSVDT_BG_L(A, C, H, B) rc = launch_bgram_mfma<A, C, H, B>(p, nbatch, nrows, na, nc, X2, xb, xr, Z2, zb, zr, W, st)
+#define RSVDT_BG(A, C)                                                  \
+        if (p.TA == A && p.TC == C) {                                   \
+            if (p.bord) {                                               \
+                if (A == C && p.herm) RSVDT_BG_L(A, C, A == C, true);   \
+                else RSVDT_BG_L(A, C, false, true);                     \
+            } else {                                                    \
+                if (A == C && p.herm) RSVDT_BG_L(A, C, A == C, false);  \
+                else RSVDT_BG_L(A, C, false, false);                    \
+            }                                                           \
+        }
+#define RSVDT_BG_ROW(A) RSVDT_BG(A, 1) RSVDT_BG(A, 2) RSVDT_BG(A, 3) RSVDT_BG(A, 4)
+        RSVDT_BG_ROW(1) RSVDT_BG_ROW(2) RSVDT_BG_ROW(3) RSVDT_BG_ROW(4)
+#undef RSVDT_BG_ROW
 #undef RSVDT_BG
-        RSVDT_LAUNCH_CHECK("rsvdt_hip_bgram(mfma)");
-        nparts = p.nch * p.nsub;
+#undef RSVDT_BG_L
+        if (rc) return rc;
+        nparts = p.nch;
+        herm = p.herm;
+        ntile = p.bord ? (int)(na / 16) : (int)((na + 15) / 16);
     } else {
         const int64_t chunk = bgram_chunk(nbatch, nrows, na, nc);
         const int64_t nch = (nrows + chunk - 1) / chunk;
@@ -521,9 +698,8 @@ extern "C" int rsvdt_hip_bgram(int64_t nbatch, int64_t nrows, int64_t na, int64_
         RSVDT_LAUNCH_CHECK("rsvdt_hip_bgram(part)");
         nparts = nch;
     }
-    const int64_t tot = nbatch * na * nc;
-    hipLaunchKernelGGL(k_bgram_reduce, dim3(ceil_div(tot, 256)), dim3(256), 0, st, nbatch, nparts, na, nc,
-                       (const double2 *)work, (double2 *)G);
+    hipLaunchKernelGGL(k_bgram_reduce, dim3(ceil_div(na * nc, 32), (unsigned)nbatch), dim3(256), 0, st, nparts, (int)na,
+                       (int)nc, herm, ntile, (const double2 *)work, (double2 *)G);
     RSVDT_LAUNCH_CHECK("rsvdt_hip_bgram(reduce)");
     return RSVDT_HIP_OK;
 }

@@ -47,3 +47,31 @@ def test_jacobi_svd_sizes(L, pkg, n, rank_def):
         t = Ul.sum(axis=0)
         big = np.abs(t) > 1e-7
         assert np.all(t.real[big] > 0) and np.all(np.abs(t.imag[big]) <= tol * np.sqrt(n))
+
+
+@pytest.mark.parametrize("na,nc", [(1, 1), (16, 16), (17, 17), (20, 20), (32, 32), (33, 33), (48, 48), (49, 49),
+                                   (64, 64), (65, 65), (81, 81), (129, 129), (65, 17), (17, 65), (33, 65), (65, 32),
+                                   (40, 64), (64, 40)])
+@pytest.mark.parametrize("nb,nr", [(1, 3), (3, 515), (2, 4100)])
+@pytest.mark.parametrize("same", [False, True])
+def test_gram_tiles(L, pkg, na, nc, nb, nr, same):
+    """X^H Z for the macro tiles, the border column (n = 16 T + 1) and the
+    triangle of X^H X, on rows that do not fill the waves' steps."""
+    if same and na != nc:
+        pytest.skip("the triangle needs X = Z")
+    rng = np.random.default_rng(na * 1000 + nc + nr)
+    X = crandn(rng, nb, nr, na)
+    Z = X if same else crandn(rng, nb, nr, nc)
+    L.rsvdt_hip_bgram_work_bytes.restype = ctypes.c_size_t
+    L.rsvdt_hip_bgram_work_bytes.argtypes = [I64] * 4
+    L.rsvdt_hip_bgram.argtypes = [I64] * 4 + [V, I64, I64, I64, V, I64, I64, I64, V, V, V]
+    dX = Dev(pkg, X)
+    dZ = dX if same else Dev(pkg, Z)
+    dG = Dev(pkg, nbytes=nb * na * nc * 16)
+    dw = Dev(pkg, nbytes=L.rsvdt_hip_bgram_work_bytes(nb, nr, na, nc))
+    for _ in range(2):
+        assert L.rsvdt_hip_bgram(nb, nr, na, nc, dX.p, nr * na, na, 1, dZ.p, nr * nc, nc, 1, dG.p, dw.p, None) == 0
+    G = dG.get(np.complex128, (nb, na, nc))
+    ref = np.einsum("bra,brc->bac", X.conj(), Z)
+    # each entry: nr products of modulus ~1, rounded sums of 4 nr real terms
+    assert np.max(np.abs(G - ref)) <= 8 * EPS * np.sqrt(nr) * (np.abs(X).max() * np.abs(Z).max()) * np.sqrt(nr)
