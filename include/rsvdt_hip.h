@@ -229,6 +229,14 @@ int rsvdt_hip_bapply(int64_t nbatch, int64_t nrows, int64_t na, int64_t nc,
                      double *Out, int64_t ob, int64_t orow, int64_t oc,
                      rsvdt_stream_t s);
 
+/* One CholeskyQR step on unit column strides: Out_b = X_b C_b with C_b upper
+ * triangular (nbatch x n x n row-major, n <= 64), and, when G is not NULL, the
+ * Gram matrix G_b = Out_b^H Out_b of the result in the same pass over the rows.
+ * X_b(r,a) = X[b*xb + r*xr + a]; Out has the same strides and may be X.  work
+ * must hold rsvdt_hip_bgram_work_bytes(nbatch, nrows, n, n) bytes (with G). */
+int rsvdt_hip_bapply_gram(int64_t nbatch, int64_t nrows, int64_t n, const double *X, int64_t xb, int64_t xr,
+                          const double *C, double *Out, double *G, void *work, rsvdt_stream_t s);
+
 /* ---- batched small dense kernels (one workgroup per matrix) ----------- */
 /* Cholesky of (G_b + shift_b*I) (upper R, G = R^H R) then Rinv_b = R^-1.
  * G, R, Rinv: nbatch x n x n complex FP64 row-major.  shift_rel >= 0:

@@ -612,6 +612,172 @@ __global__ __launch_bounds__(256) void k_bapply_mfma(
     }
 }
 
+// One CholeskyQR step on the rows: Out_b = X_b C_b with C_b upper triangular
+// (n <= 16 TC <= 64), and with GRAM the Gram matrix of the result,
+// Out_b^H Out_b, from the same registers: lane i of the apply's accumulators
+// holds Out(r0 + 4j + i/16, c0 + i%16), which is exactly the operand layout of
+// the Gram's 4-row step j, so the next pass's Gram costs MFMAs but no memory.
+// A wave walks 16 RT-row tiles, the next tile's rows loaded while the current
+// one computes; it reads all of a tile before it writes any of it and no other
+// wave touches its rows, so Out may be X.  The zero tiles of C are skipped.
+// The waves' Gram sums meet in LDS in wave order and go to k_bgram_reduce as
+// one partial per workgroup.  NT: nontemporal loads and stores for blocks
+// beyond the last-level cache.  Without GRAM (the last pass) the apply alone.
+// Bound by memory for 16 columns, by FP64 MFMA above.  16 blocks of
+// 393,216 x 16: 622 us, 5.2 TB/s (apply 612 us, then the Gram 329 us, as two
+// kernels); a whole QR of 32 blocks of 60,000 x 32 went from 3642 to 1984 us.
+template <int TC, bool GRAM, bool NT>
+__global__ __launch_bounds__(256) void k_bapply_gram(int64_t nrows, int n, const double2 *X, int64_t xb, int64_t xr,
+                                                     const double2 *__restrict__ C, double2 *Out,
+                                                     double2 *__restrict__ part)
+{
+    constexpr int RT = TC == 1 ? 2 : 1, CW = 16 * TC, NS = 4 * TC;
+    extern __shared__ double2 gsm[];             // C_b [CW][CW], then the workgroup's Gram sums
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, kr = lane >> 4, cl = lane & 15;
+    const int64_t b = blockIdx.z;
+    const double2 *Cb = C + b * n * n;
+    for (int e = threadIdx.x; e < CW * CW; e += 256) {
+        const int a = e / CW, c = e % CW;
+        double2 v = make_double2(0, 0);
+        if (a < n && c < n) v = Cb[a * n + c];
+        gsm[e] = v;
+    }
+    __syncthreads();
+    const double2 *Xb = X + b * xb;
+    double2 *Ob = Out + b * xb;
+    int ao[NS];
+    bool aok[NS];
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+        aok[q] = 4 * q + kr < n;
+        ao[q] = aok[q] ? 4 * q + kr : n - 1;
+    }
+    double2 xn[RT][NS];
+    bool rn[RT];
+    auto load = [&](int64_t tile) {
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            int64_t r = tile * (16 * RT) + 16 * t + cl;
+            rn[t] = r < nrows;
+            if (!rn[t]) r = nrows - 1;
+            const double2 *xp = Xb + r * xr;
+#pragma unroll
+            for (int q = 0; q < NS; ++q) {
+                if constexpr (NT) {
+                    const dvec2 v = __builtin_nontemporal_load((const dvec2 *)(xp + ao[q]));
+                    xn[t][q] = make_double2(v.x, v.y);
+                } else xn[t][q] = xp[ao[q]];
+            }
+        }
+    };
+    dvec4 gr[TC][TC], gi[TC][TC];
+#pragma unroll
+    for (int t = 0; t < TC; ++t)
+#pragma unroll
+        for (int u = 0; u < TC; ++u) { gr[t][u] = (dvec4){0, 0, 0, 0}; gi[t][u] = (dvec4){0, 0, 0, 0}; }
+    const int64_t ntile = (nrows + 16 * RT - 1) / (16 * RT), step = (int64_t)gridDim.x * 4;
+    int64_t tile = (int64_t)blockIdx.x * 4 + wv;
+    if (tile < ntile) load(tile);
+    for (; tile < ntile; tile += step) {
+        double2 x[RT][NS];
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int q = 0; q < NS; ++q) {
+                const bool ok = rn[t] && aok[q];
+                x[t][q] = make_double2(ok ? xn[t][q].x : 0.0, ok ? xn[t][q].y : 0.0);
+            }
+        load(tile + step < ntile ? tile + step : tile);       // the last one again: its values are not used
+        dvec4 dr[RT][TC], di[RT][TC];
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int u = 0; u < TC; ++u) { dr[t][u] = (dvec4){0, 0, 0, 0}; di[t][u] = (dvec4){0, 0, 0, 0}; }
+#pragma unroll
+        for (int q = 0; q < NS; ++q)
+#pragma unroll
+            for (int u = q / 4; u < TC; ++u) {   // C(a, c) = 0 for a > c
+                const double2 cv = gsm[(4 * q + kr) * CW + 16 * u + cl];
+#pragma unroll
+                for (int t = 0; t < RT; ++t) {
+                    dr[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t][q].x, cv.x, dr[t][u], 0, 0, 0);
+                    di[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t][q].x, cv.y, di[t][u], 0, 0, 0);
+                }
+#pragma unroll
+                for (int t = 0; t < RT; ++t) {
+                    dr[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(-x[t][q].y, cv.y, dr[t][u], 0, 0, 0);
+                    di[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t][q].y, cv.x, di[t][u], 0, 0, 0);
+                }
+            }
+        const int64_t r0 = tile * (16 * RT);
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t r = r0 + 16 * t + 4 * j + kr;
+                if (r < nrows) {
+#pragma unroll
+                    for (int u = 0; u < TC; ++u)
+                        if (16 * u + cl < n) {
+                            double2 *o = Ob + r * xr + 16 * u + cl;
+                            if constexpr (NT) {
+                                const dvec2 v = {dr[t][u][j], di[t][u][j]};
+                                __builtin_nontemporal_store(v, (dvec2 *)o);
+                            } else *o = make_double2(dr[t][u][j], di[t][u][j]);
+                        }
+                }
+            }
+        if constexpr (GRAM) {
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+#pragma unroll
+                    for (int u = 0; u < TC; ++u)
+#pragma unroll
+                        for (int v = u; v < TC; ++v) {
+                            gr[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(dr[t][u][j], dr[t][v][j], gr[u][v], 0, 0, 0);
+                            gi[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(dr[t][u][j], di[t][v][j], gi[u][v], 0, 0, 0);
+                        }
+#pragma unroll
+                    for (int u = 0; u < TC; ++u)
+#pragma unroll
+                        for (int v = u; v < TC; ++v) {
+                            gr[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(di[t][u][j], di[t][v][j], gr[u][v], 0, 0, 0);
+                            gi[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(-di[t][u][j], dr[t][v][j], gi[u][v], 0, 0, 0);
+                        }
+                }
+        }
+    }
+    if constexpr (GRAM) {
+        __syncthreads();                          // C_b is no longer read
+#pragma unroll 1
+        for (int w = 0; w < 4; ++w) {
+            if (wv == w) {
+#pragma unroll
+                for (int u = 0; u < TC; ++u) {
+#pragma unroll
+                    for (int v = u; v < TC; ++v)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            double2 *o = gsm + (16 * u + 4 * j + kr) * CW + 16 * v + cl;
+                            double2 g = make_double2(gr[u][v][j], gi[u][v][j]);
+                            if (w) g = zadd(*o, g);
+                            *o = g;
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            __syncthreads();
+        }
+        double2 *pb = part + (b * gridDim.x + blockIdx.x) * (int64_t)n * n;
+        for (int e = threadIdx.x; e < CW * CW; e += 256) {
+            const int a = e / CW, c = e % CW;
+            if (a / 16 <= c / 16 && a < n && c < n) pb[a * n + c] = gsm[e];
+        }
+    }
+}
+
 }  // namespace rsvdt
 
 using namespace rsvdt;
@@ -764,5 +930,62 @@ extern "C" int rsvdt_hip_bapply(int64_t nbatch, int64_t nrows, int64_t na, int64
                        na, nc, ncpad, rb, (const double2 *)X, xb, xr, xa, (const double2 *)C, alpha,
                        (const double2 *)Y, yb, yr, yc, (double2 *)Out, ob, orow, oc);
     RSVDT_LAUNCH_CHECK("rsvdt_hip_bapply");
+    return RSVDT_HIP_OK;
+}
+
+// Workgroups per batch: enough for the resident waves of all CUs (four
+// workgroups a CU for one column tile, two for two, one above), at most one per
+// four row tiles, and at most the partials the Gram's work buffer has room for.
+template <int TC, bool GRAM>
+static int launch_bapply_gram(int64_t nbatch, int64_t nrows, int64_t n, const double2 *X, int64_t xb, int64_t xr,
+                              const double2 *C, double2 *Out, double2 *part, int64_t *nparts, hipStream_t s)
+{
+    const int64_t ntile = (nrows + (TC == 1 ? 32 : 16) - 1) / (TC == 1 ? 32 : 16);
+    int64_t gx = ((TC == 1 ? 1024 : (TC == 2 ? 512 : 256)) + nbatch - 1) / nbatch;
+    if (gx > (ntile + 3) / 4) gx = (ntile + 3) / 4;
+    const int64_t room = bgram_work_parts(nbatch, nrows, n, n);
+    if (GRAM && gx > room) gx = room;
+    const size_t lds = (size_t)(256 * TC * TC) * 16;
+    const dim3 grid((unsigned)gx, 1, (unsigned)nbatch);
+    if ((double)nbatch * (double)nrows * (double)n * 16.0 > 256e6)
+        hipLaunchKernelGGL((k_bapply_gram<TC, GRAM, true>), grid, dim3(256), lds, s, nrows, (int)n, X, xb, xr, C, Out,
+                           part);
+    else
+        hipLaunchKernelGGL((k_bapply_gram<TC, GRAM, false>), grid, dim3(256), lds, s, nrows, (int)n, X, xb, xr, C, Out,
+                           part);
+    RSVDT_LAUNCH_CHECK("rsvdt_hip_bapply_gram");
+    *nparts = gx;
+    return RSVDT_HIP_OK;
+}
+
+extern "C" int rsvdt_hip_bapply_gram(int64_t nbatch, int64_t nrows, int64_t n, const double *X, int64_t xb, int64_t xr,
+                                     const double *C, double *Out, double *G, void *work, rsvdt_stream_t s)
+{
+    if (nbatch <= 0 || nrows <= 0 || n <= 0) return RSVDT_HIP_OK;
+    if (nbatch > 65535 || n > 64 || (G && !work)) {
+        set_error_msg("rsvdt_hip_bapply_gram: nbatch <= 65535, n <= 64 (and work with G) required");
+        return RSVDT_HIP_ERR_ARG;
+    }
+    hipStream_t st = as_stream(s);
+    int64_t np = 0;
+    int rc = RSVDT_HIP_ERR_ARG;
+    const int TC = (int)((n + 15) / 16);
+#define RSVDT_AG(T)                                                                                              \
+    if (TC == T)                                                                                                 \
+        rc = G ? launch_bapply_gram<T, true>(nbatch, nrows, n, (const double2 *)X, xb, xr, (const double2 *)C,   \
+                                             (double2 *)Out, (double2 *)work, &np, st)                           \
+               : launch_bapply_gram<T, false>(nbatch, nrows, n, (const double2 *)X, xb, xr, (const double2 *)C,  \
+                                              (double2 *)Out, nullptr, &np, st);
+    RSVDT_AG(1) RSVDT_AG(2) RSVDT_AG(3)
+#undef RSVDT_AG
+    if (TC == 4) {          // both accumulator sets do not fit beside the operands: the Gram on its own
+        rc = launch_bapply_gram<4, false>(nbatch, nrows, n, (const double2 *)X, xb, xr, (const double2 *)C,
+                                          (double2 *)Out, nullptr, &np, st);
+        return rc || !G ? rc : rsvdt_hip_bgram(nbatch, nrows, n, n, Out, xb, xr, 1, Out, xb, xr, 1, G, work, s);
+    }
+    if (rc || !G) return rc;
+    hipLaunchKernelGGL(k_bgram_reduce, dim3(ceil_div(n * n, 32), (unsigned)nbatch), dim3(256), 0, st, np, (int)n, (int)n,
+                       1, TC, (const double2 *)work, (double2 *)G);
+    RSVDT_LAUNCH_CHECK("rsvdt_hip_bapply_gram(reduce)");
     return RSVDT_HIP_OK;
 }

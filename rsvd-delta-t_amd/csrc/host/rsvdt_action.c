@@ -819,12 +819,21 @@ PetscErrorCode rsvdt_cholqr_bufs(PetscInt nb, PetscInt nrows, PetscInt n, double
     RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_zero(w->info, 256, q));
     const double shift_rel = 11.0 * ((double)nrows * (double)n + (double)n * (double)(n + 1)) * 1.1102230246251565e-16;
     double *cur = X, *oth = T ? T : X;
+    /* up to 64 contiguous columns: each apply also forms the Gram matrix of its
+     * result, so a pass after the first reads and writes the rows once (7
+     * traversals of the blocks for three passes instead of 9) */
+    const int joint = xa == 1 && n <= 64;
     for (int pass = 0; pass < npass; pass++) {
-        RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_bgram(nb, nrows, n, n, cur, xb, xr, xa, cur, xb, xr, xa, w->G, w->work, q));
+        if (!joint || pass == 0)
+            RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_bgram(nb, nrows, n, n, cur, xb, xr, xa, cur, xb, xr, xa, w->G, w->work, q));
         RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_bchol_inv(nb, n, w->G, (pass == 0 && shift_first) ? shift_rel : 0.0,
                                                        drop_tol, w->R, w->Ri, w->info, q));
-        RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_bapply(nb, nrows, n, n, cur, xb, xr, xa, w->Ri, 0.0, NULL, 0, 0, 0, oth, xb,
-                                                    xr, xa, q));
+        if (joint)
+            RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_bapply_gram(nb, nrows, n, cur, xb, xr, w->Ri, oth,
+                                                             pass + 1 < npass ? w->G : NULL, w->work, q));
+        else
+            RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_bapply(nb, nrows, n, n, cur, xb, xr, xa, w->Ri, 0.0, NULL, 0, 0, 0, oth,
+                                                        xb, xr, xa, q));
         if (T) { double *tmp = cur; cur = oth; oth = tmp; }
         if (R_out) {
             if (pass == 0) RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_memcpy_d2d(w->Ra, w->R, mat, q));

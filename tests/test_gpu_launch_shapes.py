@@ -75,3 +75,37 @@ def test_gram_tiles(L, pkg, na, nc, nb, nr, same):
     ref = np.einsum("bra,brc->bac", X.conj(), Z)
     # each entry: nr products of modulus ~1, rounded sums of 4 nr real terms
     assert np.max(np.abs(G - ref)) <= 8 * EPS * np.sqrt(nr) * (np.abs(X).max() * np.abs(Z).max()) * np.sqrt(nr)
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("nb,nr", [(1, 3), (3, 515), (2, 4100)])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_apply_gram(L, pkg, n, nb, nr, in_place):
+    """Out = X C (C upper triangular) and Out^H Out from one pass, and the
+    apply alone, against numpy."""
+    rng = np.random.default_rng(n + nr)
+    X, C = crandn(rng, nb, nr, n), np.triu(crandn(rng, nb, n, n)) / np.sqrt(n)
+    ref = np.einsum("bra,bac->brc", X, C)
+    G_ref = np.einsum("bra,brc->bac", ref.conj(), ref)
+    L.rsvdt_hip_bgram_work_bytes.restype = ctypes.c_size_t
+    L.rsvdt_hip_bgram_work_bytes.argtypes = [I64] * 4
+    L.rsvdt_hip_bapply_gram.argtypes = [I64] * 3 + [V, I64, I64, V, V, V, V, V]
+    for with_gram in (True, False):
+        dX, dC = Dev(pkg, X), Dev(pkg, C)
+        dO = dX if in_place else Dev(pkg, nbytes=X.nbytes)
+        dG = Dev(pkg, nbytes=C.nbytes)
+        dw = Dev(pkg, nbytes=L.rsvdt_hip_bgram_work_bytes(nb, nr, n, n))
+        assert L.rsvdt_hip_bapply_gram(nb, nr, n, dX.p, nr * n, n, dC.p, dO.p, dG.p if with_gram else None,
+                                       dw.p, None) == 0
+        out = dO.get(np.complex128, X.shape)
+        # sums of 4 n real products of size max|X| max|C|
+        assert np.max(np.abs(out - ref)) <= 8 * EPS * n * np.abs(X).max() * np.abs(C).max()
+        if with_gram:
+            assert np.max(np.abs(dG.get(np.complex128, C.shape) - G_ref)) <= 16 * EPS * nr * np.abs(ref).max() ** 2
+
+
+def test_apply_gram_rejects_wide(L, pkg):
+    d = Dev(pkg, nbytes=1 << 16)
+    L.rsvdt_hip_bapply_gram.argtypes = [I64] * 3 + [V, I64, I64, V, V, V, V, V]
+    assert L.rsvdt_hip_bapply_gram(1, 4, 65, d.p, 260, 65, d.p, d.p, None, None, None) == 102
+    assert L.rsvdt_hip_bapply_gram(1, 4, 8, d.p, 32, 8, d.p, d.p, d.p, None, None) == 102
