@@ -187,6 +187,20 @@ int rsvdt_hip_horner_fused_fits(int64_t nrows, int64_t nnz, int a_real, int prec
 int rsvdt_hip_horner_fused(const rsvdt_spmm_desc *d, int64_t nnz, int64_t maxrow, void *y, const void *g,
                            int64_t gstride, const double *coef, int64_t nsteps, double *snap, int64_t snap_stride,
                            int64_t i0, int64_t Nt, int64_t RR, int64_t Nstore, int dir, rsvdt_stream_t s);
+/* (column, block) pairs of rsvdt_hip_horner_fused that the GPU's 256 CUs hold
+ * at once for this operator (0: it does not fit). */
+int64_t rsvdt_hip_horner_fused_resident(int64_t nrows, int64_t nnz, int64_t maxrow, int a_real, int prec);
+/* The same from y = 0 with harmonic forcing, FP64: the forcing of step j of
+ * block m (d->nb blocks) is G_m exp(+-i phase), the phase that entry
+ * (m, sgn*2j mod nt2) of the iDFT table idft ([nt2][d->nb]) holds times 2/nt2;
+ * y (d->nb blocks) receives the state after nsteps steps, 2(nsteps-1) < nt2. */
+int rsvdt_hip_horner_fused_harm(const rsvdt_spmm_desc *d, int64_t nnz, int64_t maxrow, double *y, const double *G,
+                                const double *coef, int64_t nsteps, const double *idft, int64_t nt2, int sgn,
+                                rsvdt_stream_t s);
+/* Out_b = E X_b (+ F_b, may be NULL) for nb blocks of N x k (stride N*k): E is
+ * N x N row-major complex FP64; Out is not X. */
+int rsvdt_hip_dense_apply(int64_t N, int64_t k, int64_t nb, const double *E, const double *X, const double *F,
+                          double *Out, rsvdt_stream_t s);
 int rsvdt_hip_spmm_blocks(int64_t nrows, int64_t k, int64_t nb, const int32_t *rowptr, const int32_t *col,
                           const double *val_complex, const double *in, int64_t in_bstride,
                           double *out, int64_t out_bstride, rsvdt_stream_t s);
@@ -286,6 +300,8 @@ size_t rsvdt_qr_blocks_noalloc_bytes(int64_t nblocks, int64_t N, int64_t k);
 int rsvdt_qr_blocks_noalloc(double *Y, int64_t N, int64_t k, int64_t nblocks, rsvdt_stream_t s);
 
 /* ---- elementwise ------------------------------------------------------ */
+/* the n x n complex FP64 identity */
+int rsvdt_hip_identity(int64_t n, double *p, rsvdt_stream_t s);
 /* y = a*x (complex entries, FP64), n entries */
 int rsvdt_hip_zscale(int64_t n, double a, const double *x, double *y, rsvdt_stream_t s);
 /* y += a*x (complex entries, FP64, real a), n entries */

@@ -798,13 +798,33 @@ __host__ __device__ inline fused_lds fused_layout(int64_t nrows, int64_t nnz, in
     return l;
 }
 
-template <typename T, bool AREAL>
+
+// How the forcing term of a step is given: none, one sample per step
+// (g + step*gstride), or harmonic: block b's constant g_b times the phase
+// harm_phase(step, b), from y = 0.
+enum { FORC_NONE = 0, FORC_SAMPLES = 1, FORC_HARM = 2 };
+struct harm_desc {
+    const double2 *table;      // [nt2][nwe] iDFT table
+    int64_t nwe, nt2;
+    double scale;              // table entry -> unit phase
+    int sgn;                   // +1: entry 2 j; -1: entry -2 j mod nt2
+};
+__device__ __forceinline__ double2 harm_phase(const harm_desc &hd, int64_t j, int64_t b)
+{
+    int64_t p = 2 * j;
+    if (hd.sgn < 0 && p) p = hd.nt2 - p;
+    const double2 z = hd.table[p * hd.nwe + b];
+    return make_double2(z.x * hd.scale, z.y * hd.scale);
+}
+
+template <typename T, bool AREAL, int FORC>
 __global__ __launch_bounds__(256) void k_horner_fused(
     int nrows, int nnz, int k, int nsteps, int64_t bstride,
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ colidx, const void *__restrict__ vals_,
     typename vec2<T>::type *y, const typename vec2<T>::type *__restrict__ g, int64_t gstride,
     double c1, double c2, double c3, double c4,
-    double2 *__restrict__ snap, int64_t snap_stride, int64_t i0, int64_t Nt, int64_t RR, int64_t Nstore, int dir)
+    double2 *__restrict__ snap, int64_t snap_stride, int64_t i0, int64_t Nt, int64_t RR, int64_t Nstore, int dir,
+    harm_desc hd)
 {
     using V = typename vec2<T>::type;
     using AV = typename aval<T, AREAL>::type;
@@ -822,7 +842,10 @@ __global__ __launch_bounds__(256) void k_horner_fused(
     const AV *vals = (const AV *)vals_;
     for (int e = threadIdx.x; e < nnz; e += blockDim.x) { sv[e] = vals[e]; sci[e] = colidx[e]; }
     for (int r = threadIdx.x; r <= nrows; r += blockDim.x) srp[r] = rowptr[r];
-    for (int r = threadIdx.x; r < nrows; r += blockDim.x) sy[r] = y[boff + (int64_t)r * k + j];
+    for (int r = threadIdx.x; r < nrows; r += blockDim.x) {
+        if constexpr (FORC == FORC_HARM) sy[r] = V{};
+        else sy[r] = y[boff + (int64_t)r * k + j];
+    }
     // snapshot schedule by counters (as in k_horner_fused_reg below)
     int64_t snap_st = nsteps, spos = 0;
     if (snap != nullptr) {
@@ -839,7 +862,9 @@ __global__ __launch_bounds__(256) void k_horner_fused(
             spos = spos + 1 == Nstore ? 0 : spos + 1;
             snap_st += RR;
         }
-        const V *gs = g != nullptr ? g + (int64_t)st * gstride + boff : nullptr;
+        const V *gs = FORC == FORC_NONE ? nullptr : (FORC == FORC_HARM ? g + boff : g + (int64_t)st * gstride + boff);
+        double2 ph = make_double2(1, 0);
+        if constexpr (FORC == FORC_HARM) ph = harm_phase(hd, st, blockIdx.y);
 #pragma unroll 1
         for (int stage = 0; stage < 4; ++stage) {
             const V *vin = stage == 0 ? sy : (stage == 2 ? sb : sa);
@@ -863,10 +888,15 @@ __global__ __launch_bounds__(256) void k_horner_fused(
                 }
                 const V yv = sy[r];
                 double ox = (double)yv.x + cs * sr, oy = (double)yv.y + cs * si;
-                if (stage == 3 && gs != nullptr) {
+                if (FORC != FORC_NONE && stage == 3) {
                     const V gv = gs[(int64_t)r * k + j];
-                    ox += (double)gv.x;
-                    oy += (double)gv.y;
+                    if constexpr (FORC == FORC_HARM) {
+                        ox += ph.x * (double)gv.x - ph.y * (double)gv.y;
+                        oy += ph.x * (double)gv.y + ph.y * (double)gv.x;
+                    } else {
+                        ox += (double)gv.x;
+                        oy += (double)gv.y;
+                    }
                 }
                 V o;
                 o.x = (T)ox;
@@ -884,13 +914,14 @@ __global__ __launch_bounds__(256) void k_horner_fused(
 // The same with each thread's rows (at most RPT, 512 threads) and their
 // nonzeros (at most MAXNZ per row) held in registers for the whole launch:
 // a stage is then MAXNZ LDS reads and FMAs per row and one barrier.
-template <typename T, bool AREAL, int MAXNZ, int RPT, bool HASG>
+template <typename T, bool AREAL, int MAXNZ, int RPT, int FORC>
 __global__ __launch_bounds__(512) void k_horner_fused_reg(
     int nrows, int k, int nsteps, int64_t bstride,
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ colidx, const void *__restrict__ vals_,
     typename vec2<T>::type *y, const typename vec2<T>::type *__restrict__ g, int64_t gstride,
     double c1, double c2, double c3, double c4,
-    double2 *__restrict__ snap, int64_t snap_stride, int64_t i0, int64_t Nt, int64_t RR, int64_t Nstore, int dir)
+    double2 *__restrict__ snap, int64_t snap_stride, int64_t i0, int64_t Nt, int64_t RR, int64_t Nstore, int dir,
+    harm_desc hd)
 {
     using V = typename vec2<T>::type;
     using AV = typename aval<T, AREAL>::type;
@@ -915,7 +946,10 @@ __global__ __launch_bounds__(512) void k_horner_fused_reg(
             if (u < n) av[t][u] = vals[e0 + u];
             else av[t][u] = AV{};
         }
-        if (live[t]) sy[r] = y[boff + (int64_t)r * k + j];
+        if (live[t]) {
+            if constexpr (FORC == FORC_HARM) sy[r] = V{};
+            else sy[r] = y[boff + (int64_t)r * k + j];
+        }
     }
     // Snapshot schedule, advanced by counters: step i = i0 + st with i > Nt and
     // (i - Nt) % RR == 0 stores snapshot (i - Nt)/RR - 1 (mod Nstore), slot
@@ -927,17 +961,20 @@ __global__ __launch_bounds__(512) void k_horner_fused_reg(
         snap_st = first - rel0;
         spos = (first / RR - 1) % Nstore;
     }
-    // The forcing term (HASG: g is not null) of step st + 1 is loaded as soon
-    // as step st's is used: its latency overlaps a whole step (barriers wait
-    // on LDS only).  The load is unconditional (the last step reloads its own
-    // sample) so that nothing has to wait for it before the next step.
+    // The forcing sample of step st + 1 is loaded as soon as step st's is
+    // used: its latency overlaps a whole step (barriers wait on LDS only).  The
+    // load is unconditional (the last step reloads its own sample) so that
+    // nothing has to wait for it before the next step.  Harmonic forcing keeps
+    // its block's constant term in registers and loads one phase per step.
     V gcur[RPT];
 #pragma unroll
     for (int t = 0; t < RPT; ++t) {
         const int r = threadIdx.x + t * blockDim.x;
         gcur[t] = V{};
-        if (HASG && live[t]) gcur[t] = g[boff + (int64_t)r * k + j];
+        if (FORC != FORC_NONE && live[t]) gcur[t] = g[boff + (int64_t)r * k + j];
     }
+    double2 ph = make_double2(1, 0);
+    if constexpr (FORC == FORC_HARM) ph = harm_phase(hd, 0, blockIdx.y);
     __syncthreads();
     for (int st = 0; st < nsteps; ++st) {
         int64_t pos = -1;
@@ -946,7 +983,9 @@ __global__ __launch_bounds__(512) void k_horner_fused_reg(
             spos = spos + 1 == Nstore ? 0 : spos + 1;
             snap_st += RR;
         }
-        const V *gn = HASG ? g + (int64_t)(st + 1 < nsteps ? st + 1 : st) * gstride + boff : nullptr;
+        const V *gn = FORC == FORC_SAMPLES ? g + (int64_t)(st + 1 < nsteps ? st + 1 : st) * gstride + boff : nullptr;
+        double2 phn = ph;
+        if constexpr (FORC == FORC_HARM) phn = harm_phase(hd, st + 1 < nsteps ? st + 1 : st, blockIdx.y);
 #pragma unroll
         for (int stage = 0; stage < 4; ++stage) {
             const V *vin = stage == 0 ? sy : (stage == 2 ? sb : sa);
@@ -971,10 +1010,14 @@ __global__ __launch_bounds__(512) void k_horner_fused_reg(
                 }
                 const V yv = sy[r];
                 double ox = (double)yv.x + cs * sr, oy = (double)yv.y + cs * si;
-                if (HASG && stage == 3) {
+                if (FORC == FORC_SAMPLES && stage == 3) {
                     ox += (double)gcur[t].x;
                     oy += (double)gcur[t].y;
                     gcur[t] = gn[(int64_t)r * k + j];
+                }
+                if (FORC == FORC_HARM && stage == 3) {
+                    ox += ph.x * (double)gcur[t].x - ph.y * (double)gcur[t].y;
+                    oy += ph.x * (double)gcur[t].y + ph.y * (double)gcur[t].x;
                 }
                 V o;
                 o.x = (T)ox;
@@ -985,6 +1028,7 @@ __global__ __launch_bounds__(512) void k_horner_fused_reg(
             }
             __syncthreads();
         }
+        ph = phn;
     }
 #pragma unroll
     for (int t = 0; t < RPT; ++t) {
@@ -997,6 +1041,61 @@ extern "C" int rsvdt_hip_horner_fused_fits(int64_t nrows, int64_t nnz, int a_rea
 {
     if (nrows <= 0 || nnz < 0 || nrows > 0x7fffffff || nnz > 0x7fffffff) return 0;
     return fused_layout(nrows, nnz, a_real, prec).total <= (size_t)RSVDT_FUSED_LDS;
+}
+
+extern "C" int64_t rsvdt_hip_horner_fused_resident(int64_t nrows, int64_t nnz, int64_t maxrow, int a_real, int prec)
+{
+    if (!rsvdt_hip_horner_fused_fits(nrows, nnz, a_real, prec)) return 0;
+    const bool reg = maxrow >= 0 && maxrow <= 4 && nrows <= 1024;
+    const size_t lds = reg ? (size_t)3 * (size_t)nrows * (prec == 64 ? 16 : 8) : fused_layout(nrows, nnz, a_real, prec).total;
+    const int64_t by_lds = (int64_t)(RSVDT_FUSED_LDS / (lds + 256)), by_waves = reg ? 4 : 8;
+    const int64_t per = by_lds < by_waves ? by_lds : by_waves;
+    return 256 * (per < 1 ? 1 : per);
+}
+
+static int launch_fused(const rsvdt_spmm_desc *d, int64_t nnz, int64_t maxrow, void *y, const void *g, int64_t gstride,
+                        const double *coef, int64_t nsteps, double *snap, int64_t snap_stride, int64_t i0, int64_t Nt,
+                        int64_t RR, int64_t Nstore, int dir, int forc, const harm_desc &hd, hipStream_t st)
+{
+    const dim3 grid((unsigned)d->k, (unsigned)d->nb);
+    const int64_t bs = d->nrows * d->k;
+    const bool reg = maxrow >= 0 && maxrow <= 4 && d->nrows <= 1024;     // rows and nonzeros in registers
+    const size_t lds = reg ? (size_t)3 * (size_t)d->nrows * (d->prec == 64 ? 16 : 8)
+                           : fused_layout(d->nrows, nnz, d->a_real, d->prec).total;
+#define RSVDT_FUSED(T, AR, F)                                                                                     \
+    do {                                                                                                          \
+        if (reg)                                                                                                  \
+            hipLaunchKernelGGL((k_horner_fused_reg<T, AR, 4, 2, F>), grid, dim3(512), lds, st, (int)d->nrows,      \
+                               (int)d->k, (int)nsteps, bs, d->rowptr, d->col, d->val,                              \
+                               (typename vec2<T>::type *)y, (const typename vec2<T>::type *)g, gstride, coef[0],   \
+                               coef[1], coef[2], coef[3], (double2 *)snap, snap_stride, i0, Nt, RR, Nstore, dir,   \
+                               hd);                                                                               \
+        else                                                                                                      \
+            hipLaunchKernelGGL((k_horner_fused<T, AR, F>), grid, dim3(256), lds, st, (int)d->nrows, (int)nnz,      \
+                               (int)d->k, (int)nsteps, bs, d->rowptr, d->col, d->val,                              \
+                               (typename vec2<T>::type *)y, (const typename vec2<T>::type *)g, gstride, coef[0],   \
+                               coef[1], coef[2], coef[3], (double2 *)snap, snap_stride, i0, Nt, RR, Nstore, dir,   \
+                               hd);                                                                               \
+    } while (0)
+#define RSVDT_FUSED_F(T, AR)                                                                                      \
+    do {                                                                                                          \
+        if (forc == FORC_SAMPLES) RSVDT_FUSED(T, AR, FORC_SAMPLES);                                               \
+        else RSVDT_FUSED(T, AR, FORC_NONE);                                                                       \
+    } while (0)
+    if (forc == FORC_HARM) {
+        if (d->a_real) RSVDT_FUSED(double, true, FORC_HARM);
+        else RSVDT_FUSED(double, false, FORC_HARM);
+    } else if (d->prec == 64) {
+        if (d->a_real) RSVDT_FUSED_F(double, true);
+        else RSVDT_FUSED_F(double, false);
+    } else {
+        if (d->a_real) RSVDT_FUSED_F(float, true);
+        else RSVDT_FUSED_F(float, false);
+    }
+#undef RSVDT_FUSED_F
+#undef RSVDT_FUSED
+    RSVDT_LAUNCH_CHECK("rsvdt_hip_horner_fused");
+    return RSVDT_HIP_OK;
 }
 
 extern "C" int rsvdt_hip_horner_fused(const rsvdt_spmm_desc *d, int64_t nnz, int64_t maxrow, void *y, const void *g,
@@ -1014,50 +1113,22 @@ extern "C" int rsvdt_hip_horner_fused(const rsvdt_spmm_desc *d, int64_t nnz, int
         return RSVDT_HIP_ERR_ARG;
     }
     if (nsteps <= 0) return RSVDT_HIP_OK;
-    const dim3 grid((unsigned)d->k, (unsigned)d->nb);
-    hipStream_t st0 = as_stream(s);
-    if (maxrow >= 0 && maxrow <= 4 && d->nrows <= 1024) {    // rows and nonzeros in registers
-        const size_t lds3 = (size_t)3 * (size_t)d->nrows * (d->prec == 64 ? 16 : 8);
-#define RSVDT_FUSED_REG_G(T, AR, HG)                                                                              \
-        hipLaunchKernelGGL((k_horner_fused_reg<T, AR, 4, 2, HG>), grid, dim3(512), lds3, st0, (int)d->nrows,       \
-                           (int)d->k, (int)nsteps, d->nrows * d->k, d->rowptr, d->col, d->val,                      \
-                           (typename vec2<T>::type *)y, (const typename vec2<T>::type *)g, gstride, coef[0],       \
-                           coef[1], coef[2], coef[3], (double2 *)snap, snap_stride, i0, Nt, RR, Nstore, dir)
-#define RSVDT_FUSED_REG(T, AR)                                                                                    \
-        do {                                                                                                      \
-            if (g != nullptr) RSVDT_FUSED_REG_G(T, AR, true);                                                     \
-            else RSVDT_FUSED_REG_G(T, AR, false);                                                                 \
-        } while (0)
-        if (d->prec == 64) {
-            if (d->a_real) RSVDT_FUSED_REG(double, true);
-            else RSVDT_FUSED_REG(double, false);
-        } else {
-            if (d->a_real) RSVDT_FUSED_REG(float, true);
-            else RSVDT_FUSED_REG(float, false);
-        }
-#undef RSVDT_FUSED_REG
-#undef RSVDT_FUSED_REG_G
-        RSVDT_LAUNCH_CHECK("rsvdt_hip_horner_fused");
-        return RSVDT_HIP_OK;
+    return launch_fused(d, nnz, maxrow, y, g, gstride, coef, nsteps, snap, snap_stride, i0, Nt, RR, Nstore, dir,
+                        g != nullptr ? FORC_SAMPLES : FORC_NONE, harm_desc{nullptr, 0, 0, 0.0, 1}, as_stream(s));
+}
+
+extern "C" int rsvdt_hip_horner_fused_harm(const rsvdt_spmm_desc *d, int64_t nnz, int64_t maxrow, double *y,
+                                           const double *G, const double *coef, int64_t nsteps, const double *idft,
+                                           int64_t nt2, int sgn, rsvdt_stream_t s)
+{
+    if (!d || d->nrows <= 0 || d->k <= 0 || d->k > 65535 || d->nb <= 0 || d->nb > 65535 || !y || !G || !coef || !idft ||
+        d->prec != 64 || nsteps <= 0 || 2 * (nsteps - 1) >= nt2 || (sgn != 1 && sgn != -1) ||
+        !rsvdt_hip_horner_fused_fits(d->nrows, nnz, d->a_real, 64)) {
+        set_error_msg("rsvdt_hip_horner_fused_harm: bad arguments");
+        return RSVDT_HIP_ERR_ARG;
     }
-    const size_t lds = fused_layout(d->nrows, nnz, d->a_real, d->prec).total;
-    const int64_t bs = d->nrows * d->k;
-    hipStream_t st = as_stream(s);
-#define RSVDT_FUSED_LAUNCH(T, AR)                                                                                 \
-    hipLaunchKernelGGL((k_horner_fused<T, AR>), grid, dim3(256), lds, st, (int)d->nrows, (int)nnz, (int)d->k,      \
-                       (int)nsteps, bs, d->rowptr, d->col, d->val, (typename vec2<T>::type *)y,                    \
-                       (const typename vec2<T>::type *)g, gstride, coef[0], coef[1], coef[2], coef[3],             \
-                       (double2 *)snap, snap_stride, i0, Nt, RR, Nstore, dir)
-    if (d->prec == 64) {
-        if (d->a_real) RSVDT_FUSED_LAUNCH(double, true);
-        else RSVDT_FUSED_LAUNCH(double, false);
-    } else {
-        if (d->a_real) RSVDT_FUSED_LAUNCH(float, true);
-        else RSVDT_FUSED_LAUNCH(float, false);
-    }
-#undef RSVDT_FUSED_LAUNCH
-    RSVDT_LAUNCH_CHECK("rsvdt_hip_horner_fused");
-    return RSVDT_HIP_OK;
+    const harm_desc hd = {(const double2 *)idft, d->nb, nt2, 0.5 * (double)nt2, sgn};
+    return launch_fused(d, nnz, maxrow, y, G, 0, coef, nsteps, nullptr, 0, 0, 0, 1, 1, 1, FORC_HARM, hd, as_stream(s));
 }
 
 static int check_desc(const rsvdt_spmm_desc *d, const char *who)

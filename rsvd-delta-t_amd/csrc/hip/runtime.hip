@@ -294,6 +294,19 @@ extern "C" int rsvdt_hip_zero(void *p, size_t bytes, rsvdt_stream_t s) {
     return RSVDT_HIP_OK;
 }
 
+// N x N identity, complex FP64
+__global__ void k_identity(int64_t n, double2 *p) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n * n) p[i] = make_double2(i / n == i % n ? 1.0 : 0.0, 0.0);
+}
+extern "C" int rsvdt_hip_identity(int64_t n, double *p, rsvdt_stream_t s) {
+    if (n <= 0) return RSVDT_HIP_OK;
+    if (n > 65536) { set_error_msg("rsvdt_hip_identity: n <= 65536"); return RSVDT_HIP_ERR_ARG; }
+    hipLaunchKernelGGL(k_identity, dim3(ceil_div(n * n, 256)), dim3(256), 0, as_stream(s), n, (double2 *)p);
+    RSVDT_LAUNCH_CHECK("rsvdt_hip_identity");
+    return RSVDT_HIP_OK;
+}
+
 // ---------------------------------------------------------------- elementwise
 __global__ void k_zscale(int64_t n, double a, const double2 *x, double2 *y) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -18,7 +18,7 @@
 
 /* scratch slots */
 enum { SCR_Y = 0, SCR_U1, SCR_U2, SCR_ACC, SCR_FBUF, SCR_FBUF2, SCR_G, SCR_R, SCR_RINV, SCR_RACC, SCR_RTMP,
-       SCR_WORK, SCR_INFO, SCR_MISC, SCR_MISC2, SCR_PROJ, SCR_MASK, SCR_RMASK, SCR_CNT, SCR_FSCALE, SCR_W1, SCR_W2, SCR_QRT, SCR_GINFO, SCR_SLOTS, SCR_NSLOTS };
+       SCR_WORK, SCR_INFO, SCR_MISC, SCR_MISC2, SCR_PROJ, SCR_MASK, SCR_RMASK, SCR_CNT, SCR_FSCALE, SCR_W1, SCR_W2, SCR_QRT, SCR_GINFO, SCR_SLOTS, SCR_H, SCR_NSLOTS };
 _Static_assert(SCR_NSLOTS <= RSVDT_NSCRATCH, "scratch slot table too small");
 
 /* ------------------------------------------------------------------ stepper */
@@ -668,6 +668,124 @@ static PetscErrorCode step_range(stepper *st, Mat A, RSVDt_vars *V, Mat Yall, Pe
     return ierr;
 }
 
+/* ------------------------------------------------------------------ leaps */
+/* Operators that fit in LDS: the RR steps between two snapshots as one dense
+ * product.  With P = P(hA), step i of the folded form is
+ *   y_i = P y_{i-1} + sum_m idft(m, 2(i-1)) G_m,
+ * so RR steps from step a on are
+ *   y_{a+RR} = E y_a + sum_m idft(m, 2a) H_m,   E = P^RR,
+ *   H_m = sum_{j<RR} P^{RR-1-j} z_m^{2j} G_m.
+ * The columns of E and of the H_m are RR steps of the LDS-resident stepper
+ * from unit vectors and from rest under harmonic forcing, all of them at once
+ * (they fill the GPU, where the k columns of the state are k workgroups), and
+ * the serial chain is one small product per snapshot instead of RR steps.
+ * E belongs to the operator and the step size and is kept on the Mat.  The
+ * same recursion, rounded in another order; the Nt % RR first steps run one
+ * by one.
+ *
+ * It pays when the steps it needs, in rounds of resident columns, are well
+ * below the steps of the state, counting a product as 5 steps (a step takes
+ * 1.1 us, a product and its launch about 5): with N = 500, k = 10, Nw = 64,
+ * RR = 64 an action's stepping takes 0.84 ms (H 0.17, 70 products 0.57, samples
+ * 0.1) and E 0.11 ms once; step by step it took 5.1 ms. */
+static PetscInt fused_rounds(Mat A, int dir, PetscInt cols)
+{
+    const int64_t res = rsvdt_hip_horner_fused_resident(A->rows, A->nnz, dir ? A->maxrow : A->maxrowH, A->is_real, 64);
+    return res > 0 ? (PetscInt)((cols + res - 1) / res) : 0;
+}
+
+static int leap_pays(Mat A, int dir, RSVDt_vars *V)
+{
+    const PetscInt Nw = V->RSVD.Nw, RR = V->TS.ResRatio, Nt = V->TS.Nt, k = V->RSVD.k;
+    if (g_rsvdt.opt.precision != 64 || g_rsvdt.opt.rk4_form || !g_rsvdt.opt.fuse_small || RR < 2 || Nt < 0 ||
+        V->TS.Ns != Nw * RR || A->rows > 16384)
+        return 0;
+    const PetscInt rk = fused_rounds(A, dir, k);
+    if (!rk) return 0;
+    const PetscInt nleap = Nt / RR + Nw + (V->TS.TransientRemoval ? 1 : 0);
+    const double one_by_one = (double)(nleap * RR + Nt % RR) * (double)rk;
+    const double leaps = (double)RR * (double)(fused_rounds(A, dir, A->rows) + fused_rounds(A, dir, V->RSVD.Nw_eff * k)) +
+                         (double)(Nt % RR) * (double)rk + 5.0 * (double)nleap;
+    return leaps < 0.7 * one_by_one;
+}
+
+/* E of A (dir 1) or A^H: nsteps homogeneous steps of the identity. */
+static PetscErrorCode leap_operator(Mat A, int dir, double h, PetscInt nsteps, const double **out)
+{
+    const int q = dir ? 0 : 1;
+    const PetscInt N = A->rows;
+    if (!A->leap[q].d || A->leap[q].h != h || A->leap[q].steps != nsteps) {
+        if (!A->leap[q].d)
+            RSVDT_HIPCHK("TSActionRK4", rsvdt_hip_malloc((void **)&A->leap[q].d, (size_t)N * (size_t)N * 16));
+        A->leap[q].steps = 0;                /* not valid until both launches are queued */
+        rsvdt_spmm_desc d;
+        desc_for(&d, A, dir, 64, N, 1);
+        const double cf[4] = {h / 4, h / 3, h / 2, h};
+        RSVDT_HIPCHK("TSActionRK4", rsvdt_hip_identity(N, A->leap[q].d, g_rsvdt.stream));
+        RSVDT_HIPCHK("TSActionRK4", rsvdt_hip_horner_fused(&d, A->nnz, dir ? A->maxrow : A->maxrowH, A->leap[q].d, NULL, 0,
+                                                           cf, nsteps, NULL, 0, 0, 0, 1, 1, dir, g_rsvdt.stream));
+        A->leap[q].h = h;
+        A->leap[q].steps = nsteps;
+    }
+    *out = A->leap[q].d;
+    return 0;
+}
+
+/* The stepping of an action (as time_stepping below) by leaps: G holds the
+ * folded forcing terms, Yall receives the snapshots. */
+static PetscErrorCode leap_stepping(Mat A, DFT_matrices *D, RSVDt_vars *V, const double *G, Mat Yall, phase_timer *t_rk4,
+                                    phase_timer *t_frc, int64_t *launches)
+{
+    const int dir = V->TS.DirAdj ? 1 : 0, sgn = dir ? 1 : -1;
+    const PetscInt N = A->rows, k = V->RSVD.k, Nwe = V->RSVD.Nw_eff, RR = V->TS.ResRatio, Nt = V->TS.Nt;
+    const PetscInt nsnap = V->TS.TransientRemoval ? V->RSVD.Nw + 1 : V->RSVD.Nw, r0 = Nt % RR, nlead = Nt / RR;
+    const int64_t L = N * k, nt2 = 2 * V->TS.Ns, maxrow = dir ? A->maxrow : A->maxrowH;
+    const size_t blk = (size_t)L * 16;
+    const double h = V->TS.dt, cf[4] = {h / 4, h / 3, h / 2, h};
+    const PetscInt chunk = 256;              /* forcing terms formed at a time: samples of the first steps, then leaps */
+    rsvdt_stream_t q = g_rsvdt.stream;
+    double *H = rsvdt_scratch(SCR_H, blk * (size_t)Nwe);
+    double *y0 = rsvdt_scratch(SCR_Y, blk), *y1 = rsvdt_scratch(SCR_U1, blk);
+    const PetscInt most = r0 > nlead + nsnap ? r0 : nlead + nsnap;
+    double *f = rsvdt_scratch(SCR_FBUF, blk * (size_t)(most < chunk ? most : chunk));
+    if (!H || !y0 || !y1 || !f) return rsvdt_err(RSVDT_ERR_MEM, "TSActionRK4", "cannot allocate the RK4 work buffers");
+    const double *E;
+    rsvdt_spmm_desc d;
+    if (t_frc) pt_begin(t_frc);
+    RSVDT_CHK(leap_operator(A, dir, h, RR, &E));
+    desc_for(&d, A, dir, 64, k, Nwe);
+    RSVDT_HIPCHK("TSActionRK4", rsvdt_hip_horner_fused_harm(&d, A->nnz, maxrow, H, G, cf, RR, D->idft->d, nt2, sgn, q));
+    if (t_frc) pt_end(t_frc);
+    if (t_rk4) pt_begin(t_rk4);
+    RSVDT_HIPCHK("TSActionRK4", rsvdt_hip_zero(y0, blk, q));
+    desc_for(&d, A, dir, 64, k, 1);
+    for (PetscInt c0 = 0; c0 < r0; c0 += chunk) {
+        const PetscInt c = chunk < r0 - c0 ? chunk : r0 - c0;
+        RSVDT_HIPCHK("CreateForcingOnFly", rsvdt_hip_coef_gemm(c, Nwe, L, D->idft->d, 1, Nwe, sgn * 2 * c0, 2 * sgn, nt2,
+                                                               1.0, G, L, f, L, 64, 0.0, q));
+        RSVDT_HIPCHK("TSRK4", rsvdt_hip_horner_fused(&d, A->nnz, maxrow, y0, f, L, cf, c, NULL, 0, 0, 0, 1, 1, dir, q));
+        *launches += 1;
+    }
+    const double *y = y0;
+    for (PetscInt c0 = 0; c0 < nlead + nsnap; c0 += chunk) {
+        const PetscInt c = chunk < nlead + nsnap - c0 ? chunk : nlead + nsnap - c0;
+        RSVDT_HIPCHK("CreateForcingOnFly", rsvdt_hip_coef_gemm(c, Nwe, L, D->idft->d, 1, Nwe, sgn * 2 * (r0 + c0 * RR),
+                                                               (int)(2 * sgn * RR), nt2, 1.0, H, L, f, L, 64, 0.0, q));
+        for (PetscInt l = c0; l < c0 + c; l++) {
+            double *out = y == y0 ? y1 : y0;
+            if (l >= nlead) {                /* snapshot l - nlead (SaveSnapshots.c:17-29) */
+                const PetscInt pos = dir ? l - nlead : nsnap - 1 - (l - nlead);
+                out = Yall->d + 2 * (size_t)pos * (size_t)L;
+            }
+            RSVDT_HIPCHK("TSRK4", rsvdt_hip_dense_apply(N, k, 1, E, y, f + 2 * (size_t)(l - c0) * (size_t)L, out, q));
+            y = out;
+            *launches += 1;
+        }
+    }
+    if (t_rk4) pt_end(t_rk4);
+    return 0;
+}
+
 /* The time stepping of one action (TSActionRK4.c:38-130) over rend steps.
  * With the FP32 state and transient removal, the Nt steps before the first
  * snapshot run in FP32 and the snapshot period in FP64: the FP32 rounding
@@ -689,6 +807,16 @@ static PetscErrorCode time_stepping(Mat A, DFT_matrices *D, RSVDt_vars *V, Mat F
     const int seg_prec[2] = {prec, 64};
     int64_t launches = 0;
     PetscErrorCode ierr = 0;
+    if (Yall && !fhat_folded && max_steps <= 0 && leap_pays(A, dir, V)) {
+        if (t_frc) pt_begin(t_frc);
+        RSVDT_CHK(folded_forcing(A, dir, V->TS.dt, k, Nwe, V->TS.Ns, D->idft->d, Fhat->d, Fhat->d));
+        if (t_frc) pt_end(t_frc);
+        RSVDT_CHK(leap_stepping(A, D, V, Fhat->d, Yall, t_rk4, t_frc, &launches));
+        g_rsvdt.stats.steps = rend;
+        g_rsvdt.stats.rk4_launches = launches;
+        g_rsvdt.stats.chunk_steps = (int)V->TS.ResRatio;
+        return 0;
+    }
     double *y64 = NULL;          /* the FP32 state at step Nt, widened */
     stepper st;
     memset(&st, 0, sizeof(st));
@@ -1114,13 +1242,25 @@ static PetscErrorCode mtilde_group(LNS_vars *LNS, RSVDt_vars *V, TS_removal_matr
      * rows are gathered.  The basis work arrays E and T are free once the
      * basis is built. */
     double *Vblk = g_trg.E, *MV = g_trg.T;
+    const int dir = V->TS.DirAdj ? 1 : 0;
     double t0 = trt_mark();
-    int h = rsvdt_hip_transpose_rows(N, Ns1, g, 0, g, g_trg.V, Vblk, 1, g_rsvdt.stream);
-    if (h) return rsvdt_err(h, "CreateMtilde", "device call failed: %s", rsvdt_hip_last_error());
-    RSVDT_CHK(rsvdt_homogeneous_steps(LNS->A, V->TS.DirAdj ? 1 : 0, V->TS.dt, V->TS.ResRatio, Vblk, N, g, Ns1));
-    trt_add(TRT_STEPS, t0);
-    t0 = trt_mark();
-    h = rsvdt_hip_transpose_rows(N, Ns1, g, 0, g, Vblk, MV, 0, g_rsvdt.stream);
+    int h = 0;
+    if (leap_pays(LNS->A, dir, V)) {
+        /* the operator's dense propagator (the stepping of the same action built
+         * it) on the basis as it lies, N x Ns1 per test vector */
+        const double *E;
+        RSVDT_CHK(leap_operator(LNS->A, dir, V->TS.dt, V->TS.ResRatio, &E));
+        h = rsvdt_hip_dense_apply(N, Ns1, g, E, g_trg.V, NULL, MV, g_rsvdt.stream);
+        trt_add(TRT_STEPS, t0);
+        t0 = trt_mark();
+    } else {
+        h = rsvdt_hip_transpose_rows(N, Ns1, g, 0, g, g_trg.V, Vblk, 1, g_rsvdt.stream);
+        if (h) return rsvdt_err(h, "CreateMtilde", "device call failed: %s", rsvdt_hip_last_error());
+        RSVDT_CHK(rsvdt_homogeneous_steps(LNS->A, dir, V->TS.dt, V->TS.ResRatio, Vblk, N, g, Ns1));
+        trt_add(TRT_STEPS, t0);
+        t0 = trt_mark();
+        h = rsvdt_hip_transpose_rows(N, Ns1, g, 0, g, Vblk, MV, 0, g_rsvdt.stream);
+    }
     if (h) return rsvdt_err(h, "CreateMtilde", "device call failed: %s", rsvdt_hip_last_error());
     void *work = rsvdt_scratch(SCR_WORK, rsvdt_hip_bgram_work_bytes(g, N, Ns1, Ns1));
     if (!work) return rsvdt_err(RSVDT_ERR_MEM, "CreateMtilde", "cannot allocate work");

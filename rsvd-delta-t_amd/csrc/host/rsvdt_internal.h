@@ -76,6 +76,9 @@ struct _p_RSVDT_Mat {
      * workgroup */
     int mt_ok[2], mt_lanes[2], mt_variant[2], mt_tile[2], mt_bpw[2];
     PetscInt mt_k[2];
+    /* dense N x N propagator of `steps` homogeneous RK4 steps of size h,
+     * [0: A, 1: A^H], of an operator that fits in LDS (built on first use) */
+    struct { double h; PetscInt steps; double *d; } leap[2];
 };
 
 struct _p_RSVDT_Vec {

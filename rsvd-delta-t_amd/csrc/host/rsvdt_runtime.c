@@ -467,6 +467,7 @@ PetscErrorCode RSVDT_MatDestroy(Mat *pm)
             rsvdt_hip_free(m->tiled[d][i].d_tcol);
             rsvdt_hip_free(m->tiled[d][i].d_lidx);
         }
+    for (int d = 0; d < 2; d++) rsvdt_hip_free(m->leap[d].d);
     free(m->h_rowptrH); free(m->h_colH);
     free(m->h_rowptr); free(m->h_col); free(m->h_val);
     free(m);

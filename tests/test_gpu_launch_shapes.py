@@ -109,3 +109,52 @@ def test_apply_gram_rejects_wide(L, pkg):
     L.rsvdt_hip_bapply_gram.argtypes = [I64] * 3 + [V, I64, I64, V, V, V, V, V]
     assert L.rsvdt_hip_bapply_gram(1, 4, 65, d.p, 260, 65, d.p, d.p, None, None, None) == 102
     assert L.rsvdt_hip_bapply_gram(1, 4, 8, d.p, 32, 8, d.p, d.p, d.p, None, None) == 102
+
+
+@pytest.mark.parametrize("N", [1, 3, 15, 16, 17, 33, 130, 515])
+@pytest.mark.parametrize("k,nb", [(1, 1), (10, 1), (16, 1), (17, 2), (16, 16), (257, 1), (13, 25)])
+def test_dense_apply_sizes(L, pkg, N, k, nb):
+    rng = np.random.default_rng(N + k)
+    E, X, F = crandn(rng, N, N) / np.sqrt(N), crandn(rng, nb, N, k), crandn(rng, nb, N, k)
+    L.rsvdt_hip_dense_apply.argtypes = [I64] * 3 + [V] * 5
+    dE, dX, dF, dO = Dev(pkg, E), Dev(pkg, X), Dev(pkg, F), Dev(pkg, nbytes=X.nbytes)
+    for f in (None, dF):
+        assert L.rsvdt_hip_dense_apply(N, k, nb, dE.p, dX.p, f.p if f else None, dO.p, None) == 0
+        ref = np.einsum("ra,bac->brc", E, X) + (F if f else 0)
+        assert np.max(np.abs(dO.get(np.complex128, X.shape) - ref)) <= 8 * EPS * (N + 1) * np.abs(E).max() * np.abs(X).max() + 4 * EPS * np.abs(F).max()
+    assert L.rsvdt_hip_dense_apply(N, k, nb, dE.p, dX.p, None, dX.p, None) == 102      # never in place
+
+
+def _band_operator(N, real, width, rng):
+    import scipy.sparse as sp
+    offs = range(-(width // 2), width // 2 + 1)
+    d = [rng.standard_normal(max(N - abs(o), 0)) + (0 if real else 1j * rng.standard_normal(max(N - abs(o), 0)))
+         for o in offs]
+    return (sp.diags(d, list(offs), shape=(N, N)) - (1 + width) * sp.eye(N)).tocsr().astype(np.complex128)
+
+
+@pytest.mark.parametrize("N,real,width", [(20, False, 3), (64, True, 3), (129, False, 7), (500, False, 3), (700, True, 5)])
+@pytest.mark.parametrize("k,Nw,TL,removal", [(1, 8, 0.0, False), (3, 16, 1.0, True), (16, 15, 2.37, False), (5, 16, 7.9, True)])
+@pytest.mark.parametrize("direct", [True, False])
+def test_leaps_match_steps(pkg, N, real, width, k, Nw, TL, removal, direct):
+    """Snapshots by dense propagator products (one per snapshot) against the
+    stage kernels' step-by-step run: whole and partial leaps before the first
+    snapshot, none at all, odd numbers of frequencies, both directions."""
+    if removal and Nw + 1 > N:
+        pytest.skip("more snapshots than rows")
+    rng = np.random.default_rng(N + k)
+    A = _band_operator(N, real, width, rng)
+    kw = dict(k=k, q=0, Nw=Nw, w=0.7, TL=TL, dt=0.04, transient_removal=removal)
+    out = {}
+    for fuse in (1, 0):
+        s = pkg.Session(A, fuse_small=fuse, **kw)
+        if fuse == 1:
+            F = crandn(rng, N, k * s.Nw_eff)
+        s.set_sketch(F)
+        s.direct() if direct else s.adjoint()
+        out[fuse] = s.get_Y()
+        st = pkg.action_stats()
+        if fuse:
+            assert st["chunk_steps"] == s.RR and st["rk4_launches"] < st["steps"] // 2
+        s.close()
+    assert rel(out[1], out[0]) < (1e-9 if removal else 1e-12)
