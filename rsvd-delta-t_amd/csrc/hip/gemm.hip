@@ -29,6 +29,10 @@ namespace rsvdt {
 typedef double dvec4 __attribute__((ext_vector_type(4)));
 typedef double dvec2 __attribute__((ext_vector_type(2)));
 
+// The wave's index in its workgroup, as a scalar: loops and branches on it stay
+// uniform for the compiler.
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
+
 template <int T, typename OV>
 __global__ __launch_bounds__(256) void k_coef_gemm(
     int64_t P, int64_t K, int64_t L, const double2 *__restrict__ coef, int64_t cq, int64_t cp, int64_t p0,
@@ -254,7 +258,7 @@ __global__ __launch_bounds__(256, TA *TC <= 1 ? 4 : (TA == 4 && !HERM ? 2 : 1)) 
     constexpr int PF = TA * TC == 1 ? (HERM ? 8 : 4) : (WA * TC <= 4 ? 2 : 1);
     constexpr int CW = 16 * TC, RS = 4 * NSUB;   // columns of the macro tile; rows of the workgroup's step
     extern __shared__ double2 gsm[];             // 16 TA x 16 TC, then the borders: 16 TA, 16 TC, 1
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = wave_id();
     const int h = wv % GA, sub = wv / GA;
     const int64_t b = blockIdx.z;
     const int a0 = (int)(blockIdx.y / ntc) * (16 * TA), c0 = (int)(blockIdx.y % ntc) * CW;
@@ -533,82 +537,153 @@ __global__ __launch_bounds__(256) void k_bapply(
 // FP64 MFMA batched apply for unit column strides:
 //   Out_b(r, c) = alpha Y_b(r, c) + sum_a X_b(r, a) C_b(a, c).
 // grid.y = column tile of 16 TC columns; the workgroup stages C_b(:, tile) in
-// LDS once and its waves walk 32-row tiles (grid-stride).  A(16x4): lane i ->
+// LDS once and its waves walk 16-row tiles (grid-stride).  A(16x4): lane i ->
 // X(r0 + i%16, a0 + i/16); B(4x16): lane i -> C(a0 + i/16, c0 + i%16);
-// D: lane i holds Out(r0 + 4j + i/16, c0 + i%16).  With one column tile a
-// wave reads all of its rows before it writes them, so Out may alias X; Out
-// may always alias Y (read and written by the same lane).
-template <int TC>
+// D: lane i holds Out(r0 + 4j + i/16, c0 + i%16).  The (row tile, 4-column
+// step) sequence of a wave is one stream with PF steps of X in flight, across
+// tile boundaries too.  With one column tile a wave's loads of a row tile are
+// all issued before it writes the tile, and no other wave reads those rows, so
+// Out may alias X; Out may always alias Y (read and written by the same lane).
+// BORD: a last column beyond the 16-wide tiles (nc = 16 T + 1, the bases of
+// Nw + 1 snapshots) is a plain FMA sum on the operands the lanes hold.
+// Bound by memory and FP64 MFMA together at 32 columns (61 % of the cycles
+// hold an MFMA), by MFMA above.  8 batches of 98,304 x 65 times 65 x 32: 340 us,
+// with Y 372 us, 4.4 TB/s (413 and 520 us with one step in flight); PF = 8 is
+// slower (385 us), 16 x 16 chunks turned through LDS too (383 us).
+template <int TC, bool BORD>
 __global__ __launch_bounds__(256) void k_bapply_mfma(
-    int64_t nrows, int64_t na, int64_t nc, const double2 *X, int64_t xb, int64_t xr,
+    int64_t nrows, int na, int nc, const double2 *X, int64_t xb, int64_t xr,
     const double2 *__restrict__ C, double alpha, const double2 *Y, int64_t yb, int64_t yr,
     double2 *Out, int64_t ob, int64_t orow)
 {
-    extern __shared__ double2 cs_b[];               // [na4][16 TC]
-    constexpr int CW = 16 * TC;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    extern __shared__ double2 cs_b[];               // [na4][16 TC], then the border column [na4]
+    constexpr int CW = 16 * TC, PF = 4;
+    const int lane = threadIdx.x & 63, wv = wave_id();
     const int64_t b = blockIdx.z;
-    const int64_t c0 = (int64_t)blockIdx.y * CW;
-    const int64_t na4 = (na + 3) & ~(int64_t)3;
+    const int c0 = (int)blockIdx.y * CW;
+    const int na4 = (na + 3) & ~3, nks = na4 >> 2;
+    const int nc_t = BORD ? nc - 1 : nc;            // columns in tiles
+    const bool do_b = BORD && blockIdx.y == gridDim.y - 1;
     const double2 *Cb = C + b * na * nc;
-    for (int64_t e = threadIdx.x; e < na4 * CW; e += blockDim.x) {
-        const int64_t a = e / CW, c = c0 + e % CW;
-        cs_b[e] = (a < na && c < nc) ? Cb[a * nc + c] : make_double2(0, 0);
+    for (int e = threadIdx.x; e < na4 * CW; e += 256) {
+        const int a = e / CW, c = c0 + e % CW;
+        double2 v = make_double2(0, 0);
+        if (a < na && c < nc_t) v = Cb[(int64_t)a * nc + c];
+        cs_b[e] = v;
+    }
+    double2 *cb_l = cs_b + (int64_t)na4 * CW;
+    if constexpr (BORD) {
+        for (int a = threadIdx.x; a < na4; a += 256) {
+            double2 v = make_double2(0, 0);
+            if (a < na) v = Cb[(int64_t)a * nc + nc - 1];
+            cb_l[a] = v;
+        }
     }
     __syncthreads();
     const int kr = lane >> 4, cl = lane & 15;
     const double2 *Xb = X + b * xb;
-    const double2 zero = make_double2(0, 0);
-    const int64_t ntile = (nrows + 31) / 32;
-    for (int64_t tile = (int64_t)blockIdx.x * 4 + wv; tile < ntile; tile += (int64_t)gridDim.x * 4) {
-        const int64_t r0 = tile * 32;
-        dvec4 dr[2][TC], di[2][TC];
+    const int64_t ntile = (nrows + 15) / 16, step = (int64_t)gridDim.x * 4;
+    int64_t tile = (int64_t)blockIdx.x * 4 + wv;
+    if (tile >= ntile) return;
+    // load position: step ls of row tile lt (clamped to the last tile and row)
+    int64_t lt = tile;
+    int ls = 0;
+    auto row_ptr = [&](int64_t t) {
+        int64_t r = (t < ntile ? t : ntile - 1) * 16 + cl;
+        if (r >= nrows) r = nrows - 1;
+        return Xb + r * xr;
+    };
+    const double2 *lp = row_ptr(lt);
+    double2 ring[PF];
+    auto load = [&](int p) {
+        const int a = 4 * ls + kr;
+        ring[p] = lp[a < na ? a : na - 1];
+        if (++ls == nks) { ls = 0; lt += step; lp = row_ptr(lt); }
+    };
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+    for (int p = 0; p < PF; ++p) load(p);
+    dvec4 dr[TC], di[TC];
+    double2 bd = make_double2(0, 0);
 #pragma unroll
-            for (int u = 0; u < TC; ++u) { dr[t][u] = (dvec4){0, 0, 0, 0}; di[t][u] = (dvec4){0, 0, 0, 0}; }
-        bool rok[2];
+    for (int u = 0; u < TC; ++u) { dr[u] = (dvec4){0, 0, 0, 0}; di[u] = (dvec4){0, 0, 0, 0}; }
+    int ks = 0;
+    while (tile < ntile) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t) rok[t] = r0 + 16 * t + cl < nrows;
-        double2 xv[2];
+        for (int p = 0; p < PF; ++p) {
+            if (tile < ntile) {
+                const int a = 4 * ks + kr;
+                const bool ok = a < na;             // a column past the end has no product (X may hold anything there)
+                const double2 x = make_double2(ok ? ring[p].x : 0.0, ok ? ring[p].y : 0.0);
+                load(p);
+                const double2 *crow = cs_b + a * CW + cl;
+                double2 cv[TC];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) xv[t] = (rok[t] && kr < na) ? Xb[(r0 + 16 * t + cl) * xr + kr] : zero;
-        for (int64_t a0 = 0; a0 < na4; a0 += 4) {
-            const int64_t a = a0 + kr, an = a + 4;
-            double2 xn[2];
+                for (int u = 0; u < TC; ++u) cv[u] = crow[16 * u];
 #pragma unroll
-            for (int t = 0; t < 2; ++t) xn[t] = (rok[t] && an < na) ? Xb[(r0 + 16 * t + cl) * xr + an] : zero;
-            const double2 *crow = cs_b + a * CW + cl;
+                for (int u = 0; u < TC; ++u) {
+                    dr[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.x, cv[u].x, dr[u], 0, 0, 0);
+                    di[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.x, cv[u].y, di[u], 0, 0, 0);
+                }
 #pragma unroll
-            for (int u = 0; u < TC; ++u) {
-                const double2 cv = crow[16 * u];
+                for (int u = 0; u < TC; ++u) {
+                    dr[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(-x.y, cv[u].y, dr[u], 0, 0, 0);
+                    di[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.y, cv[u].x, di[u], 0, 0, 0);
+                }
+                if constexpr (BORD) {
+                    if (do_b) bd = zadd(bd, zmul(x, cb_l[a]));
+                }
+                if (++ks == nks) {                  // tile done: store and restart the sums
+                    const int64_t r0 = tile * 16;
+                    double2 yv[4][TC];              // clamped addresses: all loads in flight at once
+                    if (Y != nullptr) {
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    dr[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[t].x, cv.x, dr[t][u], 0, 0, 0);
-                    dr[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(-xv[t].y, cv.y, dr[t][u], 0, 0, 0);
-                    di[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[t].x, cv.y, di[t][u], 0, 0, 0);
-                    di[t][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[t].y, cv.x, di[t][u], 0, 0, 0);
+                        for (int j = 0; j < 4; ++j) {
+                            const int64_t r = r0 + 4 * j + kr < nrows ? r0 + 4 * j + kr : nrows - 1;
+#pragma unroll
+                            for (int u = 0; u < TC; ++u) {
+                                const int c = c0 + 16 * u + cl < nc_t ? c0 + 16 * u + cl : nc_t - 1;
+                                yv[j][u] = Y[b * yb + r * yr + c];
+                            }
+                        }
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+#pragma unroll
+                            for (int u = 0; u < TC; ++u) yv[j][u] = make_double2(0, 0);
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int64_t r = r0 + 4 * j + kr;
+#pragma unroll
+                        for (int u = 0; u < TC; ++u) {
+                            const int c = c0 + 16 * u + cl;
+                            double2 o = make_double2(dr[u][j], di[u][j]);
+                            if (Y != nullptr) { o.x += alpha * yv[j][u].x; o.y += alpha * yv[j][u].y; }
+                            if (r < nrows && c < nc_t) Out[b * ob + r * orow + c] = o;
+                        }
+                    }
+                    if constexpr (BORD) {
+                        if (do_b) {
+                            bd.x += __shfl_xor(bd.x, 16, 64); bd.y += __shfl_xor(bd.y, 16, 64);
+                            bd.x += __shfl_xor(bd.x, 32, 64); bd.y += __shfl_xor(bd.y, 32, 64);
+                            const int64_t r = r0 + cl;
+                            if (kr == 0 && r < nrows) {
+                                if (Y != nullptr) {
+                                    const double2 yv = Y[b * yb + r * yr + nc - 1];
+                                    bd.x += alpha * yv.x; bd.y += alpha * yv.y;
+                                }
+                                Out[b * ob + r * orow + nc - 1] = bd;
+                            }
+                            bd = make_double2(0, 0);
+                        }
+                    }
+                    ks = 0;
+                    tile += step;
+#pragma unroll
+                    for (int u = 0; u < TC; ++u) { dr[u] = (dvec4){0, 0, 0, 0}; di[u] = (dvec4){0, 0, 0, 0}; }
                 }
             }
-#pragma unroll
-            for (int t = 0; t < 2; ++t) xv[t] = xn[t];
         }
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int u = 0; u < TC; ++u)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int64_t r = r0 + 16 * t + 4 * j + kr, c = c0 + 16 * u + cl;
-                    if (r < nrows && c < nc) {
-                        double2 o = make_double2(dr[t][u][j], di[t][u][j]);
-                        if (Y != nullptr) {
-                            const double2 yv = Y[b * yb + r * yr + c];
-                            o.x += alpha * yv.x; o.y += alpha * yv.y;
-                        }
-                        Out[b * ob + r * orow + c] = o;
-                    }
-                }
     }
 }
 
@@ -633,7 +708,7 @@ __global__ __launch_bounds__(256) void k_bapply_gram(int64_t nrows, int n, const
 {
     constexpr int RT = TC == 1 ? 2 : 1, CW = 16 * TC, NS = 4 * TC;
     extern __shared__ double2 gsm[];             // C_b [CW][CW], then the workgroup's Gram sums
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, kr = lane >> 4, cl = lane & 15;
+    const int lane = threadIdx.x & 63, wv = wave_id(), kr = lane >> 4, cl = lane & 15;
     const int64_t b = blockIdx.z;
     const double2 *Cb = C + b * n * n;
     for (int e = threadIdx.x; e < CW * CW; e += 256) {
@@ -792,7 +867,7 @@ __global__ __launch_bounds__(512) void k_dense_apply(int N, int k, int ncol, con
 {
     constexpr int PF = CT == 1 ? 8 : 4, CW = 16 * CT;
     __shared__ double2 red[8][16][CW];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, kr = lane >> 4, cl = lane & 15;
+    const int lane = threadIdx.x & 63, wv = wave_id(), kr = lane >> 4, cl = lane & 15;
     const int r0 = blockIdx.x * 16, c0 = blockIdx.y * CW;
     const int64_t bs = (int64_t)N * k;
     const double2 *er = E + (int64_t)min(r0 + cl, N - 1) * N;
@@ -945,21 +1020,20 @@ extern "C" int rsvdt_hip_bgram(int64_t nbatch, int64_t nrows, int64_t na, int64_
     return RSVDT_HIP_OK;
 }
 
-template <int TC>
-static int launch_bapply_mfma(int64_t nbatch, int64_t nrows, int64_t na, int64_t nc, const double *X, int64_t xb,
-                              int64_t xr, const double *C, double alpha, const double *Y, int64_t yb, int64_t yr,
-                              double *Out, int64_t ob, int64_t orow, hipStream_t s)
+template <int TC, bool BORD>
+static int launch_bapply_mfma(int64_t nct, int64_t nbatch, int64_t nrows, int64_t na, int64_t nc, const double *X,
+                              int64_t xb, int64_t xr, const double *C, double alpha, const double *Y, int64_t yb,
+                              int64_t yr, double *Out, int64_t ob, int64_t orow, hipStream_t s)
 {
-    const int64_t nct = (nc + 16 * TC - 1) / (16 * TC);
     const int64_t na4 = (na + 3) & ~(int64_t)3;
-    const size_t lds = (size_t)na4 * 16 * TC * 16;
-    const int64_t ntile = (nrows + 31) / 32;
+    const size_t lds = (size_t)na4 * (16 * TC + (BORD ? 1 : 0)) * 16;
+    const int64_t ntile = (nrows + 15) / 16;
     int64_t gx = (ntile + 3) / 4;
-    const int64_t cap = (2048 + nct * nbatch - 1) / (nct * nbatch);
+    const int64_t cap = (1024 + nct * nbatch - 1) / (nct * nbatch);       // four workgroups per CU
     if (gx > cap) gx = cap < 1 ? 1 : cap;
-    hipLaunchKernelGGL((k_bapply_mfma<TC>), dim3((unsigned)gx, (unsigned)nct, (unsigned)nbatch), dim3(256), lds, s,
-                       nrows, na, nc, (const double2 *)X, xb, xr, (const double2 *)C, alpha, (const double2 *)Y, yb,
-                       yr, (double2 *)Out, ob, orow);
+    hipLaunchKernelGGL((k_bapply_mfma<TC, BORD>), dim3((unsigned)gx, (unsigned)nct, (unsigned)nbatch), dim3(256), lds, s,
+                       nrows, (int)na, (int)nc, (const double2 *)X, xb, xr, (const double2 *)C, alpha,
+                       (const double2 *)Y, yb, yr, (double2 *)Out, ob, orow);
     RSVDT_LAUNCH_CHECK("rsvdt_hip_bapply(mfma)");
     return RSVDT_HIP_OK;
 }
@@ -978,18 +1052,24 @@ extern "C" int rsvdt_hip_bapply(int64_t nbatch, int64_t nrows, int64_t na, int64
     const bool unit = xa == 1 && oc == 1 && (Y == nullptr || yc == 1);
     const int64_t na4 = (na + 3) & ~(int64_t)3;
     if (unit && na > 0 && na4 * 64 * 16 <= 150 * 1024) {
-        const int TC = nc <= 16 ? 1 : (nc <= 32 ? 2 : (nc <= 48 ? 3 : (nc <= 64 ? 4 : 3)));
-        const bool multi_tile = nc > 16 * TC;
-        if (multi_tile && X == Out) {
+        // column tiles of at most 64, as even as their number allows; with more
+        // than one, rows are read by several workgroups, so not in place (65
+        // columns are one tile and a border, and stay refused as before)
+        const bool bord = nc > 16 && nc % 16 == 1;
+        const int64_t t16 = bord ? nc / 16 : (nc + 15) / 16, nct = (t16 + 3) / 4;
+        const int TC = (int)((t16 + nct - 1) / nct);
+        if (nc > 64 && X == Out) {
             set_error_msg("rsvdt_hip_bapply: in place needs nc <= 64 with unit strides");
             return RSVDT_HIP_ERR_ARG;
         }
-        switch (TC) {
-        case 1: return launch_bapply_mfma<1>(nbatch, nrows, na, nc, X, xb, xr, C, alpha, Y, yb, yr, Out, ob, orow, st);
-        case 2: return launch_bapply_mfma<2>(nbatch, nrows, na, nc, X, xb, xr, C, alpha, Y, yb, yr, Out, ob, orow, st);
-        case 3: return launch_bapply_mfma<3>(nbatch, nrows, na, nc, X, xb, xr, C, alpha, Y, yb, yr, Out, ob, orow, st);
-        default: return launch_bapply_mfma<4>(nbatch, nrows, na, nc, X, xb, xr, C, alpha, Y, yb, yr, Out, ob, orow, st);
-        }
+#define RSVDT_BA(T)                                                                                               \
+        if (TC == T)                                                                                              \
+            return bord ? launch_bapply_mfma<T, true>(nct, nbatch, nrows, na, nc, X, xb, xr, C, alpha, Y, yb, yr, \
+                                                      Out, ob, orow, st)                                          \
+                        : launch_bapply_mfma<T, false>(nct, nbatch, nrows, na, nc, X, xb, xr, C, alpha, Y, yb,    \
+                                                       yr, Out, ob, orow, st);
+        RSVDT_BA(1) RSVDT_BA(2) RSVDT_BA(3) RSVDT_BA(4)
+#undef RSVDT_BA
     }
     if (nc > 256 || na > 512) {
         set_error_msg("rsvdt_hip_bapply: nc <= 256, na <= 512 required");

@@ -158,3 +158,51 @@ def test_leaps_match_steps(pkg, N, real, width, k, Nw, TL, removal, direct):
             assert st["chunk_steps"] == s.RR and st["rk4_launches"] < st["steps"] // 2
         s.close()
     assert rel(out[1], out[0]) < (1e-9 if removal else 1e-12)
+
+
+@pytest.mark.parametrize("na,nc", [(1, 1), (5, 17), (16, 16), (33, 48), (65, 65), (65, 32), (65, 33), (64, 64), (129, 129),
+                                   (129, 64), (140, 65), (146, 64), (146, 97), (4, 200)])
+@pytest.mark.parametrize("nb,nr", [(1, 3), (3, 515), (2, 4100)])
+@pytest.mark.parametrize("with_y", [False, True])
+def test_apply_tiles(L, pkg, na, nc, nb, nr, with_y):
+    """Out = alpha Y + X C over column tiles, the border column and row
+    remainders; the entries of X past a row's end (the next row, or NaN after
+    the last) must not reach the result."""
+    rng = np.random.default_rng(na * 7 + nc + nr)
+    X, C, Y = crandn(rng, nb, nr, na), crandn(rng, nb, na, nc) / np.sqrt(na), crandn(rng, nb, nr, nc)
+    pad = np.full(64, np.nan + 1j * np.nan)
+    dX, dC, dY = Dev(pkg, np.concatenate([X.ravel(), pad])), Dev(pkg, C), Dev(pkg, Y)
+    dO = Dev(pkg, nbytes=Y.nbytes)
+    L.rsvdt_hip_bapply.argtypes = [I64] * 4 + [V, I64, I64, I64, V, ctypes.c_double, V, I64, I64, I64, V, I64, I64, I64, V]
+    assert L.rsvdt_hip_bapply(nb, nr, na, nc, dX.p, nr * na, na, 1, dC.p, 0.5, dY.p if with_y else None, nr * nc, nc, 1,
+                              dO.p, nr * nc, nc, 1, None) == 0
+    ref = np.einsum("bra,bac->brc", X, C) + (0.5 * Y if with_y else 0)
+    assert np.max(np.abs(dO.get(np.complex128, Y.shape) - ref)) <= 8 * EPS * (na + 1) * np.abs(X).max() * max(np.abs(C).max(), 1)
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 65, 140, 141, 150])
+def test_trmm_sizes(L, pkg, n):
+    rng = np.random.default_rng(n)
+    A, B = np.triu(crandn(rng, 3, n, n)), np.triu(crandn(rng, 3, n, n))
+    dA, dB, dC = Dev(pkg, A), Dev(pkg, B), Dev(pkg, nbytes=A.nbytes)
+    L.rsvdt_hip_btrmm_upper.argtypes = [I64, I64, V, V, V, V]
+    assert L.rsvdt_hip_btrmm_upper(3, n, dA.p, dB.p, dC.p, None) == 0
+    out = dC.get(np.complex128, A.shape)
+    assert np.max(np.abs(out - A @ B)) <= 8 * EPS * (n + 1) * np.abs(A).max() * np.abs(B).max()
+    assert np.all(np.tril(out, -1) == 0)
+
+
+@pytest.mark.parametrize("n,kt,b0,kb", [(1, 1, 0, 1), (65, 16, 8, 8), (65, 9, 2, 7), (3, 100, 1, 60), (129, 32, 0, 32),
+                                        (17, 5, 4, 1), (2, 3, 0, 3), (481, 16, 0, 16)])
+@pytest.mark.parametrize("N", [1, 2, 515])
+def test_transpose_row_groups(L, pkg, n, kt, b0, kb, N):
+    rng = np.random.default_rng(n + N)
+    src = crandn(rng, n, N, kt)
+    dS, dD, dB = Dev(pkg, src), Dev(pkg, nbytes=kb * N * n * 16), Dev(pkg, np.zeros_like(src))
+    L.rsvdt_hip_transpose_rows.argtypes = [I64] * 5 + [V, V, ctypes.c_int, V]
+    assert L.rsvdt_hip_transpose_rows(N, n, kt, b0, kb, dS.p, dD.p, 0, None) == 0
+    assert np.array_equal(dD.get(np.complex128, (kb, N, n)), src[:, :, b0:b0 + kb].transpose(2, 1, 0))
+    assert L.rsvdt_hip_transpose_rows(N, n, kt, b0, kb, dD.p, dB.p, 1, None) == 0
+    back = np.zeros_like(src)
+    back[:, :, b0:b0 + kb] = src[:, :, b0:b0 + kb]
+    assert np.array_equal(dB.get(np.complex128, src.shape), back)
