@@ -101,7 +101,8 @@ typedef struct {
     int prec;
     int lanes;            /* 0 = default choice */
     int xcd_remap;        /* workgroup -> rows map: 0 identity, 1 one contiguous row range per XCD,
-                             2 / 3 chunks of 64 / 256 row blocks dealt round-robin to the XCDs */
+                             2 / 3 chunks of 64 / 256 row blocks dealt round-robin to the XCDs
+                             (one block; with several the tiled forms choose by their tiles) */
     int variant;          /* 0: 16-nonzero gather batches; 1: + nontemporal row-local
                              streams; 2: 8-nonzero batches; 3: 8 + nontemporal; 4: 12-nonzero
                              batches; 5: 12 + nontemporal (variants 1-3 apply to the RK4 stage

@@ -4,9 +4,10 @@ import ctypes
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 from conftest import crandn, rel
-from gpu_util import Dev, init
+from gpu_util import Desc, Dev, init, tiled_form
 
 pytestmark = pytest.mark.gpu
 V, I64 = ctypes.c_void_p, ctypes.c_int64
@@ -206,3 +207,22 @@ def test_transpose_row_groups(L, pkg, n, kt, b0, kb, N):
     back = np.zeros_like(src)
     back[:, :, b0:b0 + kb] = src[:, :, b0:b0 + kb]
     assert np.array_equal(dB.get(np.complex128, src.shape), back)
+
+
+@pytest.mark.parametrize("ntile,nb,bpw", [(63, 2, 8), (64, 3, 1), (511, 3, 2), (513, 2, 1), (1100, 3, 8)])
+def test_tiles_of_several_blocks(L, pkg, ntile, nb, bpw):
+    """The Horner stage on several blocks, its tiles dealt to the XCDs in runs
+    (one run each, or runs of 64 and a rest): every tile once, no tile twice."""
+    rng = np.random.default_rng(ntile)
+    N, k, c = 32 * ntile - 5, 6, 0.03
+    A = sp.diags([rng.standard_normal(N - abs(o)) for o in (-40, -1, 0, 1, 40)], [-40, -1, 0, 1, 40], format="csr")
+    y = crandn(rng, nb, N, k)
+    tptr, tcol, lidx, hmax, emax = tiled_form(A, 32)
+    held = [Dev(pkg, x) for x in (A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data, tptr, tcol, lidx, y)]
+    rp, ci, v, tp, tc, li, dy = (h.p for h in held)
+    out = Dev(pkg, nbytes=y.nbytes)
+    d = Desc(N, k, nb, rp, ci, v, 1, 64, 8, 0, 9, 0, None, None, None, 32, hmax, emax, tp, tc, li, bpw)
+    L.rsvdt_hip_horner_stage.argtypes = [ctypes.POINTER(Desc), V, V, V, V, ctypes.c_double, V, V, V]
+    assert L.rsvdt_hip_horner_stage(ctypes.byref(d), dy, dy, None, None, c, out.p, None, None) == 0
+    ref = np.stack([y[b] + c * (A @ y[b]) for b in range(nb)])
+    assert rel(out.get(np.complex128, y.shape), ref) < 1e-14
