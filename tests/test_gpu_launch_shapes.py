@@ -226,3 +226,47 @@ def test_tiles_of_several_blocks(L, pkg, ntile, nb, bpw):
     assert L.rsvdt_hip_horner_stage(ctypes.byref(d), dy, dy, None, None, c, out.p, None, None) == 0
     ref = np.stack([y[b] + c * (A @ y[b]) for b in range(nb)])
     assert rel(out.get(np.complex128, y.shape), ref) < 1e-14
+
+
+@pytest.mark.parametrize("off,pad", [(0, 0), (0, 4), (1, 0), (0, 3)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (64, 64, 64), (68, 60, 68), (65, 63, 66), (132, 72, 130), (40, 64, 4100)])
+@pytest.mark.parametrize("ak,bk", [(True, True), (True, False), (False, True), (False, False)])
+def test_gemm_bf16_loads(L, pkg, M, N, K, ak, bk, off, pad):
+    """Both load widths of the BF16 GEMM: operands on and off a 16-byte
+    boundary (off), padded leading dimensions (pad), K-steps and tiles that do
+    not divide, and a split reduction."""
+    rng = np.random.default_rng(M + K)
+    A, B = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+
+    def put(X):                        # row-major with a padded row, `off` floats into its buffer
+        ld = X.shape[1] + pad
+        buf = np.full(off + X.shape[0] * ld, np.nan, np.float32)
+        buf[off:].reshape(X.shape[0], ld)[:, :X.shape[1]] = X
+        d = Dev(pkg, buf)
+        return d, d.p.value + 4 * off if isinstance(d.p, V) else d.p + 4 * off, ld
+
+    dA, pA, lda = put(A if ak else A.T)
+    dB, pB, ldb = put(B.T if bk else B)
+    dC = Dev(pkg, nbytes=M * N * 4)
+    L.rsvdt_hip_gemm_bf16.argtypes = [I64] * 3 + [V, I64, I64, V, I64, I64, V, I64, ctypes.c_int, V, V, I64, V]
+    assert L.rsvdt_hip_gemm_bf16(M, N, K, pA, lda if ak else 1, 1 if ak else lda, pB, 1 if bk else ldb,
+                                 ldb if bk else 1, dC.p, N, 0, None, None, 0, None) == 0
+
+    def bf16(X):
+        u = X.view(np.uint32).astype(np.uint64)
+        return ((u + 0x7fff + ((u >> 16) & 1)) & 0xffff0000).astype(np.uint32).view(np.float32).astype(np.float64)
+    ref = bf16(A) @ bf16(B)
+    assert np.max(np.abs(dC.get(np.float32, (M, N)) - ref)) <= 6e-8 * 4 * np.sqrt(K) * max(1.0, np.max(np.abs(ref)))
+
+
+@pytest.mark.parametrize("M", [1, 3, 31, 127, 128, 129, 1000])
+@pytest.mark.parametrize("N,lda", [(1, 1), (63, 70), (64, 64), (200, 200)])
+def test_colsum_sizes(L, pkg, M, N, lda):
+    """Column sums over row chunks that the four row slots do not divide."""
+    rng = np.random.default_rng(M + N)
+    A = rng.standard_normal((M, lda)).astype(np.float32)
+    dA, out = Dev(pkg, A), Dev(pkg, np.full(N, np.nan, np.float32))
+    L.rsvdt_hip_colsum.argtypes = [I64, I64, V, I64, V, V]
+    assert L.rsvdt_hip_colsum(M, N, dA.p, lda, out.p, None) == 0
+    ref = A[:, :N].astype(np.float64).sum(0)
+    assert np.max(np.abs(out.get(np.float32, (N,)) - ref)) <= 6e-8 * M * np.max(np.abs(A))
