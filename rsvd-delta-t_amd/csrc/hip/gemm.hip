@@ -42,7 +42,7 @@ __global__ __launch_bounds__(256) void k_coef_gemm(
     extern __shared__ double2 cs[];                 // [Kpad][T*16 + 4]
     constexpr int PW = T * 16;
     constexpr int PS = PW + 4;                      // row pitch: the 4 rows a K-step reads hit different banks
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = wave_id();
     const int64_t pbase = (int64_t)blockIdx.y * PW;
     const int64_t Kpad = (K + 3) & ~(int64_t)3;
     for (int64_t e = threadIdx.x; e < Kpad * PW; e += 256) {
@@ -59,34 +59,41 @@ __global__ __launch_bounds__(256) void k_coef_gemm(
     const int kq = lane >> 4, cl = lane & 15;
     const int64_t ntile = (L + 63) / 64;
     // The workgroup's (tile, K-step) sequence is walked as one stream with the
-    // streamed operand loaded PF steps ahead, across tile boundaries too
-    // (measured on the 64 x 64 x 6.3M forcing chunk: PF = 2, 4, 8, 12, 16 ->
-    // 74.6, 69.5, 66.4, 65.0, 65.7 us per sample).
+    // streamed operand loaded PF steps ahead, across tile boundaries too; both
+    // ends of the stream count steps and move pointers (finding a step's tile by
+    // 64-bit division cost more vector instructions than all the rest).  Bound
+    // by the FP64 matrix cores: the 64 x 64 x 6.3M forcing chunk takes 3.78 ms
+    // (4.18 ms with divisions), 81 % of their cycles at the 2.05 GHz that this
+    // load runs at; PF = 8, 12, 16: 3.87, 3.78, 3.82 ms.
     constexpr int PF = 12;
     const int nks = (int)(Kpad >> 2);
     const int64_t nmine = blockIdx.x < ntile ? (ntile - 1 - blockIdx.x) / gridDim.x + 1 : 0;
-    const int64_t nsteps = nmine * nks;
-    auto load_step = [&](int64_t gs) -> double2 {
-        if (gs >= nsteps) return make_double2(0, 0);
-        const int64_t it = gs / nks, q = (gs - it * nks) * 4 + kq;
-        const int64_t l = (blockIdx.x + it * gridDim.x) * 64 + wv * 16 + cl;
-        return (l < L && q < K) ? in[q * ldi + l] : make_double2(0, 0);
+    const int64_t nsteps = nmine * nks, hop = (int64_t)gridDim.x * 64;
+    int64_t lo = (int64_t)blockIdx.x * 64 + wv * 16 + cl, ll = lo, lleft = nsteps;
+    int lks = 0, ks = 0;
+    const double2 *lp = in + (kq < K ? kq : 0) * ldi;
+    auto load_step = [&]() -> double2 {
+        double2 v = make_double2(0, 0);
+        if (lleft > 0) {
+            if (ll < L && lks * 4 + kq < K) v = lp[ll];
+            --lleft;
+            lp += 4 * ldi;
+            if (++lks == nks) { lks = 0; ll += hop; lp = in + (kq < K ? kq : 0) * ldi; }
+        }
+        return v;
     };
     double2 ring[PF];
 #pragma unroll
-    for (int p = 0; p < PF; ++p) ring[p] = load_step(p);
+    for (int p = 0; p < PF; ++p) ring[p] = load_step();
     dvec4 ar[T], ai[T];
 #pragma unroll
     for (int t = 0; t < T; ++t) { ar[t] = (dvec4){0, 0, 0, 0}; ai[t] = (dvec4){0, 0, 0, 0}; }
     for (int64_t g0 = 0; g0 < nsteps; g0 += PF) {
 #pragma unroll
         for (int p = 0; p < PF; ++p) {
-            const int64_t gs = g0 + p;
-            if (gs < nsteps) {
+            if (g0 + p < nsteps) {
                 const double2 x = ring[p];
-                ring[p] = load_step(gs + PF);
-                const int64_t it = gs / nks;
-                const int ks = (int)(gs - it * nks);
+                ring[p] = load_step();
                 const double2 *crow = cs + ((int64_t)ks * 4 + kq) * PS + cl;
                 double2 c[T];
 #pragma unroll
@@ -102,8 +109,10 @@ __global__ __launch_bounds__(256) void k_coef_gemm(
                     ar[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-c[t].y, x.y, ar[t], 0, 0, 0);
                     ai[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(c[t].y, x.x, ai[t], 0, 0, 0);
                 }
-                if (ks == nks - 1) {                  // tile done: store and restart the sums
-                    const int64_t l = (blockIdx.x + it * gridDim.x) * 64 + wv * 16 + cl;
+                if (++ks == nks) {                    // tile done: store and restart the sums
+                    ks = 0;
+                    const int64_t l = lo;
+                    lo += hop;
                     if (l < L) {
 #pragma unroll
                         for (int t = 0; t < T; ++t)

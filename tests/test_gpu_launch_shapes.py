@@ -270,3 +270,23 @@ def test_colsum_sizes(L, pkg, M, N, lda):
     assert L.rsvdt_hip_colsum(M, N, dA.p, lda, out.p, None) == 0
     ref = A[:, :N].astype(np.float64).sum(0)
     assert np.max(np.abs(out.get(np.float32, (N,)) - ref)) <= 6e-8 * M * np.max(np.abs(A))
+
+
+@pytest.mark.parametrize("P,K,ncol", [(1, 1, 1), (5, 3, 65), (16, 4, 63), (17, 5, 64), (64, 52, 700), (31, 3, 140001),
+                                      (64, 64, 133000), (130, 20, 1000)])
+@pytest.mark.parametrize("prec,beta", [(64, 0.0), (64, 0.5), (32, 0.0)])
+def test_coef_gemm_stream(L, pkg, P, K, ncol, prec, beta):
+    """The streamed coefficient product: fewer and more K-steps than are in
+    flight, one and several column tiles a workgroup, ragged last tiles."""
+    rng = np.random.default_rng(P + K + ncol)
+    cmod = P + 3
+    C, X, Y = crandn(rng, K, cmod), crandn(rng, K, ncol), crandn(rng, P, ncol)
+    cdt = np.complex128 if prec == 64 else np.complex64
+    dC, dX, dY = Dev(pkg, C), Dev(pkg, X), Dev(pkg, Y.astype(cdt))
+    L.rsvdt_hip_coef_gemm.argtypes = [I64, I64, I64, V, I64, I64, I64, ctypes.c_int, I64, ctypes.c_double, V, I64, V,
+                                      I64, ctypes.c_int, ctypes.c_double, V]
+    assert L.rsvdt_hip_coef_gemm(P, K, ncol, dC.p, cmod, 1, 2, -1, cmod, 0.7, dX.p, ncol, dY.p, ncol, prec, beta,
+                                 None) == 0
+    ref = 0.7 * (C[:, (2 - np.arange(P)) % cmod].T @ X) + beta * Y
+    tol = (4 * K * EPS if prec == 64 else 2.4e-7) * max(1.0, np.max(np.abs(ref)))
+    assert np.max(np.abs(dY.get(cdt, (P, ncol)) - ref)) <= tol
