@@ -1178,27 +1178,73 @@ extern "C" int rsvdt_hip_horner_stage(const rsvdt_spmm_desc *d, const void *vin,
 // matrices of SourceCode/ApplyWeightMats.c:16-80 and SVDAllFreqs.c:63-64
 // applied to all frequencies at once).  M is rows x cols CSR, complex FP64;
 // In blocks are cols x k, Out blocks rows x k.
+//
+// k lanes own a row (any k up to 256, not a power of two: a workgroup is a
+// flat run of 256 / k rows).  Bound by latency: neighbouring rows gather the
+// same rows of In, so few distinct bytes are in flight unless a wave works on
+// several blocks at once.  It gathers two entries for BB blocks together (four,
+// or as many as there are), the row's first entries kept in registers over the
+// bpw blocks a workgroup forms.
+// 393,216 x 16, 8 blocks, 1 to 5 entries a row: 591 us one block and entry at
+// a time, 557 with six entries of one block in flight, 345 as here (4.8 TB/s;
+// four blocks x three entries, two x three, eight x three: 1 %, 6 %, 18 % more).
 namespace rsvdt {
-__global__ __launch_bounds__(256) void k_spmm_blocks(int nrows, int k, int lpr, const int32_t *__restrict__ rowptr,
+template <bool NT, int BB>
+__global__ __launch_bounds__(256) void k_spmm_blocks(int nrows, int k, int kl, int rpb, int nb, int bpw,
+                                                     const int32_t *__restrict__ rowptr,
                                                      const int32_t *__restrict__ colidx, const double2 *__restrict__ val,
                                                      const double2 *__restrict__ in, int64_t ibs,
                                                      double2 *__restrict__ out, int64_t obs)
 {
-    const int rpb = 256 / lpr;
-    const int lane = threadIdx.x % lpr;
-    const int row = blockIdx.x * rpb + threadIdx.x / lpr;
-    if (row >= nrows) return;
-    const double2 *ib = in + (int64_t)blockIdx.y * ibs;
-    double2 *ob = out + (int64_t)blockIdx.y * obs;
-    for (int j = lane; j < k; j += lpr) {
-        double sr = 0, si = 0;
-        for (int e = rowptr[row]; e < rowptr[row + 1]; ++e) {
-            const double2 a = val[e], x = ib[(int64_t)colidx[e] * k + j];
-            sr += a.x * x.x - a.y * x.y;
-            si += a.x * x.y + a.y * x.x;
+    constexpr int ME = BB == 1 ? 1 : 2;         // entries in flight, for each of BB blocks
+    // the quotient: half a unit from any whole number, exact for 256 threads
+    const int slot = (int)(((float)threadIdx.x + 0.5f) * (1.0f / (float)kl)), lane = threadIdx.x - slot * kl;
+    const int64_t row = (int64_t)xcd_block(blockIdx.x, gridDim.x, gridDim.x < 512 ? 1 : 2) * rpb + slot;
+    if (slot >= rpb || row >= nrows) return;
+    const int e0 = rowptr[row], e1 = rowptr[row + 1];
+    int64_t co[ME];
+    double2 av[ME];
+    int held = e0;                              // first of the entries in registers
+    auto entries = [&](int eb) {
+        held = eb;
+#pragma unroll
+        for (int u = 0; u < ME; ++u)
+            if (eb + u < e1) {
+                co[u] = (int64_t)colidx[eb + u] * k;
+                av[u] = val[eb + u];
+            }
+    };
+    entries(e0);
+    const int b0 = blockIdx.y * bpw, b1 = nb - b0 < bpw ? nb : b0 + bpw;
+    for (int b = b0; b < b1; b += BB)
+        for (int j = lane; j < k; j += kl) {
+            const double2 *ib = in + (int64_t)b * ibs + j;
+            double sr[BB], si[BB];
+#pragma unroll
+            for (int q = 0; q < BB; ++q) { sr[q] = 0; si[q] = 0; }
+            for (int eb = e0; eb < e1; eb += ME) {
+                if (eb != held) entries(eb);
+                double2 x[BB][ME];
+#pragma unroll
+                for (int q = 0; q < BB; ++q)
+                    if (b + q < b1)
+#pragma unroll
+                        for (int u = 0; u < ME; ++u)
+                            if (eb + u < e1) x[q][u] = ib[q * ibs + co[u]];
+#pragma unroll
+                for (int u = 0; u < ME; ++u)
+                    if (eb + u < e1)
+#pragma unroll
+                        for (int q = 0; q < BB; ++q)
+                            if (b + q < b1) {
+                                sr[q] += av[u].x * x[q][u].x - av[u].y * x[q][u].y;
+                                si[q] += av[u].x * x[q][u].y + av[u].y * x[q][u].x;
+                            }
+            }
+#pragma unroll
+            for (int q = 0; q < BB; ++q)
+                if (b + q < b1) st_stream(out + (b + q) * obs + row * k + j, make_double2(sr[q], si[q]), NT);
         }
-        ob[(int64_t)row * k + j] = make_double2(sr, si);
-    }
 }
 }  // namespace rsvdt
 
@@ -1208,12 +1254,29 @@ extern "C" int rsvdt_hip_spmm_blocks(int64_t nrows, int64_t k, int64_t nb, const
 {
     if (nrows <= 0 || k <= 0 || nb <= 0) return RSVDT_HIP_OK;
     if (nb > 65535 || nrows > 0x7fffffffLL) { set_error_msg("rsvdt_hip_spmm_blocks: bad size"); return RSVDT_HIP_ERR_ARG; }
-    int lpr = 1;
-    while (lpr < k && lpr < 64) lpr <<= 1;
-    const int rpb = 256 / lpr;
-    hipLaunchKernelGGL(k_spmm_blocks, dim3(ceil_div(nrows, rpb), (unsigned)nb), dim3(256), 0, as_stream(s), (int)nrows,
-                       (int)k, lpr, rowptr, col, (const double2 *)val_complex, (const double2 *)in, in_bstride,
-                       (double2 *)out, out_bstride);
+    const int kl = k < 256 ? (int)k : 256, rpb = 256 / kl;
+    const int64_t gx = ceil_div(nrows, rpb);
+    // blocks a workgroup forms: as many as leave four workgroups a CU (a group
+    // of four in flight hides more latency than more workgroups do: 28 blocks
+    // of 2549 x 23 take 26.9 us one block at a time, 18.2 us in fours), at most 8
+    int64_t bpw = gx * nb / 1024;
+    bpw = bpw < 1 ? 1 : (bpw >= 8 ? 8 : (bpw > 4 ? 4 : bpw));
+    if (bpw > nb) bpw = nb;
+    const dim3 grid((unsigned)gx, ceil_div(nb, bpw));
+    const double bytes = 16.0 * (double)nrows * (double)k * (double)nb;
+#define RSVDT_SPB(NT, BB)                                                                                          \
+    hipLaunchKernelGGL((k_spmm_blocks<NT, BB>), grid, dim3(256), 0, as_stream(s), (int)nrows, (int)k, kl, rpb,       \
+                       (int)nb, (int)bpw, rowptr, col, (const double2 *)val_complex, (const double2 *)in,           \
+                       in_bstride, (double2 *)out, out_bstride)
+#define RSVDT_SPN(BB)                                                                                              \
+    if (nt) RSVDT_SPB(true, BB);                                                                                   \
+    else RSVDT_SPB(false, BB)
+    const bool nt = bytes > 256e6;              // beyond the last-level cache: no point in keeping it there
+    if (bpw == 1) { RSVDT_SPN(1); }
+    else if (bpw == 2) { RSVDT_SPN(2); }
+    else { RSVDT_SPN(4); }
+#undef RSVDT_SPN
+#undef RSVDT_SPB
     RSVDT_LAUNCH_CHECK("rsvdt_hip_spmm_blocks");
     return RSVDT_HIP_OK;
 }

@@ -290,3 +290,24 @@ def test_coef_gemm_stream(L, pkg, P, K, ncol, prec, beta):
     ref = 0.7 * (C[:, (2 - np.arange(P)) % cmod].T @ X) + beta * Y
     tol = (4 * K * EPS if prec == 64 else 2.4e-7) * max(1.0, np.max(np.abs(ref)))
     assert np.max(np.abs(dY.get(cdt, (P, ncol)) - ref)) <= tol
+
+
+@pytest.mark.parametrize("rows,cols,k,nb", [(1, 1, 1, 1), (37, 90, 7, 3), (500, 500, 64, 4), (513, 200, 100, 5),
+                                            (33, 40, 256, 2), (20, 31, 257, 6), (70000, 70000, 3, 9)])
+@pytest.mark.parametrize("wmax", [0, 1, 2, 7])
+def test_spmm_blocks_shapes(L, pkg, rows, cols, k, nb, wmax):
+    """Out_b = M In_b with 0 .. wmax entries a row (empty rows among them), for
+    rows that do not fill a workgroup and blocks that do not fill a group."""
+    rng = np.random.default_rng(rows + wmax)
+    cnt = rng.integers(0, min(wmax, cols) + 1, rows)
+    rp = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32)
+    ci = np.concatenate([np.sort((rng.integers(cols) + np.arange(c)) % cols) for c in cnt] + [[0]]).astype(np.int32)
+    v, x = crandn(rng, len(ci)), crandn(rng, nb, cols, k)
+    M = sp.csr_matrix((v[:-1], ci[:-1], rp), shape=(rows, cols))
+    held = [Dev(pkg, a) for a in (rp, ci, v, x)]
+    out = Dev(pkg, np.full((nb, rows, k), np.nan + 0j))
+    L.rsvdt_hip_spmm_blocks.argtypes = [I64] * 3 + [V, V, V, V, I64, V, I64, V]
+    assert L.rsvdt_hip_spmm_blocks(rows, k, nb, *[h.p for h in held], cols * k, out.p, rows * k, None) == 0
+    got = out.get(np.complex128, (nb, rows, k))
+    ref = np.stack([M @ x[b] for b in range(nb)])
+    assert np.max(np.abs(got - ref)) <= 30 * EPS * max(wmax, 1) * 4
