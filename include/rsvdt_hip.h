@@ -319,6 +319,12 @@ int rsvdt_hip_zcopy3(int64_t nb, int64_t nr, int64_t nc,
  * c*rows + r (uniform [0,1) + i[0,1) when gauss = 0, complex N(0,1) when 1). */
 int rsvdt_hip_fill_random(int64_t rows, int64_t kb, int64_t nblk, uint64_t seed, int gauss, double *out,
                           rsvdt_stream_t s);
+/* Columns c0 .. c0+nc-1 of a dense matrix between column-major (cm: these
+ * columns alone, rows x nc) and the blocked layout (nblk row-major blocks of
+ * kb columns; column c is in block c / kb for order 0, c % nblk for order 1).
+ * to_cm 0: cm -> blk; 1: blk -> cm.  nc <= 32 x 65535. */
+int rsvdt_hip_cm_relayout(int64_t rows, int64_t kb, int64_t nblk, int order, int64_t c0, int64_t nc, double *cm,
+                          double *blk, int to_cm, rsvdt_stream_t s);
 /* Per-row transpose between the block layout [s][r][b] (n blocks, block s
  * an nrows x kt row-major slab) and the per-batch row-major layout [j][r][s]
  * (kb batches, batch j an nrows x n row-major matrix), for the batches

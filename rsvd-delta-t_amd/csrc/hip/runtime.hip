@@ -100,6 +100,7 @@ extern "C" int rsvdt_hip_malloc(void **p, size_t bytes) {
         e = hipMalloc(p, r);
     }
     if (e != hipSuccess) {
+        (void)hipGetLastError();                // reported here; callers may go on without the block
         *p = nullptr;
         set_error("hipMalloc", e);
         return RSVDT_HIP_ERR_RUNTIME;
@@ -588,6 +589,53 @@ extern "C" int rsvdt_hip_znorm2(int64_t n, const double *x, double *out, void *w
     hipLaunchKernelGGL(k_znorm2_part, dim3(nblk), dim3(256), 0, as_stream(s), n, (const double2 *)x, (double *)work);
     hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(256), 0, as_stream(s), nblk, (const double *)work, out);
     RSVDT_LAUNCH_CHECK("rsvdt_hip_znorm2");
+    return RSVDT_HIP_OK;
+}
+
+// Columns c0 .. c0+nc-1 of a dense host matrix (column-major, `cm` a device
+// copy of just these columns) to or from the blocked layout: kb-column
+// row-major blocks, column c in block c / kb (order 0) or c % nblk (order 1).
+// A workgroup turns a 32 x 32 tile in LDS, whole cache lines on both sides.
+// On the host the same relayout, with its temporary's page faults, was most of
+// what a small action spent outside the GPU.
+template <bool TO_CM>
+__global__ __launch_bounds__(256) void k_cm_relayout(int64_t rows, int64_t kb, int64_t nblk, int order, int64_t c0,
+                                                     int64_t nc, double2 *cm, double2 *blk) {
+    __shared__ double2 tile[32][33];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const int64_t r0 = (int64_t)blockIdx.x * 32, t0 = (int64_t)blockIdx.y * 32;
+    const int64_t c = c0 + t0 + tx, b = order ? c % nblk : c / kb, j = order ? c / nblk : c - b * kb;
+    const bool cok = t0 + tx < nc;
+    double2 *bp = blk + b * rows * kb + j;
+#pragma unroll
+    for (int i = ty; i < 32; i += 8) {
+        if (TO_CM) {
+            if (cok && r0 + i < rows) tile[tx][i] = bp[(r0 + i) * kb];
+        } else if (t0 + i < nc && r0 + tx < rows) tile[i][tx] = cm[(t0 + i) * rows + r0 + tx];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = ty; i < 32; i += 8) {
+        if (TO_CM) {
+            if (t0 + i < nc && r0 + tx < rows) cm[(t0 + i) * rows + r0 + tx] = tile[i][tx];
+        } else if (cok && r0 + i < rows) bp[(r0 + i) * kb] = tile[tx][i];
+    }
+}
+extern "C" int rsvdt_hip_cm_relayout(int64_t rows, int64_t kb, int64_t nblk, int order, int64_t c0, int64_t nc,
+                                     double *cm, double *blk, int to_cm, rsvdt_stream_t s) {
+    if (rows <= 0 || nc <= 0) return RSVDT_HIP_OK;
+    if (kb <= 0 || nblk <= 0 || c0 < 0 || c0 + nc > kb * nblk || nc > 65535LL * 32 || rows > 0x7fffffffLL * 32) {
+        set_error_msg("rsvdt_hip_cm_relayout: columns outside the matrix, or more than 32 x 65535 of them");
+        return RSVDT_HIP_ERR_ARG;
+    }
+    const dim3 grid(ceil_div(rows, 32), ceil_div(nc, 32));
+    if (to_cm)
+        hipLaunchKernelGGL(k_cm_relayout<true>, grid, dim3(256), 0, as_stream(s), rows, kb, nblk, order, c0, nc,
+                           (double2 *)cm, (double2 *)blk);
+    else
+        hipLaunchKernelGGL(k_cm_relayout<false>, grid, dim3(256), 0, as_stream(s), rows, kb, nblk, order, c0, nc,
+                           (double2 *)cm, (double2 *)blk);
+    RSVDT_LAUNCH_CHECK("rsvdt_hip_cm_relayout");
     return RSVDT_HIP_OK;
 }
 

@@ -404,17 +404,56 @@ static void blocked_to_host(const Mat m, const double *blk, double *cm)
     }
 }
 
+/* The host matrix goes to the device (or comes back) as it is, 64 MB of columns
+ * at a time, and is turned into (from) blocks there: 5 MB in and out take 195 +
+ * 372 us, 325 + 719 us with the relayout and its temporary on the host.  Below
+ * 256 KB the extra launch and wait cost more (16 KB: 54 + 46 us, 45 + 30 us on
+ * the host), so there, and without room on the device, the host does it.
+ * Returns an error code of the HIP layer. */
+static int dense_transfer(Mat m, double *host, int to_host)
+{
+    const PetscInt nb = m->cols / m->kb;
+    if (m->rows <= 0 || m->cols <= 0) return 0;
+    PetscInt step = ((int64_t)64 << 20) / 16 / m->rows;
+    if (step < 1) step = 1;
+    if (step > 32 * 65535) step = 32 * 65535;
+    if (step > m->cols) step = m->cols;
+    double *cm = NULL;
+    int rc = 0;
+    const size_t all = (size_t)m->rows * (size_t)m->cols * 16;
+    if (all < 262144 || rsvdt_hip_malloc((void **)&cm, (size_t)step * (size_t)m->rows * 16)) {
+        double *tmp = malloc(all);
+        if (!tmp) return RSVDT_ERR_MEM;
+        if (to_host) {
+            rc = rsvdt_hip_memcpy_d2h(tmp, m->d, all);
+            if (!rc) blocked_to_host(m, tmp, host);
+        } else {
+            host_to_blocked(m, host, tmp);
+            rc = rsvdt_hip_memcpy_h2d(m->d, tmp, all);
+        }
+        free(tmp);
+        return rc;
+    }
+    /* the copies wait for the device on both sides, so cm can be refilled */
+    for (PetscInt c0 = 0; c0 < m->cols && !rc; c0 += step) {
+        const PetscInt nc = m->cols - c0 < step ? m->cols - c0 : step;
+        double *h = host + 2 * (size_t)c0 * (size_t)m->rows;
+        const size_t bytes = (size_t)nc * (size_t)m->rows * 16;
+        if (!to_host) rc = rsvdt_hip_memcpy_h2d(cm, h, bytes);
+        if (!rc) rc = rsvdt_hip_cm_relayout(m->rows, m->kb, nb, m->order, c0, nc, cm, m->d, to_host, g_rsvdt.stream);
+        if (!rc && to_host) rc = rsvdt_hip_memcpy_d2h(h, cm, bytes);
+    }
+    rsvdt_hip_free(cm);
+    return rc;
+}
+
 PetscErrorCode RSVDT_MatCreateDenseBlocked(PetscInt rows, PetscInt cols, PetscInt kb, const double *host, Mat *out)
 {
     Mat m;
     RSVDT_CHK(rsvdt_mat_alloc_dense(rows, cols, kb, 0, &m));
     if (host) {
-        size_t n = (size_t)rows * (size_t)cols * 2;
-        double *tmp = malloc(n * sizeof(double));
-        if (!tmp) return rsvdt_err(RSVDT_ERR_MEM, "MatCreateDense", "out of memory");
-        host_to_blocked(m, host, tmp);
-        int rc = rsvdt_hip_memcpy_h2d(m->d, tmp, n * sizeof(double));
-        free(tmp);
+        int rc = dense_transfer(m, (double *)host, 0);
+        if (rc == RSVDT_ERR_MEM) return rsvdt_err(RSVDT_ERR_MEM, "MatCreateDense", "out of memory");
         if (rc) return rsvdt_err(rc, "MatCreateDense", "%s", rsvdt_hip_last_error());
     }
     *out = m;
@@ -429,14 +468,10 @@ PetscErrorCode RSVDT_MatCreateDense(PetscInt rows, PetscInt cols, const double *
 PetscErrorCode RSVDT_MatGetDense(Mat m, double *host)
 {
     if (!m || m->kind != RSVDT_MAT_DENSE) return rsvdt_err(RSVDT_ERR_USER, "MatGetDense", "not a dense Mat");
-    size_t n = (size_t)m->rows * (size_t)m->cols * 2;
-    double *tmp = malloc(n * sizeof(double) + 16);
-    if (!tmp) return rsvdt_err(RSVDT_ERR_MEM, "MatGetDense", "out of memory");
     int rc = rsvdt_hip_sync();
-    if (!rc) rc = rsvdt_hip_memcpy_d2h(tmp, m->d, n * sizeof(double));
-    if (rc) { free(tmp); return rsvdt_err(rc, "MatGetDense", "%s", rsvdt_hip_last_error()); }
-    blocked_to_host(m, tmp, host);
-    free(tmp);
+    if (!rc) rc = dense_transfer(m, host, 1);
+    if (rc == RSVDT_ERR_MEM) return rsvdt_err(RSVDT_ERR_MEM, "MatGetDense", "out of memory");
+    if (rc) return rsvdt_err(rc, "MatGetDense", "%s", rsvdt_hip_last_error());
     return 0;
 }
 

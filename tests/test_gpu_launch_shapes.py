@@ -311,3 +311,28 @@ def test_spmm_blocks_shapes(L, pkg, rows, cols, k, nb, wmax):
     got = out.get(np.complex128, (nb, rows, k))
     ref = np.stack([M @ x[b] for b in range(nb)])
     assert np.max(np.abs(got - ref)) <= 30 * EPS * max(wmax, 1) * 4
+
+
+@pytest.mark.parametrize("rows,cols,kb", [(1, 1, 1), (5, 6, 3), (31, 40, 10), (32, 64, 32), (33, 66, 33), (500, 640, 10),
+                                          (70001, 66, 2), (4200003, 3, 3)])
+def test_dense_round_trip(L, pkg, rows, cols, kb):
+    """A host matrix to blocks on the device and back: the blocks' layout and
+    every entry, for ragged tiles and more columns than one transfer takes."""
+    rng = np.random.default_rng(rows)
+    F = np.asfortranarray(rng.standard_normal((rows, cols)) + 1j * rng.standard_normal((rows, cols)))
+    m = pkg.mat_from_dense(F, kb)
+    assert np.array_equal(pkg.mat_to_dense(m), F)
+    pkg.destroy(m)
+    if rows * cols > 10 ** 6:
+        return
+    nblk = cols // kb
+    dc, db = Dev(pkg, np.ascontiguousarray(F.T)), Dev(pkg, nbytes=F.nbytes)
+    L.rsvdt_hip_cm_relayout.argtypes = [I64] * 3 + [ctypes.c_int, I64, I64, V, V, ctypes.c_int, V]
+    for order in (0, 1):
+        assert L.rsvdt_hip_cm_relayout(rows, kb, nblk, order, 0, cols, dc.p, db.p, 0, None) == 0
+        c = np.arange(cols).reshape((nblk, kb) if order == 0 else (kb, nblk))
+        ref = F[:, c if order == 0 else c.T].transpose(1, 0, 2)
+        assert np.array_equal(db.get(np.complex128, (nblk, rows, kb)), ref)
+        back = Dev(pkg, nbytes=F.nbytes)
+        assert L.rsvdt_hip_cm_relayout(rows, kb, nblk, order, 0, cols, back.p, db.p, 1, None) == 0
+        assert np.array_equal(back.get(np.complex128, (cols, rows)), F.T)
