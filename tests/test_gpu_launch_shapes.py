@@ -336,3 +336,15 @@ def test_dense_round_trip(L, pkg, rows, cols, kb):
         back = Dev(pkg, nbytes=F.nbytes)
         assert L.rsvdt_hip_cm_relayout(rows, kb, nblk, order, 0, cols, back.p, db.p, 1, None) == 0
         assert np.array_equal(back.get(np.complex128, (cols, rows)), F.T)
+
+
+@pytest.mark.parametrize("M,N,K", [(64 * 7, 190, 40), (64 * 8, 190, 40), (64 * 17 - 3, 70, 20), (130, 70, 64 * 72)])
+def test_gemm_bf16_tile_order(L, pkg, M, N, K):
+    """Fewer than eight, eight, and eight and a rest of the groups of tiles (or
+    of splits) that go to one XCD: every tile of C once."""
+    rng = np.random.default_rng(M)
+    A, B = (rng.integers(-4, 5, s).astype(np.float32) for s in ((M, K), (K, N)))
+    dA, dB, dC = Dev(pkg, A), Dev(pkg, B), Dev(pkg, np.full((M, N), np.nan, np.float32))
+    L.rsvdt_hip_gemm_bf16.argtypes = [I64] * 3 + [V, I64, I64, V, I64, I64, V, I64, ctypes.c_int, V, V, I64, V]
+    assert L.rsvdt_hip_gemm_bf16(M, N, K, dA.p, K, 1, dB.p, N, 1, dC.p, N, 0, None, None, 0, None) == 0
+    assert np.array_equal(dC.get(np.float32, (M, N)), A @ B)     # whole numbers: exact
