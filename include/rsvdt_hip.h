@@ -319,6 +319,12 @@ int rsvdt_hip_zcopy3(int64_t nb, int64_t nr, int64_t nc,
  * c*rows + r (uniform [0,1) + i[0,1) when gauss = 0, complex N(0,1) when 1). */
 int rsvdt_hip_fill_random(int64_t rows, int64_t kb, int64_t nblk, uint64_t seed, int gauss, double *out,
                           rsvdt_stream_t s);
+/* Window coefficients and shifts of the Galerkin projection: C holds C1, then
+ * Ct, kb x (Nw+1) x Nwe each, ph k x Nwe (every test vector the same), from the
+ * Nw x Nwe dft table: d(j, m) = RR dft(j, m), zero for j outside 0 .. Nw-1;
+ * ph_m = exp(i sw m dT), C1(s, m) = d(s-w1, m), Ct = ph_m C1 - d(s-w2, m). */
+int rsvdt_hip_tr_windows(int64_t kb, int64_t k, int64_t Nw, int64_t Nwe, const double *dft, double RR, double sw,
+                         double dT, int w1, int w2, double *C, double *ph, rsvdt_stream_t s);
 /* Columns c0 .. c0+nc-1 of a dense matrix between column-major (cm: these
  * columns alone, rows x nc) and the blocked layout (nblk row-major blocks of
  * kb columns; column c is in block c / kb for order 0, c % nblk for order 1).

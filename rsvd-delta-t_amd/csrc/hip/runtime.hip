@@ -592,6 +592,44 @@ extern "C" int rsvdt_hip_znorm2(int64_t n, const double *x, double *out, void *w
     return RSVDT_HIP_OK;
 }
 
+// Window coefficients of the Galerkin projection for kb test vectors (C1, then
+// Ct, kb x (Nw+1) x Nwe each) and the shifts ph (k x Nwe) of GalerkinProj.c:30-50:
+// with d(j, m) = RR dft(j, m), zero outside 0 <= j < Nw, and ph_m = exp(i sw m dT),
+// C1(s, m) = d(s - w1, m), Ct(s, m) = ph_m d(s - w1, m) - d(s - w2, m).  Made where
+// it is used: on the host the table, its copies and the wait for the stepping
+// left the GPU idle for 0.4 ms of the Ginzburg-Landau action.
+__global__ __launch_bounds__(256) void k_tr_windows(int kb, int k, int Nw, int Nwe, const double2 *__restrict__ dft,
+                                                    double RR, double sw, double dT, int w1, int w2, double2 *C,
+                                                    double2 *ph) {
+    const int64_t ne = (int64_t)(Nw + 1) * Nwe, e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= ne) return;
+    const int s = (int)(e / Nwe), m = (int)(e - (int64_t)s * Nwe), j1 = s - w1, j2 = s - w2;
+    double pi, pr;
+    sincos(sw * (double)m * dT, &pi, &pr);
+    double2 d1 = make_double2(0, 0), d2 = d1;
+    if (j1 >= 0 && j1 < Nw) { d1 = dft[(int64_t)j1 * Nwe + m]; d1.x *= RR; d1.y *= RR; }
+    if (j2 >= 0 && j2 < Nw) { d2 = dft[(int64_t)j2 * Nwe + m]; d2.x *= RR; d2.y *= RR; }
+    const double2 ct = make_double2(pr * d1.x - pi * d1.y - d2.x, pr * d1.y + pi * d1.x - d2.y);
+    for (int b = 0; b < kb; ++b) {
+        C[b * ne + e] = d1;
+        C[(kb + b) * ne + e] = ct;
+    }
+    if (s == 0)
+        for (int i = 0; i < k; ++i) ph[(int64_t)i * Nwe + m] = make_double2(pr, pi);
+}
+extern "C" int rsvdt_hip_tr_windows(int64_t kb, int64_t k, int64_t Nw, int64_t Nwe, const double *dft, double RR,
+                                    double sw, double dT, int w1, int w2, double *C, double *ph, rsvdt_stream_t s) {
+    if (kb <= 0 || k <= 0 || Nw <= 0 || Nwe <= 0) return RSVDT_HIP_OK;
+    if (kb > 0x7fffffff || k > 0x7fffffff || Nw >= 0x7fffffff || Nwe > 0x7fffffff) {
+        set_error_msg("rsvdt_hip_tr_windows: sizes below 2^31 required");
+        return RSVDT_HIP_ERR_ARG;
+    }
+    hipLaunchKernelGGL(k_tr_windows, dim3(ceil_div((Nw + 1) * Nwe, 256)), dim3(256), 0, as_stream(s), (int)kb, (int)k,
+                       (int)Nw, (int)Nwe, (const double2 *)dft, RR, sw, dT, w1, w2, (double2 *)C, (double2 *)ph);
+    RSVDT_LAUNCH_CHECK("rsvdt_hip_tr_windows");
+    return RSVDT_HIP_OK;
+}
+
 // Columns c0 .. c0+nc-1 of a dense host matrix (column-major, `cm` a device
 // copy of just these columns) to or from the blocked layout: kb-column
 // row-major blocks, column c in block c / kb (order 0) or c % nblk (order 1).

@@ -1371,43 +1371,18 @@ static PetscErrorCode gal_begin(gal_ctx *c, Mat Yall, RSVDt_vars *V, DFT_matrice
     int dir = V->TS.DirAdj ? 1 : 0;
     double dT = V->TS.dt * (double)V->TS.ResRatio;
     double RR = (double)V->TS.ResRatio;
-    /* host: dft (Nw x Nwe), the window coefficients for every test vector of a
-     * group (C1 then Ct, kb x Ns1 x Nwe each) and the shifts ph (k x Nwe) */
-    double *dft = malloc(sizeof(double) * 2 * (size_t)(Nw * Nwe));
-    double *C = calloc((size_t)(2 * kb * Ns1 * Nwe) * 2, sizeof(double));
-    double *ph = malloc(sizeof(double) * 2 * (size_t)(k * Nwe));
-    if (!dft || !C || !ph) { free(dft); free(C); free(ph); return rsvdt_err(RSVDT_ERR_MEM, "GalerkinProjAllModes", "out of memory"); }
-    int h = rsvdt_hip_memcpy_d2h(dft, D->dft->d, sizeof(double) * 2 * (size_t)(Nw * Nwe));
-    if (h) { free(dft); free(C); free(ph); return rsvdt_err(h, "GalerkinProjAllModes", "device call failed: %s", rsvdt_hip_last_error()); }
-    const PetscInt w1 = dir ? 0 : 1, w2 = dir ? 1 : 0;
-    for (PetscInt m = 0; m < Nwe; m++) {
-        double ang = (dir ? 1.0 : -1.0) * V->RSVD.w * (double)m * dT;   /* GalerkinProj.c:49-50 */
-        double pr = cos(ang), pi = sin(ang);
-        for (PetscInt ik = 0; ik < k; ik++) { ph[2 * (ik * Nwe + m)] = pr; ph[2 * (ik * Nwe + m) + 1] = pi; }
-        for (PetscInt s = 0; s < Ns1; s++) {
-            double d1r = 0, d1i = 0, d2r = 0, d2i = 0;
-            PetscInt j1 = s - w1, j2 = s - w2;
-            if (j1 >= 0 && j1 < Nw) { d1r = RR * dft[2 * (j1 * Nwe + m)]; d1i = RR * dft[2 * (j1 * Nwe + m) + 1]; }
-            if (j2 >= 0 && j2 < Nw) { d2r = RR * dft[2 * (j2 * Nwe + m)]; d2i = RR * dft[2 * (j2 * Nwe + m) + 1]; }
-            for (PetscInt b = 0; b < kb; b++) {
-                double *c1 = C + 2 * (size_t)((b * Ns1 + s) * Nwe + m);
-                double *ct = C + 2 * (size_t)(((kb + b) * Ns1 + s) * Nwe + m);
-                c1[0] = d1r; c1[1] = d1i;
-                ct[0] = pr * d1r - pi * d1i - d2r;
-                ct[1] = pr * d1i + pi * d1r - d2i;
-            }
-        }
-    }
-    free(dft);
+    /* the window coefficients for every test vector of a group (C1 then Ct,
+     * kb x Ns1 x Nwe each) and the shifts ph (k x Nwe; GalerkinProj.c:49-50) */
+    const int w1 = dir ? 0 : 1, w2 = dir ? 1 : 0;
     const size_t csz = sizeof(double) * 2 * (size_t)(2 * kb * Ns1 * Nwe);
     const size_t ybytes = (size_t)kb * (size_t)N * (size_t)Nwe * 16;
     PetscErrorCode ierr = 0;
     if (rsvdt_hip_malloc((void **)&c->dC, csz) || rsvdt_hip_malloc((void **)&c->dph, sizeof(double) * 2 * (size_t)(k * Nwe)) ||
         rsvdt_hip_malloc((void **)&c->Ybrm, ybytes))
         ierr = rsvdt_err(RSVDT_ERR_MEM, "GalerkinProjAllModes", "cannot allocate work");
-    if (!ierr && (rsvdt_hip_memcpy_h2d(c->dC, C, csz) || rsvdt_hip_memcpy_h2d(c->dph, ph, sizeof(double) * 2 * (size_t)(k * Nwe))))
+    if (!ierr && rsvdt_hip_tr_windows(kb, k, Nw, Nwe, D->dft->d, RR, (dir ? 1.0 : -1.0) * V->RSVD.w, dT, w1, w2, c->dC,
+                                      c->dph, g_rsvdt.stream))
         ierr = rsvdt_err(RSVDT_HIP_ERR_RUNTIME, "GalerkinProjAllModes", "device call failed: %s", rsvdt_hip_last_error());
-    free(C); free(ph);
     if (!ierr) ierr = rsvdt_mat_alloc_dense(N, Nwe * k, k, 1, &c->Yup);
     size_t nb_b = (size_t)kb * (size_t)Ns1 * (size_t)Nwe * 16, nb_w = (size_t)kb * (size_t)Ns1 * (size_t)Ns1 * 16;
     c->B = rsvdt_scratch(SCR_MISC, nb_b);

@@ -348,3 +348,23 @@ def test_gemm_bf16_tile_order(L, pkg, M, N, K):
     L.rsvdt_hip_gemm_bf16.argtypes = [I64] * 3 + [V, I64, I64, V, I64, I64, V, I64, ctypes.c_int, V, V, I64, V]
     assert L.rsvdt_hip_gemm_bf16(M, N, K, dA.p, K, 1, dB.p, N, 1, dC.p, N, 0, None, None, 0, None) == 0
     assert np.array_equal(dC.get(np.float32, (M, N)), A @ B)     # whole numbers: exact
+
+
+@pytest.mark.parametrize("kb,k,Nw,Nwe", [(1, 1, 1, 1), (2, 5, 8, 4), (3, 3, 15, 15), (4, 7, 64, 32), (1, 2, 300, 300)])
+@pytest.mark.parametrize("direct", [True, False])
+def test_removal_windows(L, pkg, kb, k, Nw, Nwe, direct):
+    """The Galerkin projection's window coefficients and shifts against numpy."""
+    rng = np.random.default_rng(Nw)
+    dft, RR, sw, dT = crandn(rng, Nw, Nwe), 16.0, 0.05 if direct else -0.05, 1.9
+    dd, dC, dp = Dev(pkg, dft), Dev(pkg, nbytes=2 * kb * (Nw + 1) * Nwe * 16), Dev(pkg, nbytes=k * Nwe * 16)
+    D = ctypes.c_double
+    L.rsvdt_hip_tr_windows.argtypes = [I64] * 4 + [V, D, D, D, ctypes.c_int, ctypes.c_int, V, V, V]
+    w1, w2 = (0, 1) if direct else (1, 0)
+    assert L.rsvdt_hip_tr_windows(kb, k, Nw, Nwe, dd.p, RR, sw, dT, w1, w2, dC.p, dp.p, None) == 0
+    C, ph = dC.get(np.complex128, (2, kb, Nw + 1, Nwe)), dp.get(np.complex128, (k, Nwe))
+    ref = np.exp(1j * (sw * np.arange(Nwe) * dT))
+    d = np.zeros((2, Nw + 1, Nwe), complex)
+    d[0, w1:w1 + Nw], d[1, w2:w2 + Nw] = RR * dft, RR * dft
+    assert np.max(np.abs(ph - ref)) <= 2 * EPS
+    assert np.array_equal(C[0], np.broadcast_to(d[0], C[0].shape))
+    assert np.max(np.abs(C[1] - (ref * d[0] - d[1]))) <= 6 * EPS * np.max(np.abs(d))
