@@ -12,6 +12,7 @@
 //   * bapply: batched row-local small products Out = alpha*Y + X*C (the
 //     triangular applies of CholeskyQR, Q*U of the SVD, y1 - V*a).
 #include "common.h"
+#include <type_traits>
 
 namespace rsvdt {
 
@@ -864,22 +865,27 @@ __global__ __launch_bounds__(256) void k_bapply_gram(int64_t nrows, int n, const
 
 // Dense propagator times N x k blocks: Out_b = E X_b (+ F_b), E an N x N
 // row-major matrix, the blocks' columns taken together as nb*k columns.  A
-// workgroup owns 16 rows and 16 CT columns; its 8 waves take every eighth
+// workgroup owns ROWS rows and 16 CT columns; its 8 waves take every eighth
 // 4-column step of E (the product is a few MFLOP and follows the previous one
 // on the stream, so the reduction is split for latency, not for work) and
 // their sums meet in LDS in wave order.  PF steps of both operands are in
-// flight per wave.  N = 500, k = 10: 8.1 us; 650 columns (CT = 2): 35 us.
-template <int CT>
+// flight per wave.  With one column tile the FP64 MFMAs of 16 rows would take 3.4
+// us on the few CUs that have work: ROWS = 4 spreads them over four times as many
+// with the 4x4x4 MFMA, its four blocks the tile's four groups of columns (lane i
+// holds A[i%4][i/16], B[i/16][i%16], D[i/16][i%16]; checked with known products).
+// N = 500, k = 10: 6.6 us (7.8 with 16 rows); 650 columns (CT = 2): 35 us.
+template <int CT, int ROWS>
 __global__ __launch_bounds__(512) void k_dense_apply(int N, int k, int ncol, const double2 *__restrict__ E,
                                                      const double2 *__restrict__ X, const double2 *__restrict__ F,
                                                      double2 *__restrict__ Out)
 {
+    using acc = typename std::conditional<ROWS == 16, dvec4, double>::type;
     constexpr int PF = CT == 1 ? 8 : 4, CW = 16 * CT;
-    __shared__ double2 red[8][16][CW];
+    __shared__ double2 red[8][ROWS][CW];
     const int lane = threadIdx.x & 63, wv = wave_id(), kr = lane >> 4, cl = lane & 15;
-    const int r0 = blockIdx.x * 16, c0 = blockIdx.y * CW;
+    const int r0 = blockIdx.x * ROWS, c0 = blockIdx.y * CW;
     const int64_t bs = (int64_t)N * k;
-    const double2 *er = E + (int64_t)min(r0 + cl, N - 1) * N;
+    const double2 *er = E + (int64_t)min(r0 + cl % ROWS, N - 1) * N;
     const double2 *xc[CT];
 #pragma unroll
     for (int u = 0; u < CT; ++u) {
@@ -893,9 +899,13 @@ __global__ __launch_bounds__(512) void k_dense_apply(int N, int k, int ncol, con
 #pragma unroll
         for (int u = 0; u < CT; ++u) xv[p][u] = xc[u][(int64_t)a * k];
     };
-    dvec4 dr[CT], di[CT];
+    auto mfma = [](double x, double y, acc c) -> acc {
+        if constexpr (ROWS == 16) return __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, c, 0, 0, 0);
+        else return __builtin_amdgcn_mfma_f64_4x4x4f64(x, y, c, 0, 0, 0);
+    };
+    acc dr[CT], di[CT];
 #pragma unroll
-    for (int u = 0; u < CT; ++u) { dr[u] = (dvec4){0, 0, 0, 0}; di[u] = (dvec4){0, 0, 0, 0}; }
+    for (int u = 0; u < CT; ++u) { dr[u] = acc{}; di[u] = acc{}; }
 #pragma unroll
     for (int p = 0; p < PF; ++p) load(p, 4 * wv + 32 * p);
     for (int q0 = 4 * wv; q0 < N; q0 += 32 * PF) {
@@ -910,22 +920,25 @@ __global__ __launch_bounds__(512) void k_dense_apply(int N, int k, int ncol, con
             load(p, q + 32 * PF);
 #pragma unroll
             for (int u = 0; u < CT; ++u) {
-                dr[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(e.x, x[u].x, dr[u], 0, 0, 0);
-                di[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(e.x, x[u].y, di[u], 0, 0, 0);
+                dr[u] = mfma(e.x, x[u].x, dr[u]);
+                di[u] = mfma(e.x, x[u].y, di[u]);
             }
 #pragma unroll
             for (int u = 0; u < CT; ++u) {
-                dr[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(-e.y, x[u].y, dr[u], 0, 0, 0);
-                di[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(e.y, x[u].x, di[u], 0, 0, 0);
+                dr[u] = mfma(-e.y, x[u].y, dr[u]);
+                di[u] = mfma(e.y, x[u].x, di[u]);
             }
         }
     }
 #pragma unroll
-    for (int u = 0; u < CT; ++u)
+    for (int u = 0; u < CT; ++u) {
+        if constexpr (ROWS == 16) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) red[wv][4 * j + kr][16 * u + cl] = make_double2(dr[u][j], di[u][j]);
+            for (int j = 0; j < 4; ++j) red[wv][4 * j + kr][16 * u + cl] = make_double2(dr[u][j], di[u][j]);
+        } else red[wv][kr][16 * u + cl] = make_double2(dr[u], di[u]);
+    }
     __syncthreads();
-    for (int e = threadIdx.x; e < 16 * CW; e += 512) {
+    for (int e = threadIdx.x; e < ROWS * CW; e += 512) {
         const int r = r0 + e / CW, c = c0 + e % CW;
         if (r >= N || c >= ncol) continue;
         double2 s = red[0][e / CW][e % CW];
@@ -1163,11 +1176,18 @@ extern "C" int rsvdt_hip_dense_apply(int64_t N, int64_t k, int64_t nb, const dou
         return RSVDT_HIP_ERR_ARG;
     }
     const int ncol = (int)(k * nb);
-    if (ncol <= 256)
-        hipLaunchKernelGGL(k_dense_apply<1>, dim3(ceil_div(N, 16), ceil_div(ncol, 16)), dim3(512), 0, as_stream(s), (int)N,
+    // one column tile: 16 rows a workgroup would leave most CUs idle (us, 16 and 4
+    // rows: N = 300 7.7, 6.7; 500 7.8, 6.6; 700 10.5, 8.5; 1000 13.3, 12.6); with
+    // more column tiles the rows of X that every workgroup reads cost more (N =
+    // 500, 33 columns: 8.0, 10.4)
+    if (ncol <= 16 && N <= 1024)
+        hipLaunchKernelGGL((k_dense_apply<1, 4>), dim3(ceil_div(N, 4)), dim3(512), 0, as_stream(s), (int)N, (int)k, ncol,
+                           (const double2 *)E, (const double2 *)X, (const double2 *)F, (double2 *)Out);
+    else if (ncol <= 256)
+        hipLaunchKernelGGL((k_dense_apply<1, 16>), dim3(ceil_div(N, 16), ceil_div(ncol, 16)), dim3(512), 0, as_stream(s), (int)N,
                            (int)k, ncol, (const double2 *)E, (const double2 *)X, (const double2 *)F, (double2 *)Out);
     else
-        hipLaunchKernelGGL(k_dense_apply<2>, dim3(ceil_div(N, 16), ceil_div(ncol, 32)), dim3(512), 0, as_stream(s), (int)N,
+        hipLaunchKernelGGL((k_dense_apply<2, 16>), dim3(ceil_div(N, 16), ceil_div(ncol, 32)), dim3(512), 0, as_stream(s), (int)N,
                            (int)k, ncol, (const double2 *)E, (const double2 *)X, (const double2 *)F, (double2 *)Out);
     RSVDT_LAUNCH_CHECK("rsvdt_hip_dense_apply");
     return RSVDT_HIP_OK;
