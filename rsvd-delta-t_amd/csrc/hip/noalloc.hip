@@ -97,7 +97,7 @@ extern "C" int rsvdt_qr_blocks_noalloc(double *Y, int64_t N, int64_t k, int64_t 
     w.Ra = nullptr;
     w.Rt = nullptr;
     // shifted CholeskyQR3, as QRAllFreqs; asynchronous on s, no pivot readback
-    const PetscErrorCode ierr = rsvdt_cholqr_bufs(nblocks, N, k, Y, N * k, k, 1, nullptr, 3, 1, 0.0, nullptr,
+    const PetscErrorCode ierr = rsvdt_cholqr_bufs(nblocks, N, k, nullptr, Y, N * k, k, 1, nullptr, 3, 1, 0.0, nullptr,
                                                   (size_t)nblocks * (size_t)N * (size_t)k * 16, &w, s, 0);
     return ierr ? (ierr == RSVDT_ERR_USER ? RSVDT_HIP_ERR_ARG : ierr) : RSVDT_HIP_OK;
 }

@@ -18,7 +18,7 @@
 
 /* scratch slots */
 enum { SCR_Y = 0, SCR_U1, SCR_U2, SCR_ACC, SCR_FBUF, SCR_FBUF2, SCR_G, SCR_R, SCR_RINV, SCR_RACC, SCR_RTMP,
-       SCR_WORK, SCR_INFO, SCR_MISC, SCR_MISC2, SCR_PROJ, SCR_MASK, SCR_RMASK, SCR_CNT, SCR_FSCALE, SCR_W1, SCR_W2, SCR_QRT, SCR_GINFO, SCR_SLOTS, SCR_H, SCR_NSLOTS };
+       SCR_WORK, SCR_INFO, SCR_MISC, SCR_MISC2, SCR_PROJ, SCR_MASK, SCR_RMASK, SCR_FSCALE, SCR_W1, SCR_W2, SCR_QRT, SCR_GINFO, SCR_SLOTS, SCR_H, SCR_NSLOTS };
 _Static_assert(SCR_NSLOTS <= RSVDT_NSCRATCH, "scratch slot table too small");
 
 /* ------------------------------------------------------------------ stepper */
@@ -938,41 +938,45 @@ PetscErrorCode rsvdt_homogeneous_steps(Mat A, int dir, double h, PetscInt nsteps
  * (optional) receives the product of the passes' factors.  T (optional): a
  * buffer like X of `bytes` bytes; the applies then alternate between X and
  * T (required for more than 64 columns with unit column strides, where the
- * apply cannot work in place) and the result is copied back into X. */
-PetscErrorCode rsvdt_cholqr_bufs(PetscInt nb, PetscInt nrows, PetscInt n, double *X, int64_t xb, int64_t xr,
+ * apply cannot work in place) and the result is copied back into X if it ends
+ * in T.  X0 (optional, with T): the rows to start from, in place of X, which
+ * then only receives the result; an odd number of passes ends in X. */
+PetscErrorCode rsvdt_cholqr_bufs(PetscInt nb, PetscInt nrows, PetscInt n, const double *X0, double *X, int64_t xb, int64_t xr,
                                  int64_t xa, double *R_out, int npass, int shift_first, double drop_tol, double *T,
                                  size_t bytes, const rsvdt_cholqr_work *w, rsvdt_stream_t q, int report)
 {
-    const size_t mat = (size_t)nb * (size_t)n * (size_t)n * 16;
     RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_zero(w->info, 256, q));
     const double shift_rel = 11.0 * ((double)nrows * (double)n + (double)n * (double)(n + 1)) * 1.1102230246251565e-16;
-    double *cur = X, *oth = T ? T : X;
+    const double *cur = X0 ? X0 : X;
+    double *oth = X0 || !T ? X : T;
     /* up to 64 contiguous columns: each apply also forms the Gram matrix of its
      * result, so a pass after the first reads and writes the rows once (7
      * traversals of the blocks for three passes instead of 9) */
     const int joint = xa == 1 && n <= 64;
+    double *acc = NULL;            /* product of the passes' factors so far */
     for (int pass = 0; pass < npass; pass++) {
+        const int end = pass + 1 == npass;
+        double *R = R_out && pass == 0 ? (end ? R_out : w->Ra) : w->R;
         if (!joint || pass == 0)
             RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_bgram(nb, nrows, n, n, cur, xb, xr, xa, cur, xb, xr, xa, w->G, w->work, q));
         RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_bchol_inv(nb, n, w->G, (pass == 0 && shift_first) ? shift_rel : 0.0,
-                                                       drop_tol, w->R, w->Ri, w->info, q));
+                                                       drop_tol, R, w->Ri, w->info, q));
         if (joint)
             RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_bapply_gram(nb, nrows, n, cur, xb, xr, w->Ri, oth,
-                                                             pass + 1 < npass ? w->G : NULL, w->work, q));
+                                                             end ? NULL : w->G, w->work, q));
         else
             RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_bapply(nb, nrows, n, n, cur, xb, xr, xa, w->Ri, 0.0, NULL, 0, 0, 0, oth,
                                                         xb, xr, xa, q));
-        if (T) { double *tmp = cur; cur = oth; oth = tmp; }
-        if (R_out) {
-            if (pass == 0) RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_memcpy_d2d(w->Ra, w->R, mat, q));
-            else {
-                RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_btrmm_upper(nb, n, w->R, w->Ra, w->Rt, q));
-                RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_memcpy_d2d(w->Ra, w->Rt, mat, q));
-            }
+        cur = oth;
+        if (T) oth = cur == X ? T : X;
+        if (R_out && pass == 0) acc = R;
+        else if (R_out) {
+            double *dst = end ? R_out : (acc == w->Ra ? w->Rt : w->Ra);
+            RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_btrmm_upper(nb, n, w->R, acc, dst, q));
+            acc = dst;
         }
     }
     if (cur != X) RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_memcpy_d2d(X, cur, bytes, q));
-    if (R_out) RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_memcpy_d2d(R_out, w->Ra, mat, q));
     if (report) {
         int hinfo = 0;
         RSVDT_HIPCHK("QRAllFreqs", rsvdt_hip_memcpy_d2h(&hinfo, w->info, sizeof(int)));
@@ -981,9 +985,9 @@ PetscErrorCode rsvdt_cholqr_bufs(PetscInt nb, PetscInt nrows, PetscInt n, double
     return 0;
 }
 
-static PetscErrorCode cholqr_passes(PetscInt nb, PetscInt nrows, PetscInt n, double *X, int64_t xb, int64_t xr,
-                                    int64_t xa, double *R_out, int npass, int shift_first, double drop_tol,
-                                    double *T, size_t bytes)
+static PetscErrorCode cholqr_passes(PetscInt nb, PetscInt nrows, PetscInt n, const double *X0, double *X, int64_t xb,
+                                    int64_t xr, int64_t xa, double *R_out, int npass, int shift_first,
+                                    double drop_tol, double *T, size_t bytes, int report)
 {
     size_t mat = (size_t)nb * (size_t)n * (size_t)n * 16;
     rsvdt_cholqr_work w;
@@ -996,8 +1000,8 @@ static PetscErrorCode cholqr_passes(PetscInt nb, PetscInt nrows, PetscInt n, dou
     w.info = rsvdt_scratch(SCR_INFO, 256);
     if (!w.G || !w.R || !w.Ri || (R_out && (!w.Ra || !w.Rt)) || !w.work || !w.info)
         return rsvdt_err(RSVDT_ERR_MEM, "QRAllFreqs", "cannot allocate CholeskyQR work");
-    return rsvdt_cholqr_bufs(nb, nrows, n, X, xb, xr, xa, R_out, npass, shift_first, drop_tol, T, bytes, &w,
-                             g_rsvdt.stream, 1);
+    return rsvdt_cholqr_bufs(nb, nrows, n, X0, X, xb, xr, xa, R_out, npass, shift_first, drop_tol, T, bytes, &w,
+                             g_rsvdt.stream, report);
 }
 
 PetscErrorCode rsvdt_cholqr(PetscInt nb, PetscInt nrows, PetscInt n, double *X, int64_t xb, int64_t xr, int64_t xa,
@@ -1012,7 +1016,7 @@ PetscErrorCode rsvdt_cholqr(PetscInt nb, PetscInt nrows, PetscInt n, double *X, 
         T = rsvdt_scratch(SCR_QRT, bytes);
         if (!T) return rsvdt_err(RSVDT_ERR_MEM, "QRAllFreqs", "cannot allocate CholeskyQR work");
     }
-    return cholqr_passes(nb, nrows, n, X, xb, xr, xa, R_out, 3, 1, drop_tol, T, bytes);
+    return cholqr_passes(nb, nrows, n, NULL, X, xb, xr, xa, R_out, 3, 1, drop_tol, T, bytes, 1);
 }
 
 PetscErrorCode rsvdt_span_basis(PetscInt nb, PetscInt nrows, PetscInt n, const double *X, double *Q, double *E,
@@ -1022,33 +1026,34 @@ PetscErrorCode rsvdt_span_basis(PetscInt nb, PetscInt nrows, PetscInt n, const d
     double *C = rsvdt_scratch(SCR_PROJ, mat);
     double *D = rsvdt_scratch(SCR_MASK, mat);
     double *Rm = rsvdt_scratch(SCR_RMASK, mat);
-    int *cnt = rsvdt_scratch(SCR_CNT, 256);
+    int *info = rsvdt_scratch(SCR_INFO, 256);   /* the passes' pivot count, and at 16 the dropped columns */
     void *work = rsvdt_scratch(SCR_WORK, rsvdt_hip_bgram_work_bytes(nb, nrows, n, n));
-    if (!C || !D || !Rm || !cnt || !work) return rsvdt_err(RSVDT_ERR_MEM, "CreateMtilde", "cannot allocate basis work");
+    if (!C || !D || !Rm || !info || !work) return rsvdt_err(RSVDT_ERR_MEM, "CreateMtilde", "cannot allocate basis work");
     rsvdt_stream_t q = g_rsvdt.stream;
     const int64_t nel = (int64_t)(bytes / 16);
-    /* level 1 */
-    RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_memcpy_d2d(Q, X, bytes, q));
-    RSVDT_CHK(cholqr_passes(nb, nrows, n, Q, xb, xr, xa, Rm, 3, 1, drop_tol, T, bytes));
-    RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_zero(cnt, 256, q));
-    RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_bdrop_mask(nb, n, Rm, D, cnt, q));
-    int ndrop = 0;
-    RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_memcpy_d2h(&ndrop, cnt, sizeof(int)));
+    /* level 1, from X straight into Q; one wait for both counts (the passes clear
+     * all of info before they start) */
+    RSVDT_CHK(cholqr_passes(nb, nrows, n, X, Q, xb, xr, xa, Rm, 3, 1, drop_tol, T, bytes, 0));
+    RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_bdrop_mask(nb, n, Rm, D, info + 16, q));
+    int cnt[17];
+    RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_memcpy_d2h(cnt, info, sizeof(cnt)));
+    const int ndrop = cnt[16];
+    if (cnt[0]) rsvdt_printf("[rsvdt] warning: CholeskyQR met %d non-positive pivots (rank-deficient input)\n", cnt[0]);
     if (ndrop == 0) return 0;
     /* level 2: E = ((I - Q Q^H) X) D, the residuals of the dropped columns */
     RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_bgram(nb, nrows, n, n, Q, xb, xr, xa, X, xb, xr, xa, C, work, q));
     RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_zscale((int64_t)nb * n * n, -1.0, C, C, q));
     RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_bapply(nb, nrows, n, n, Q, xb, xr, xa, C, 1.0, X, xb, xr, xa, T, xb, xr, xa, q));
     RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_bapply(nb, nrows, n, n, T, xb, xr, xa, D, 0.0, NULL, 0, 0, 0, E, xb, xr, xa, q));
-    RSVDT_CHK(cholqr_passes(nb, nrows, n, E, xb, xr, xa, NULL, 3, 1, drop_tol, T, bytes));
+    RSVDT_CHK(cholqr_passes(nb, nrows, n, NULL, E, xb, xr, xa, NULL, 3, 1, drop_tol, T, bytes, 1));
     /* reorthogonalise against the level-1 basis (into T) and renormalise */
     RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_bgram(nb, nrows, n, n, Q, xb, xr, xa, E, xb, xr, xa, C, work, q));
     RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_zscale((int64_t)nb * n * n, -1.0, C, C, q));
     RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_bapply(nb, nrows, n, n, Q, xb, xr, xa, C, 1.0, E, xb, xr, xa, T, xb, xr, xa, q));
-    RSVDT_CHK(cholqr_passes(nb, nrows, n, T, xb, xr, xa, NULL, 2, 0, drop_tol, E, bytes));
+    RSVDT_CHK(cholqr_passes(nb, nrows, n, NULL, T, xb, xr, xa, NULL, 2, 0, drop_tol, E, bytes, 1));
     /* the level-2 columns take the dropped columns' places; one more pass */
     RSVDT_HIPCHK("CreateMtilde", rsvdt_hip_zaxpy(nel, 1.0, T, Q, q));
-    RSVDT_CHK(cholqr_passes(nb, nrows, n, Q, xb, xr, xa, NULL, 1, 0, drop_tol, T, bytes));
+    RSVDT_CHK(cholqr_passes(nb, nrows, n, NULL, Q, xb, xr, xa, NULL, 1, 0, drop_tol, T, bytes, 1));
     return 0;
 }
 

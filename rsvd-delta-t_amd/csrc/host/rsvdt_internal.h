@@ -153,7 +153,7 @@ PetscErrorCode rsvdt_cholqr(PetscInt nbatch, PetscInt nrows, PetscInt n, double 
  * rsvdt_hip_bgram_work_bytes bytes; info 256 bytes), enqueued on stream q.
  * report: read the non-positive pivot count back (synchronises) and warn. */
 typedef struct { double *G, *R, *Ri, *Ra, *Rt; void *work; int *info; } rsvdt_cholqr_work;
-PetscErrorCode rsvdt_cholqr_bufs(PetscInt nb, PetscInt nrows, PetscInt n, double *X, int64_t xb, int64_t xr,
+PetscErrorCode rsvdt_cholqr_bufs(PetscInt nb, PetscInt nrows, PetscInt n, const double *X0, double *X, int64_t xb, int64_t xr,
                                  int64_t xa, double *R_out, int npass, int shift_first, double drop_tol, double *T,
                                  size_t bytes, const rsvdt_cholqr_work *w, rsvdt_stream_t q, int report);
 /* Orthonormal basis Q of the column span of nbatch tall matrices X (same
