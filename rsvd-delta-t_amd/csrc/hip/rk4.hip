@@ -1237,8 +1237,9 @@ __global__ __launch_bounds__(256) void k_spmm_blocks(int nrows, int k, int kl, i
 #pragma unroll
                         for (int q = 0; q < BB; ++q)
                             if (b + q < b1) {
-                                sr[q] += av[u].x * x[q][u].x - av[u].y * x[q][u].y;
-                                si[q] += av[u].x * x[q][u].y + av[u].y * x[q][u].x;
+                                // written out: the same rounding whichever BB
+                                sr[q] += fma(av[u].x, x[q][u].x, -(av[u].y * x[q][u].y));
+                                si[q] += fma(av[u].y, x[q][u].x, av[u].x * x[q][u].y);
                             }
             }
 #pragma unroll
