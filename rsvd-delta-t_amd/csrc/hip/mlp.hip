@@ -240,7 +240,9 @@ __global__ void k_gemm_reduce(int64_t M, int64_t N, int nsplit, const float *__r
 
 // out[n] = sum_m A[m*lda + n] (bias gradients); out must be zeroed first.  A
 // workgroup sums 64 columns over 4 x `rows` rows: four row slots, eight loads
-// in flight each, joined in LDS before the one atomic per column.
+// in flight each, joined in LDS before the one atomic per column.  Up to 512
+// rows are at most two chunks of 256, whose two atomics onto zero give the same
+// bits in either order; above, chunks of 128 rows put more loads in flight.
 __global__ __launch_bounds__(256) void k_colsum(int64_t M, int64_t N, int rows, const float *__restrict__ A, int64_t lda,
                                                 float *__restrict__ out)
 {
@@ -441,7 +443,7 @@ extern "C" int rsvdt_hip_colsum(int64_t M, int64_t N, const float *A, int64_t ld
     int rc = rsvdt_hip_zero(out, (size_t)N * sizeof(float), s);
     if (rc || M <= 0) return rc;
     if ((M + 255) / 256 > 65535) { set_error_msg("rsvdt_hip_colsum: M too large"); return RSVDT_HIP_ERR_ARG; }
-    const int rows = M <= 65535 * 128 ? 32 : 64;
+    const int rows = M > 512 && M <= 65535 * 128 ? 32 : 64;
     hipLaunchKernelGGL(k_colsum, dim3(ceil_div(N, 64), ceil_div(M, 4 * rows)), dim3(256), 0, as_stream(s), M, N, rows,
                        A, lda, out);
     RSVDT_LAUNCH_CHECK("rsvdt_hip_colsum");

@@ -1,0 +1,44 @@
+"""What the kernels keep over the whole range of their arguments: sums in a
+fixed order, entries they must not read, sizes beyond one launch."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from conftest import crandn, rel
+from gpu_util import Dev, init
+
+pytestmark = pytest.mark.gpu
+V, I64 = ctypes.c_void_p, ctypes.c_int64
+EPS = 2.2e-16
+
+
+@pytest.fixture(scope="module")
+def L(pkg):
+    return init(pkg)
+
+
+def at(d, nbytes):
+    """The device pointer nbytes into a buffer."""
+    return V(d.p.value + nbytes)
+
+
+@pytest.mark.parametrize("M", [3, 200, 256, 257, 300, 384, 385, 511, 512])
+def test_colsum_order(L, pkg, M):
+    """Up to 512 rows a column is the sum of at most two chunks of 256 rows
+    (four row slots each), and so the same bits on every run: two addends onto
+    zero in either order."""
+    rng = np.random.default_rng(M)
+    N = 70
+    A = rng.standard_normal((M, N)).astype(np.float32)
+    L.rsvdt_hip_colsum.argtypes = [I64, I64, V, I64, V, V]
+    dA, out = Dev(pkg, A), Dev(pkg, np.full(N, np.nan, np.float32))
+    ref = np.zeros(N, np.float32)
+    for m0 in range(0, M, 256):
+        slot = np.zeros((4, N), np.float32)
+        for m in range(m0, min(m0 + 256, M)):
+            slot[(m - m0) % 4] += A[m]
+        ref += (slot[0] + slot[1]) + (slot[2] + slot[3])
+    for _ in range(3):
+        assert L.rsvdt_hip_colsum(M, N, dA.p, N, out.p, None) == 0
+        assert np.array_equal(out.get(np.float32, (N,)), ref)
