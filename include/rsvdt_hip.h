@@ -266,7 +266,8 @@ int rsvdt_hip_bchol_inv(int64_t nbatch, int64_t n, const double *G, double shift
  * dropping Cholesky zeroed), else 0; *count (device int, may be NULL) is
  * increased by the number of such columns.  R, D: nbatch x n x n.         */
 int rsvdt_hip_bdrop_mask(int64_t nbatch, int64_t n, const double *R, double *D, int *count, rsvdt_stream_t s);
-/* Rout_b = Ra_b * Rb_b for upper-triangular n x n (row-major). */
+/* Rout_b = Ra_b * Rb_b for upper-triangular n x n (row-major); what lies below
+ * their diagonals is not read, Rout's is zero.  Rout is neither Ra nor Rb. */
 int rsvdt_hip_btrmm_upper(int64_t nbatch, int64_t n, const double *Ra, const double *Rb,
                           double *Rout, rsvdt_stream_t s);
 /* One-sided Jacobi SVD of R_b (n x n): R = U diag(sig) W^H, sig descending.

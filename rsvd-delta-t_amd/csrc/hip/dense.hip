@@ -292,18 +292,24 @@ __global__ void k_bdrop_mask(int64_t tot, int n, const double2 *__restrict__ R, 
     D[e] = make_double2(v, 0.0);
 }
 
-// C = A B for upper-triangular A, B beyond the size of the MFMA apply below.
-__global__ void k_btrmm_upper(int n, const double2 *__restrict__ A, const double2 *__restrict__ B,
-                              double2 *__restrict__ C)
+// C = A B for upper-triangular A and B: C(i, c) = sum of A(i, l) B(l, c) over
+// i <= l <= c, so that nothing below the diagonals is read and an infinite entry
+// reaches only the sums it belongs to (a full product would multiply it by the
+// zeros).  Bound by the latency of its loads: one entry a thread, eight of its
+// terms in flight, the entries of a matrix over as many workgroups as they fill.
+// 10 products of 65 x 65: 10.8 us (21 us as a full MFMA product, 74 us with one
+// workgroup a matrix); 10 of 141 x 141: 24 us (547 us with one workgroup).
+__global__ __launch_bounds__(256) void k_btrmm_upper(int n, const double2 *__restrict__ A,
+                                                     const double2 *__restrict__ B, double2 *__restrict__ C)
 {
-    const int64_t b = blockIdx.x;
-    const double2 *Ab = A + b * n * n, *Bb = B + b * n * n;
-    double2 *Cb = C + b * n * n;
-    for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
-        const int i = e / n, c = e % n;
+    const int64_t b = blockIdx.x, nn = (int64_t)n * n;
+    const double2 *Ab = A + b * nn, *Bb = B + b * nn;
+    for (int64_t e = (int64_t)blockIdx.y * 256 + threadIdx.x; e < nn; e += (int64_t)gridDim.y * 256) {
+        const int i = (int)(e / n), c = (int)(e - (int64_t)i * n);
         double2 s = make_double2(0, 0);
-        for (int l = i; l <= c; ++l) s = zadd(s, zmul(Ab[i * n + l], Bb[l * n + c]));
-        Cb[e] = s;
+#pragma unroll 8
+        for (int l = i; l <= c; ++l) s = zadd(s, zmul(Ab[(int64_t)i * n + l], Bb[(int64_t)l * n + c]));
+        C[b * nn + e] = s;
     }
 }
 
@@ -838,13 +844,9 @@ extern "C" int rsvdt_hip_btrmm_upper(int64_t nbatch, int64_t n, const double *Ra
                                      rsvdt_stream_t s)
 {
     if (nbatch <= 0 || n <= 0) return RSVDT_HIP_OK;
-    // The zeros below the diagonals add nothing, so the product is the batched
-    // MFMA apply (10 products of 65 x 65: 106 us with a serial sum per entry,
-    // 24 us); larger matrices do not fit its LDS tile.
-    if (n <= 140 && nbatch <= 65535)
-        return rsvdt_hip_bapply(nbatch, n, n, n, Ra, n * n, n, 1, Rb, 0.0, nullptr, 0, 0, 0, Rout, n * n, n, 1, s);
-    hipLaunchKernelGGL(k_btrmm_upper, dim3((unsigned)nbatch), dim3(256), 0, as_stream(s), (int)n,
-                       (const double2 *)Ra, (const double2 *)Rb, (double2 *)Rout);
+    const int64_t gy = (n * n + 255) / 256;
+    hipLaunchKernelGGL(k_btrmm_upper, dim3((unsigned)nbatch, (unsigned)(gy < 65535 ? gy : 65535)), dim3(256), 0,
+                       as_stream(s), (int)n, (const double2 *)Ra, (const double2 *)Rb, (double2 *)Rout);
     RSVDT_LAUNCH_CHECK("rsvdt_hip_btrmm_upper");
     return RSVDT_HIP_OK;
 }

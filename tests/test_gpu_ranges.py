@@ -42,3 +42,23 @@ def test_colsum_order(L, pkg, M):
     for _ in range(3):
         assert L.rsvdt_hip_colsum(M, N, dA.p, N, out.p, None) == 0
         assert np.array_equal(out.get(np.float32, (N,)), ref)
+
+
+@pytest.mark.parametrize("n", [2, 17, 65, 140, 141])
+def test_trmm_reads_the_upper_triangles(L, pkg, n):
+    """Whatever lies below the diagonals is not read, and an infinite entry
+    reaches only the entries that its row and column form."""
+    rng = np.random.default_rng(n)
+    A, B = crandn(rng, 3, n, n), crandn(rng, 3, n, n)
+    low = np.tril_indices(n, -1)
+    ref = np.triu(A) @ np.triu(B)
+    A[0][low], B[1][low] = np.nan, np.inf
+    A[2, 0, n - 1] = np.inf                # enters Out(0, n-1) alone
+    dA, dB, dC = Dev(pkg, A), Dev(pkg, B), Dev(pkg, nbytes=A.nbytes)
+    L.rsvdt_hip_btrmm_upper.argtypes = [I64, I64, V, V, V, V]
+    assert L.rsvdt_hip_btrmm_upper(3, n, dA.p, dB.p, dC.p, None) == 0
+    out = dC.get(np.complex128, A.shape)
+    assert not np.isfinite(out[2, 0, n - 1])
+    out[2, 0, n - 1] = ref[2, 0, n - 1] = 0
+    assert np.max(np.abs(out - ref)) <= 8 * EPS * (n + 1) * 36        # |entries| < 6
+    assert np.all(np.tril(out, -1) == 0)
