@@ -1256,28 +1256,33 @@ extern "C" int rsvdt_hip_spmm_blocks(int64_t nrows, int64_t k, int64_t nb, const
     if (nrows <= 0 || k <= 0 || nb <= 0) return RSVDT_HIP_OK;
     if (nb > 65535 || nrows > 0x7fffffffLL) { set_error_msg("rsvdt_hip_spmm_blocks: bad size"); return RSVDT_HIP_ERR_ARG; }
     const int kl = k < 256 ? (int)k : 256, rpb = 256 / kl;
-    const int64_t gx = ceil_div(nrows, rpb);
-    // blocks a workgroup forms: as many as leave four workgroups a CU (a group
-    // of four in flight hides more latency than more workgroups do: 28 blocks
-    // of 2549 x 23 take 26.9 us one block at a time, 18.2 us in fours), at most 8
-    int64_t bpw = gx * nb / 1024;
-    bpw = bpw < 1 ? 1 : (bpw >= 8 ? 8 : (bpw > 4 ? 4 : bpw));
-    if (bpw > nb) bpw = nb;
-    const dim3 grid((unsigned)gx, ceil_div(nb, bpw));
     const double bytes = 16.0 * (double)nrows * (double)k * (double)nb;
-#define RSVDT_SPB(NT, BB)                                                                                          \
-    hipLaunchKernelGGL((k_spmm_blocks<NT, BB>), grid, dim3(256), 0, as_stream(s), (int)nrows, (int)k, kl, rpb,       \
-                       (int)nb, (int)bpw, rowptr, col, (const double2 *)val_complex, (const double2 *)in,           \
-                       in_bstride, (double2 *)out, out_bstride)
-#define RSVDT_SPN(BB)                                                                                              \
-    if (nt) RSVDT_SPB(true, BB);                                                                                   \
-    else RSVDT_SPB(false, BB)
     const bool nt = bytes > 256e6;              // beyond the last-level cache: no point in keeping it there
-    if (bpw == 1) { RSVDT_SPN(1); }
-    else if (bpw == 2) { RSVDT_SPN(2); }
-    else { RSVDT_SPN(4); }
+    // a launch takes fewer than 2^24 workgroups (2^32 threads): further rows in
+    // further launches
+    const int64_t most = (((int64_t)1 << 24) - 1) * rpb;
+    for (int64_t r0 = 0; r0 < nrows; r0 += most) {
+        const int64_t nr = nrows - r0 < most ? nrows - r0 : most, gx = ceil_div(nr, rpb);
+        // blocks a workgroup forms: as many as leave four workgroups a CU (a group
+        // of four in flight hides more latency than more workgroups do: 28 blocks
+        // of 2549 x 23 take 26.9 us one block at a time, 18.2 us in fours), at most 8
+        int64_t bpw = gx * nb / 1024;
+        bpw = bpw < 1 ? 1 : (bpw >= 8 ? 8 : (bpw > 4 ? 4 : bpw));
+        if (bpw > nb) bpw = nb;
+        const dim3 grid((unsigned)gx, ceil_div(nb, bpw));
+#define RSVDT_SPB(NT, BB)                                                                                          \
+        hipLaunchKernelGGL((k_spmm_blocks<NT, BB>), grid, dim3(256), 0, as_stream(s), (int)nr, (int)k, kl, rpb,     \
+                           (int)nb, (int)bpw, rowptr + r0, col, (const double2 *)val_complex, (const double2 *)in,  \
+                           in_bstride, (double2 *)out + r0 * k, out_bstride)
+#define RSVDT_SPN(BB)                                                                                              \
+        if (nt) RSVDT_SPB(true, BB);                                                                               \
+        else RSVDT_SPB(false, BB)
+        if (bpw == 1) { RSVDT_SPN(1); }
+        else if (bpw == 2) { RSVDT_SPN(2); }
+        else { RSVDT_SPN(4); }
 #undef RSVDT_SPN
 #undef RSVDT_SPB
+    }
     RSVDT_LAUNCH_CHECK("rsvdt_hip_spmm_blocks");
     return RSVDT_HIP_OK;
 }

@@ -62,3 +62,35 @@ def test_trmm_reads_the_upper_triangles(L, pkg, n):
     out[2, 0, n - 1] = ref[2, 0, n - 1] = 0
     assert np.max(np.abs(out - ref)) <= 8 * EPS * (n + 1) * 36        # |entries| < 6
     assert np.all(np.tril(out, -1) == 0)
+
+
+def test_spmm_blocks_many_rows(L, pkg):
+    """More rows than one launch has workgroups for (one row each above 128
+    columns): the rows around the seam and at both ends."""
+    rows, k, cols = (1 << 24) + 100, 171, 5
+    rng = np.random.default_rng(1)
+    at_rows = [0, (1 << 24) - 2, (1 << 24) - 1, 1 << 24, rows - 1]
+    cnt = np.zeros(rows + 1, np.int32)
+    cnt[np.array(at_rows) + 1] = 1
+    rp = np.cumsum(cnt, dtype=np.int64).astype(np.int32)
+    ci = np.arange(5, dtype=np.int32)
+    v, x = crandn(rng, 5), crandn(rng, cols, k)
+    held = [Dev(pkg, a) for a in (rp, ci, v, x)]
+    out = Dev(pkg, nbytes=rows * k * 16)
+    L.rsvdt_hip_spmm_blocks.argtypes = [I64] * 3 + [V, V, V, V, I64, V, I64, V]
+    span = 4
+    for r in at_rows:
+        r0 = min(r, rows - span)
+        nan = np.full((span, k), np.nan + 0j)
+        assert L.rsvdt_hip_memcpy_h2d(at(out, r0 * k * 16), nan.ctypes.data_as(V), nan.nbytes) == 0
+    assert L.rsvdt_hip_spmm_blocks(rows, k, 1, *[h.p for h in held], cols * k, out.p, rows * k, None) == 0
+    for r in at_rows:
+        r0 = min(r, rows - span)
+        got = np.empty((span, k), complex)
+        assert L.rsvdt_hip_memcpy_d2h(got.ctypes.data_as(V), at(out, r0 * k * 16), got.nbytes) == 0
+        ref = np.zeros((span, k), complex)
+        for q in range(span):
+            if r0 + q in at_rows:
+                e = at_rows.index(r0 + q)
+                ref[q] = v[e] * x[e]
+        assert np.max(np.abs(got - ref)) <= 4 * EPS * 36
