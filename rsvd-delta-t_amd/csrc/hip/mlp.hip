@@ -172,8 +172,11 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(int M, int N, int K, int kchu
     __shared__ __align__(16) __bf16 As[GT * GP];
     __shared__ __align__(16) __bf16 Bs[GT * GP];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int nM = (M + GT - 1) / GT, nN = (N + GT - 1) / GT;
-    const gemm_tile bt = gemm_tile_of(blockIdx.x, nM, nN, nsplit);
+    const int nM = (M - 1) / GT + 1, nN = (N - 1) / GT + 1;
+    // two grid dimensions, as one holds less than 2^24 workgroups of 256 threads
+    const unsigned f = blockIdx.y * gridDim.x + blockIdx.x;
+    if (f >= (unsigned)(nM * nN * nsplit)) return;
+    const gemm_tile bt = gemm_tile_of((int)f, nM, nN, nsplit);
     const int64_t m0 = (int64_t)bt.m * GT, n0 = (int64_t)bt.n * GT;
     const int wm = (wv >> 1) * 32, wn = (wv & 1) * 32;
     const int64_t kb = (int64_t)bt.s * kchunk;
@@ -399,7 +402,8 @@ extern "C" int rsvdt_hip_gemm_bf16(int64_t M, int64_t N, int64_t K, const float 
         }
         part = g_gemm_part;
     }
-    dim3 grid((unsigned)(tiles * nsplit));
+    const int64_t gx = tiles * nsplit < (1 << 22) ? tiles * nsplit : 1 << 22;
+    dim3 grid((unsigned)gx, ceil_div(tiles * nsplit, gx));
     hipStream_t st = as_stream(s);
     // AK: A k-contiguous (sak == 1), else read along its rows; BK: likewise for B
     const bool ak = sak == 1, bk = sbk == 1;

@@ -94,3 +94,26 @@ def test_spmm_blocks_many_rows(L, pkg):
                 e = at_rows.index(r0 + q)
                 ref[q] = v[e] * x[e]
         assert np.max(np.abs(got - ref)) <= 4 * EPS * 36
+
+
+def test_gemm_bf16_many_tiles(L, pkg):
+    """More tiles of C than one grid dimension has workgroups for."""
+    M, N = 65, (1 << 29) + 70
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    L.rsvdt_hip_mem_info.argtypes = [V, V]
+    assert L.rsvdt_hip_mem_info(ctypes.byref(free), ctypes.byref(total)) == 0
+    if free.value < 150e9:
+        pytest.skip("needs 150 GB of device memory")
+    a = np.arange(1, M + 1, dtype=np.float32)         # whole numbers: exact in BF16
+    b = np.array([3], np.float32)
+    dA, dB, dC = Dev(pkg, a), Dev(pkg, b), Dev(pkg, nbytes=M * N * 4)
+    L.rsvdt_hip_gemm_bf16.argtypes = [I64] * 3 + [V, I64, I64, V, I64, I64, V, I64, ctypes.c_int, V, V, I64, V]
+    places = [(0, 0), (0, (1 << 29) - 64), (0, N - 128), (64, 0), (64, (1 << 29) - 64), (64, N - 128)]
+    for m, n in places:
+        nan = np.full(128, np.nan, np.float32)
+        assert L.rsvdt_hip_memcpy_h2d(at(dC, (m * N + n) * 4), nan.ctypes.data_as(V), nan.nbytes) == 0
+    assert L.rsvdt_hip_gemm_bf16(M, N, 1, dA.p, 1, 1, dB.p, 1, 0, dC.p, N, 0, None, None, 0, None) == 0
+    for m, n in places:
+        got = np.empty(128, np.float32)
+        assert L.rsvdt_hip_memcpy_d2h(got.ctypes.data_as(V), at(dC, (m * N + n) * 4), got.nbytes) == 0
+        assert np.array_equal(got, np.full(128, 3.0 * a[m], np.float32))
