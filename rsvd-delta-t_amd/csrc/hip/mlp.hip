@@ -448,8 +448,13 @@ extern "C" int rsvdt_hip_colsum(int64_t M, int64_t N, const float *A, int64_t ld
     if (rc || M <= 0) return rc;
     if ((M + 255) / 256 > 65535) { set_error_msg("rsvdt_hip_colsum: M too large"); return RSVDT_HIP_ERR_ARG; }
     const int rows = M > 512 && M <= 65535 * 128 ? 32 : 64;
-    hipLaunchKernelGGL(k_colsum, dim3(ceil_div(N, 64), ceil_div(M, 4 * rows)), dim3(256), 0, as_stream(s), M, N, rows,
-                       A, lda, out);
+    // a launch takes fewer than 2^24 workgroups: further columns in further launches
+    const int64_t most = (int64_t)1 << 29;
+    for (int64_t n0 = 0; n0 < N; n0 += most) {
+        const int64_t nc = N - n0 < most ? N - n0 : most;
+        hipLaunchKernelGGL(k_colsum, dim3(ceil_div(nc, 64), ceil_div(M, 4 * rows)), dim3(256), 0, as_stream(s), M, nc,
+                           rows, A + n0, lda, out + n0);
+    }
     RSVDT_LAUNCH_CHECK("rsvdt_hip_colsum");
     return RSVDT_HIP_OK;
 }

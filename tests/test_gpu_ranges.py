@@ -117,3 +117,20 @@ def test_gemm_bf16_many_tiles(L, pkg):
         got = np.empty(128, np.float32)
         assert L.rsvdt_hip_memcpy_d2h(got.ctypes.data_as(V), at(dC, (m * N + n) * 4), got.nbytes) == 0
         assert np.array_equal(got, np.full(128, 3.0 * a[m], np.float32))
+
+
+def test_colsum_many_columns(L, pkg):
+    """More columns than one launch has threads for: both ends."""
+    M, N = 2, (1 << 30) + 72
+    A = np.arange(M * 256, dtype=np.float32).reshape(M, 256)
+    dA, out = Dev(pkg, nbytes=M * N * 4), Dev(pkg, nbytes=N * 4)
+    L.rsvdt_hip_colsum.argtypes = [I64, I64, V, I64, V, V]
+    places = [0, N - 256]
+    for n in places:
+        for m in range(M):
+            assert L.rsvdt_hip_memcpy_h2d(at(dA, (m * N + n) * 4), A[m].ctypes.data_as(V), 1024) == 0
+    assert L.rsvdt_hip_colsum(M, N, dA.p, N, out.p, None) == 0
+    for n in places:
+        got = np.empty(256, np.float32)
+        assert L.rsvdt_hip_memcpy_d2h(got.ctypes.data_as(V), at(out, n * 4), 1024) == 0
+        assert np.array_equal(got, A.sum(0))
