@@ -637,11 +637,11 @@ extern "C" int rsvdt_hip_tr_windows(int64_t kb, int64_t k, int64_t Nw, int64_t N
 // On the host the same relayout, with its temporary's page faults, was most of
 // what a small action spent outside the GPU.
 template <bool TO_CM>
-__global__ __launch_bounds__(256) void k_cm_relayout(int64_t rows, int64_t kb, int64_t nblk, int order, int64_t c0,
-                                                     int64_t nc, double2 *cm, double2 *blk) {
+__global__ __launch_bounds__(256) void k_cm_relayout(int64_t row0, int64_t rows, int64_t kb, int64_t nblk, int order,
+                                                     int64_t c0, int64_t nc, double2 *cm, double2 *blk) {
     __shared__ double2 tile[32][33];
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    const int64_t r0 = (int64_t)blockIdx.x * 32, t0 = (int64_t)blockIdx.y * 32;
+    const int64_t r0 = row0 + (int64_t)blockIdx.x * 32, t0 = (int64_t)blockIdx.y * 32;
     const int64_t c = c0 + t0 + tx, b = order ? c % nblk : c / kb, j = order ? c / nblk : c - b * kb;
     const bool cok = t0 + tx < nc;
     double2 *bp = blk + b * rows * kb + j;
@@ -666,13 +666,17 @@ extern "C" int rsvdt_hip_cm_relayout(int64_t rows, int64_t kb, int64_t nblk, int
         set_error_msg("rsvdt_hip_cm_relayout: columns outside the matrix, or more than 32 x 65535 of them");
         return RSVDT_HIP_ERR_ARG;
     }
-    const dim3 grid(ceil_div(rows, 32), ceil_div(nc, 32));
-    if (to_cm)
-        hipLaunchKernelGGL(k_cm_relayout<true>, grid, dim3(256), 0, as_stream(s), rows, kb, nblk, order, c0, nc,
-                           (double2 *)cm, (double2 *)blk);
-    else
-        hipLaunchKernelGGL(k_cm_relayout<false>, grid, dim3(256), 0, as_stream(s), rows, kb, nblk, order, c0, nc,
-                           (double2 *)cm, (double2 *)blk);
+    // a launch takes fewer than 2^24 workgroups: further rows in further launches
+    const int64_t most = (int64_t)1 << 28;
+    for (int64_t row0 = 0; row0 < rows; row0 += most) {
+        const dim3 grid(ceil_div(rows - row0 < most ? rows - row0 : most, 32), ceil_div(nc, 32));
+        if (to_cm)
+            hipLaunchKernelGGL(k_cm_relayout<true>, grid, dim3(256), 0, as_stream(s), row0, rows, kb, nblk, order, c0,
+                               nc, (double2 *)cm, (double2 *)blk);
+        else
+            hipLaunchKernelGGL(k_cm_relayout<false>, grid, dim3(256), 0, as_stream(s), row0, rows, kb, nblk, order, c0,
+                               nc, (double2 *)cm, (double2 *)blk);
+    }
     RSVDT_LAUNCH_CHECK("rsvdt_hip_cm_relayout");
     return RSVDT_HIP_OK;
 }

@@ -134,3 +134,24 @@ def test_colsum_many_columns(L, pkg):
         got = np.empty(256, np.float32)
         assert L.rsvdt_hip_memcpy_d2h(got.ctypes.data_as(V), at(out, n * 4), 1024) == 0
         assert np.array_equal(got, A.sum(0))
+
+
+def test_relayout_many_rows(L, pkg):
+    """More rows than one launch has threads for: both ends, both ways."""
+    rows, kb = (1 << 29) + 33, 1
+    rng = np.random.default_rng(2)
+    src, dst = Dev(pkg, nbytes=rows * 16), Dev(pkg, nbytes=rows * 16)
+    x = crandn(rng, 100)
+    L.rsvdt_hip_cm_relayout.argtypes = [I64] * 3 + [ctypes.c_int, I64, I64, V, V, ctypes.c_int, V]
+    places = [0, rows - 100]
+    for to_cm in (0, 1):
+        for r in places:
+            assert L.rsvdt_hip_memcpy_h2d(at(src, r * 16), x.ctypes.data_as(V), x.nbytes) == 0
+            nan = np.full(100, np.nan + 0j)
+            assert L.rsvdt_hip_memcpy_h2d(at(dst, r * 16), nan.ctypes.data_as(V), nan.nbytes) == 0
+        cm, blk = (dst, src) if to_cm else (src, dst)
+        assert L.rsvdt_hip_cm_relayout(rows, kb, 1, 0, 0, 1, cm.p, blk.p, to_cm, None) == 0
+        for r in places:
+            got = np.empty(100, complex)
+            assert L.rsvdt_hip_memcpy_d2h(got.ctypes.data_as(V), at(dst, r * 16), got.nbytes) == 0
+            assert np.array_equal(got, x)
