@@ -200,9 +200,10 @@ __global__ __launch_bounds__(256) void k_bgram_part(
 }
 
 // G_b(a, c) = sum over the nch partial matrices of batch b, in a fixed order:
-// 32 entries x 8 slices of the partials per workgroup, the slices' sums
-// combined through LDS.  One thread per entry walking all partials was a
-// serial chain of loads (165 us for 16 batches of 512 partials of 16 x 16).
+// 32 entries x 8 slices of the partials per workgroup (and further entries, as
+// a launch takes fewer than 2^24 workgroups), the slices' sums combined through
+// LDS.  One thread per entry walking all partials was a serial chain of loads
+// (165 us for 16 batches of 512 partials of 16 x 16).
 // herm: the tiles below the diagonal (and the border row) were not formed and
 // are the conjugates of their mirrors; ntile: the 16-wide tiles (columns from
 // 16 ntile on are the border).
@@ -212,26 +213,29 @@ __global__ __launch_bounds__(256) void k_bgram_reduce(int64_t nch, int na, int n
     __shared__ double2 sh[8][32];
     const int64_t b = blockIdx.y;
     const int64_t per = (int64_t)na * nc;
-    const int64_t e = (int64_t)blockIdx.x * 32 + (int)(threadIdx.x & 31);
     const int sl = threadIdx.x >> 5;
-    double2 s = make_double2(0, 0);
-    bool mir = false;
-    if (e < per) {
-        const int a = (int)(e / nc), c = (int)(e % nc);
-        const int ta = min(a / 16, ntile), tc = min(c / 16, ntile);
-        mir = herm && ta > tc;
-        const double2 *p = part + b * nch * per + (mir ? (int64_t)c * nc + a : e);
-        for (int64_t ch = sl; ch < nch; ch += 8) {
-            const double2 v = p[ch * per];
-            s.x += v.x; s.y += v.y;
+    for (int64_t e0 = (int64_t)blockIdx.x * 32; e0 < per; e0 += (int64_t)gridDim.x * 32) {
+        const int64_t e = e0 + (int)(threadIdx.x & 31);
+        double2 s = make_double2(0, 0);
+        bool mir = false;
+        if (e < per) {
+            const int a = (int)(e / nc), c = (int)(e % nc);
+            const int ta = min(a / 16, ntile), tc = min(c / 16, ntile);
+            mir = herm && ta > tc;
+            const double2 *p = part + b * nch * per + (mir ? (int64_t)c * nc + a : e);
+            for (int64_t ch = sl; ch < nch; ch += 8) {
+                const double2 v = p[ch * per];
+                s.x += v.x; s.y += v.y;
+            }
         }
-    }
-    sh[sl][threadIdx.x & 31] = s;
-    __syncthreads();
-    if (sl == 0 && e < per) {
+        sh[sl][threadIdx.x & 31] = s;
+        __syncthreads();
+        if (sl == 0 && e < per) {
 #pragma unroll
-        for (int q = 1; q < 8; ++q) { s.x += sh[q][threadIdx.x].x; s.y += sh[q][threadIdx.x].y; }
-        G[b * per + e] = make_double2(s.x, mir ? -s.y : s.y);
+            for (int q = 1; q < 8; ++q) { s.x += sh[q][threadIdx.x].x; s.y += sh[q][threadIdx.x].y; }
+            G[b * per + e] = make_double2(s.x, mir ? -s.y : s.y);
+        }
+        __syncthreads();
     }
 }
 
@@ -261,7 +265,7 @@ __global__ __launch_bounds__(256) void k_bgram_reduce(int64_t nch, int na, int n
 // two waves per SIMD for half tiles (742 us with one).
 template <int TA, int TC, bool HERM, bool BORD>
 __global__ __launch_bounds__(256, TA *TC <= 1 ? 4 : (TA == 4 && !HERM ? 2 : 1)) void k_bgram_mfma(
-    int64_t nrows, int na, int nc, int64_t chunk, int ntc, const double2 *X, int64_t xb, int64_t xr,
+    int64_t nrows, int na, int nc, int64_t chunk, int tile0, int ntc, const double2 *X, int64_t xb, int64_t xr,
     const double2 *Z, int64_t zb, int64_t zr, double2 *__restrict__ part)
 {
     constexpr int GA = TA == 4 && !HERM ? 2 : 1, WA = TA / GA, NSUB = 4 / GA;
@@ -271,7 +275,7 @@ __global__ __launch_bounds__(256, TA *TC <= 1 ? 4 : (TA == 4 && !HERM ? 2 : 1)) 
     const int lane = threadIdx.x & 63, wv = wave_id();
     const int h = wv % GA, sub = wv / GA;
     const int64_t b = blockIdx.z;
-    const int a0 = (int)(blockIdx.y / ntc) * (16 * TA), c0 = (int)(blockIdx.y % ntc) * CW;
+    const int mt = tile0 + (int)blockIdx.y, a0 = (mt / ntc) * (16 * TA), c0 = (mt % ntc) * CW;
     const int aw = a0 + 16 * WA * h;             // first row of G of this wave
     const int64_t r_begin = (int64_t)blockIdx.x * chunk;
     const int64_t r_end = r_begin + chunk < nrows ? r_begin + chunk : nrows;
@@ -439,6 +443,12 @@ __global__ __launch_bounds__(256, TA *TC <= 1 ? 4 : (TA == 4 && !HERM ? 2 : 1)) 
     }
 }
 
+static dim3 bgram_reduce_grid(int64_t entries, int64_t nbatch)
+{
+    const int64_t gx = (entries + 31) / 32;
+    return dim3((unsigned)(gx < (1 << 20) ? gx : 1 << 20), (unsigned)nbatch);
+}
+
 // Partials that rsvdt_hip_bgram_work_bytes has room for (the plans below use
 // at most as many): about 2048 workgroups of four tiles of up to 48 x 48.
 static int64_t bgram_work_parts(int64_t nbatch, int64_t nrows, int64_t na, int64_t nc)
@@ -492,8 +502,11 @@ static int launch_bgram_mfma(const bgram_mfma_plan &p, int64_t nbatch, int64_t n
                              double2 *part, hipStream_t s)
 {
     const size_t lds = (size_t)(256 * TA * TC + 16 * TA + 16 * TC + 1) * 16;
-    hipLaunchKernelGGL((k_bgram_mfma<TA, TC, HERM, BORD>), dim3((unsigned)p.nch, (unsigned)p.ntiles, (unsigned)nbatch),
-                       dim3(256), lds, s, nrows, (int)na, (int)nc, p.chunk, p.ntc, X, xb, xr, Z, zb, zr, part);
+    for (int t0 = 0; t0 < p.ntiles; t0 += 65535) {     // what a launch takes in this dimension
+        const unsigned gy = (unsigned)(p.ntiles - t0 < 65535 ? p.ntiles - t0 : 65535);
+        hipLaunchKernelGGL((k_bgram_mfma<TA, TC, HERM, BORD>), dim3((unsigned)p.nch, gy, (unsigned)nbatch), dim3(256), lds,
+                           s, nrows, (int)na, (int)nc, p.chunk, t0, p.ntc, X, xb, xr, Z, zb, zr, part);
+    }
     RSVDT_LAUNCH_CHECK("rsvdt_hip_bgram(mfma)");
     return RSVDT_HIP_OK;
 }
@@ -1036,7 +1049,7 @@ extern "C" int rsvdt_hip_bgram(int64_t nbatch, int64_t nrows, int64_t na, int64_
         RSVDT_LAUNCH_CHECK("rsvdt_hip_bgram(part)");
         nparts = nch;
     }
-    hipLaunchKernelGGL(k_bgram_reduce, dim3(ceil_div(na * nc, 32), (unsigned)nbatch), dim3(256), 0, st, nparts, (int)na,
+    hipLaunchKernelGGL(k_bgram_reduce, bgram_reduce_grid(na * nc, nbatch), dim3(256), 0, st, nparts, (int)na,
                        (int)nc, herm, ntile, (const double2 *)work, (double2 *)G);
     RSVDT_LAUNCH_CHECK("rsvdt_hip_bgram(reduce)");
     return RSVDT_HIP_OK;
@@ -1161,7 +1174,7 @@ extern "C" int rsvdt_hip_bapply_gram(int64_t nbatch, int64_t nrows, int64_t n, c
         return rc || !G ? rc : rsvdt_hip_bgram(nbatch, nrows, n, n, Out, xb, xr, 1, Out, xb, xr, 1, G, work, s);
     }
     if (rc || !G) return rc;
-    hipLaunchKernelGGL(k_bgram_reduce, dim3(ceil_div(n * n, 32), (unsigned)nbatch), dim3(256), 0, st, np, (int)n, (int)n,
+    hipLaunchKernelGGL(k_bgram_reduce, bgram_reduce_grid(n * n, nbatch), dim3(256), 0, st, np, (int)n, (int)n,
                        1, TC, (const double2 *)work, (double2 *)G);
     RSVDT_LAUNCH_CHECK("rsvdt_hip_bapply_gram(reduce)");
     return RSVDT_HIP_OK;

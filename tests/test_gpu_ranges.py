@@ -155,3 +155,22 @@ def test_relayout_many_rows(L, pkg):
             got = np.empty(100, complex)
             assert L.rsvdt_hip_memcpy_d2h(got.ctypes.data_as(V), at(dst, r * 16), got.nbytes) == 0
             assert np.array_equal(got, x)
+
+
+@pytest.mark.parametrize("n", [16449, 23200])
+def test_gram_many_tiles(L, pkg, n):
+    """More macro tiles than one grid dimension takes, and more entries than
+    one launch of the reduction: corners of X^H Z."""
+    nr = 3
+    rng = np.random.default_rng(n)
+    X, Z = crandn(rng, nr, n), crandn(rng, nr, n)
+    L.rsvdt_hip_bgram_work_bytes.restype = ctypes.c_size_t
+    L.rsvdt_hip_bgram_work_bytes.argtypes = [I64] * 4
+    L.rsvdt_hip_bgram.argtypes = [I64] * 4 + [V, I64, I64, I64, V, I64, I64, I64, V, V, V]
+    dX, dZ, dG = Dev(pkg, X), Dev(pkg, Z), Dev(pkg, nbytes=n * n * 16)
+    dw = Dev(pkg, nbytes=L.rsvdt_hip_bgram_work_bytes(1, nr, n, n))
+    assert L.rsvdt_hip_bgram(1, nr, n, n, dX.p, nr * n, n, 1, dZ.p, nr * n, n, 1, dG.p, dw.p, None) == 0
+    for a in (0, 63, n // 2, 16383, 16384, n - 2, n - 1):
+        row = np.empty(n, complex)
+        assert L.rsvdt_hip_memcpy_d2h(row.ctypes.data_as(V), at(dG, a * n * 16), row.nbytes) == 0
+        assert np.max(np.abs(row - X[:, a].conj() @ Z)) <= 8 * EPS * nr * 36
