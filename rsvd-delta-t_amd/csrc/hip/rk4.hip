@@ -1179,8 +1179,8 @@ extern "C" int rsvdt_hip_horner_stage(const rsvdt_spmm_desc *d, const void *vin,
 // applied to all frequencies at once).  M is rows x cols CSR, complex FP64;
 // In blocks are cols x k, Out blocks rows x k.
 //
-// k lanes own a row (any k up to 256, not a power of two: a workgroup is a
-// flat run of 256 / k rows).  Bound by latency: neighbouring rows gather the
+// kl lanes own a row, k of them where they fit (not a power of two: a workgroup
+// is a flat run of 256 / kl rows).  Bound by latency: neighbouring rows gather the
 // same rows of In, so few distinct bytes are in flight unless a wave works on
 // several blocks at once.  It gathers two entries for BB blocks together (four,
 // or as many as there are), the row's first entries kept in registers over the
@@ -1255,7 +1255,13 @@ extern "C" int rsvdt_hip_spmm_blocks(int64_t nrows, int64_t k, int64_t nb, const
 {
     if (nrows <= 0 || k <= 0 || nb <= 0) return RSVDT_HIP_OK;
     if (nb > 65535 || nrows > 0x7fffffffLL) { set_error_msg("rsvdt_hip_spmm_blocks: bad size"); return RSVDT_HIP_ERR_ARG; }
-    const int kl = k < 256 ? (int)k : 256, rpb = 256 / kl;
+    // lanes a row: a column each, up to 256.  One block alone has no second block to
+    // keep in flight: where a workgroup would have two rows or one, from 86 to 320
+    // columns, at most 64 lanes a row with two to five columns each keep as much in
+    // flight and leave fewer lanes without a row (one block of 100,000 x 128 with an
+    // entry a row: 81 -> 73 us, x 129: 119 -> 78 us, x 200: 140 -> 122 us)
+    const int64_t cpl = nb == 1 && k >= 86 && k <= 320 ? (k + 63) / 64 : 1;
+    const int kl = (int)(cpl > 1 ? (k + cpl - 1) / cpl : (k < 256 ? k : 256)), rpb = 256 / kl;
     const double bytes = 16.0 * (double)nrows * (double)k * (double)nb;
     const bool nt = bytes > 256e6;              // beyond the last-level cache: no point in keeping it there
     // a launch takes fewer than 2^24 workgroups (2^32 threads): further rows in
@@ -1268,6 +1274,9 @@ extern "C" int rsvdt_hip_spmm_blocks(int64_t nrows, int64_t k, int64_t nb, const
         // of 2549 x 23 take 26.9 us one block at a time, 18.2 us in fours), at most 8
         int64_t bpw = gx * nb / 1024;
         bpw = bpw < 1 ? 1 : (bpw >= 8 ? 8 : (bpw > 4 ? 4 : bpw));
+        // two above 120 columns, to 128: rows of 2 KB in four blocks at once slow the
+        // matrices with an entry a row (8 blocks of 100,000 x 127: 640 -> 561 us)
+        if (k > 120 && k <= 128 && bpw > 2) bpw = 2;
         if (bpw > nb) bpw = nb;
         const dim3 grid((unsigned)gx, ceil_div(nb, bpw));
 #define RSVDT_SPB(NT, BB)                                                                                          \

@@ -4,6 +4,7 @@ import ctypes
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 from conftest import crandn, rel
 from gpu_util import Dev, init
@@ -174,3 +175,28 @@ def test_gram_many_tiles(L, pkg, n):
         row = np.empty(n, complex)
         assert L.rsvdt_hip_memcpy_d2h(row.ctypes.data_as(V), at(dG, a * n * 16), row.nbytes) == 0
         assert np.max(np.abs(row - X[:, a].conj() @ Z)) <= 8 * EPS * nr * 36
+
+
+@pytest.mark.parametrize("rows,k", [(700, 85), (700, 86), (515, 128), (515, 129), (300, 171), (300, 320), (300, 321),
+                                    (40000, 121)])
+@pytest.mark.parametrize("nb", [1, 2, 9])
+def test_spmm_blocks_wide(L, pkg, rows, k, nb):
+    """Lanes of several columns each (one block of 86 to 320 columns) and blocks
+    of wide rows, with 0 to 7 entries a row: against scipy, and a block of a
+    group the same bits as the block alone."""
+    rng = np.random.default_rng(rows + k)
+    cnt = rng.integers(0, 8, rows)
+    rp = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32)
+    ci = np.concatenate([np.sort((rng.integers(rows) + np.arange(c)) % rows) for c in cnt]).astype(np.int32)
+    v, x = crandn(rng, len(ci)), crandn(rng, nb, rows, k)
+    held = [Dev(pkg, a) for a in (rp, ci, v)]
+    dx, out, one = Dev(pkg, x), Dev(pkg, np.full((nb, rows, k), np.nan + 0j)), Dev(pkg, nbytes=rows * k * 16)
+    L.rsvdt_hip_spmm_blocks.argtypes = [I64] * 3 + [V, V, V, V, I64, V, I64, V]
+    p = [h.p for h in held]
+    assert L.rsvdt_hip_spmm_blocks(rows, k, nb, *p, dx.p, rows * k, out.p, rows * k, None) == 0
+    got = out.get(np.complex128, (nb, rows, k))
+    M = sp.csr_matrix((v, ci, rp), shape=(rows, rows))
+    for b in (0, nb - 1):
+        assert np.max(np.abs(got[b] - M @ x[b])) <= 4 * 7 * EPS * 36      # sums of 7 products of |.| < 6 each
+        assert L.rsvdt_hip_spmm_blocks(rows, k, 1, *p, at(dx, b * rows * k * 16), rows * k, one.p, rows * k, None) == 0
+        assert np.array_equal(got[b], one.get(np.complex128, (rows, k)))
