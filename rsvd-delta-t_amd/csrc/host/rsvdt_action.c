@@ -709,14 +709,15 @@ static int leap_pays(Mat A, int dir, RSVDt_vars *V)
     return leaps < 0.7 * one_by_one;
 }
 
-/* E of A (dir 1) or A^H: nsteps homogeneous steps of the identity. */
+/* E of A (dir 1) or A^H: nsteps homogeneous steps of the identity.  *out is NULL
+ * when there is no room for it: the caller steps one by one. */
 static PetscErrorCode leap_operator(Mat A, int dir, double h, PetscInt nsteps, const double **out)
 {
     const int q = dir ? 0 : 1;
     const PetscInt N = A->rows;
+    *out = NULL;
     if (!A->leap[q].d || A->leap[q].h != h || A->leap[q].steps != nsteps) {
-        if (!A->leap[q].d)
-            RSVDT_HIPCHK("TSActionRK4", rsvdt_hip_malloc((void **)&A->leap[q].d, (size_t)N * (size_t)N * 16));
+        if (!A->leap[q].d && rsvdt_hip_malloc((void **)&A->leap[q].d, (size_t)N * (size_t)N * 16)) return 0;
         A->leap[q].steps = 0;                /* not valid until both launches are queued */
         rsvdt_spmm_desc d;
         desc_for(&d, A, dir, 64, N, 1);
@@ -731,10 +732,38 @@ static PetscErrorCode leap_operator(Mat A, int dir, double h, PetscInt nsteps, c
     return 0;
 }
 
+/* What a leaping action needs beside its data: E, the H_m, the state and the
+ * forcing terms formed at a time (samples of the first steps, then of leaps). */
+enum { LEAP_CHUNK = 256 };
+typedef struct { const double *E; double *H, *y0, *y1, *f; } leap_bufs;
+
+/* E is NULL when one of them cannot be had (the others then are given back). */
+static PetscErrorCode leap_reserve(Mat A, RSVDt_vars *V, leap_bufs *b, phase_timer *t_frc)
+{
+    const PetscInt Nw = V->RSVD.Nw, RR = V->TS.ResRatio, r0 = V->TS.Nt % RR;
+    const PetscInt nleap = V->TS.Nt / RR + (V->TS.TransientRemoval ? Nw + 1 : Nw), most = r0 > nleap ? r0 : nleap;
+    const size_t blk = (size_t)A->rows * (size_t)V->RSVD.k * 16;
+    memset(b, 0, sizeof(*b));
+    b->H = rsvdt_scratch(SCR_H, blk * (size_t)V->RSVD.Nw_eff);
+    b->y0 = b->H ? rsvdt_scratch(SCR_Y, blk) : NULL;
+    b->y1 = b->y0 ? rsvdt_scratch(SCR_U1, blk) : NULL;
+    b->f = b->y1 ? rsvdt_scratch(SCR_FBUF, blk * (size_t)(most < LEAP_CHUNK ? most : LEAP_CHUNK)) : NULL;
+    if (b->f) {
+        if (t_frc) pt_begin(t_frc);
+        RSVDT_CHK(leap_operator(A, V->TS.DirAdj ? 1 : 0, V->TS.dt, RR, &b->E));
+        if (t_frc) pt_end(t_frc);
+    }
+    if (!b->E) {
+        rsvdt_scratch_release(SCR_H);
+        rsvdt_scratch_release(SCR_FBUF);
+    }
+    return 0;
+}
+
 /* The stepping of an action (as time_stepping below) by leaps: G holds the
  * folded forcing terms, Yall receives the snapshots. */
-static PetscErrorCode leap_stepping(Mat A, DFT_matrices *D, RSVDt_vars *V, const double *G, Mat Yall, phase_timer *t_rk4,
-                                    phase_timer *t_frc, int64_t *launches)
+static PetscErrorCode leap_stepping(Mat A, DFT_matrices *D, RSVDt_vars *V, const double *G, Mat Yall, const leap_bufs *b,
+                                    phase_timer *t_rk4, phase_timer *t_frc, int64_t *launches)
 {
     const int dir = V->TS.DirAdj ? 1 : 0, sgn = dir ? 1 : -1;
     const PetscInt N = A->rows, k = V->RSVD.k, Nwe = V->RSVD.Nw_eff, RR = V->TS.ResRatio, Nt = V->TS.Nt;
@@ -742,17 +771,12 @@ static PetscErrorCode leap_stepping(Mat A, DFT_matrices *D, RSVDt_vars *V, const
     const int64_t L = N * k, nt2 = 2 * V->TS.Ns, maxrow = dir ? A->maxrow : A->maxrowH;
     const size_t blk = (size_t)L * 16;
     const double h = V->TS.dt, cf[4] = {h / 4, h / 3, h / 2, h};
-    const PetscInt chunk = 256;              /* forcing terms formed at a time: samples of the first steps, then leaps */
+    const PetscInt chunk = LEAP_CHUNK;
     rsvdt_stream_t q = g_rsvdt.stream;
-    double *H = rsvdt_scratch(SCR_H, blk * (size_t)Nwe);
-    double *y0 = rsvdt_scratch(SCR_Y, blk), *y1 = rsvdt_scratch(SCR_U1, blk);
-    const PetscInt most = r0 > nlead + nsnap ? r0 : nlead + nsnap;
-    double *f = rsvdt_scratch(SCR_FBUF, blk * (size_t)(most < chunk ? most : chunk));
-    if (!H || !y0 || !y1 || !f) return rsvdt_err(RSVDT_ERR_MEM, "TSActionRK4", "cannot allocate the RK4 work buffers");
-    const double *E;
+    const double *E = b->E;
+    double *H = b->H, *y0 = b->y0, *y1 = b->y1, *f = b->f;
     rsvdt_spmm_desc d;
     if (t_frc) pt_begin(t_frc);
-    RSVDT_CHK(leap_operator(A, dir, h, RR, &E));
     desc_for(&d, A, dir, 64, k, Nwe);
     RSVDT_HIPCHK("TSActionRK4", rsvdt_hip_horner_fused_harm(&d, A->nnz, maxrow, H, G, cf, RR, D->idft->d, nt2, sgn, q));
     if (t_frc) pt_end(t_frc);
@@ -786,6 +810,16 @@ static PetscErrorCode leap_stepping(Mat A, DFT_matrices *D, RSVDt_vars *V, const
     return 0;
 }
 
+/* In an action, forcing buffers of more than 1 GiB go back to the device: the
+ * transient removal that follows sizes its groups to the free memory. */
+static void release_chunks(void)
+{
+    if (rsvdt_scratch_size(SCR_FBUF) + rsvdt_scratch_size(SCR_FBUF2) + rsvdt_scratch_size(SCR_H) <= ((size_t)1 << 30)) return;
+    rsvdt_scratch_release(SCR_FBUF);
+    rsvdt_scratch_release(SCR_FBUF2);
+    rsvdt_scratch_release(SCR_H);
+}
+
 /* The time stepping of one action (TSActionRK4.c:38-130) over rend steps.
  * With the FP32 state and transient removal, the Nt steps before the first
  * snapshot run in FP32 and the snapshot period in FP64: the FP32 rounding
@@ -807,11 +841,15 @@ static PetscErrorCode time_stepping(Mat A, DFT_matrices *D, RSVDt_vars *V, Mat F
     const int seg_prec[2] = {prec, 64};
     int64_t launches = 0;
     PetscErrorCode ierr = 0;
-    if (Yall && !fhat_folded && max_steps <= 0 && leap_pays(A, dir, V)) {
+    leap_bufs lb = {0};
+    if (Yall && !fhat_folded && max_steps <= 0 && leap_pays(A, dir, V)) RSVDT_CHK(leap_reserve(A, V, &lb, t_frc));
+    if (lb.E) {
         if (t_frc) pt_begin(t_frc);
-        RSVDT_CHK(folded_forcing(A, dir, V->TS.dt, k, Nwe, V->TS.Ns, D->idft->d, Fhat->d, Fhat->d));
+        ierr = folded_forcing(A, dir, V->TS.dt, k, Nwe, V->TS.Ns, D->idft->d, Fhat->d, Fhat->d);
         if (t_frc) pt_end(t_frc);
-        RSVDT_CHK(leap_stepping(A, D, V, Fhat->d, Yall, t_rk4, t_frc, &launches));
+        if (!ierr) ierr = leap_stepping(A, D, V, Fhat->d, Yall, &lb, t_rk4, t_frc, &launches);
+        release_chunks();
+        RSVDT_CHK(ierr);
         g_rsvdt.stats.steps = rend;
         g_rsvdt.stats.rk4_launches = launches;
         g_rsvdt.stats.chunk_steps = (int)V->TS.ResRatio;
@@ -859,12 +897,7 @@ static PetscErrorCode time_stepping(Mat A, DFT_matrices *D, RSVDt_vars *V, Mat F
         rsvdt_hip_free(y64);
     }
     stepper_free(&st);
-    /* in an action, chunk buffers of more than 1 GiB go back to the device:
-     * the transient removal that follows sizes its groups to the free memory */
-    if (Yall && rsvdt_scratch_size(SCR_FBUF) + rsvdt_scratch_size(SCR_FBUF2) > ((size_t)1 << 30)) {
-        rsvdt_scratch_release(SCR_FBUF);
-        rsvdt_scratch_release(SCR_FBUF2);
-    }
+    if (Yall) release_chunks();
     RSVDT_CHK(ierr);
     g_rsvdt.stats.steps = rend;
     g_rsvdt.stats.rk4_launches = launches;
@@ -1250,11 +1283,11 @@ static PetscErrorCode mtilde_group(LNS_vars *LNS, RSVDt_vars *V, TS_removal_matr
     const int dir = V->TS.DirAdj ? 1 : 0;
     double t0 = trt_mark();
     int h = 0;
-    if (leap_pays(LNS->A, dir, V)) {
-        /* the operator's dense propagator (the stepping of the same action built
-         * it) on the basis as it lies, N x Ns1 per test vector */
-        const double *E;
-        RSVDT_CHK(leap_operator(LNS->A, dir, V->TS.dt, V->TS.ResRatio, &E));
+    /* the operator's dense propagator (the stepping of the same action built it)
+     * on the basis as it lies, N x Ns1 per test vector */
+    const double *E = NULL;
+    if (leap_pays(LNS->A, dir, V)) RSVDT_CHK(leap_operator(LNS->A, dir, V->TS.dt, V->TS.ResRatio, &E));
+    if (E) {
         h = rsvdt_hip_dense_apply(N, Ns1, g, E, g_trg.V, NULL, MV, g_rsvdt.stream);
         trt_add(TRT_STEPS, t0);
         t0 = trt_mark();

@@ -1,0 +1,86 @@
+"""Snapshot-to-snapshot stepping of small operators: when it is taken, and what
+happens when it cannot be."""
+import os
+import shutil
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+from conftest import ROOT, crandn, load_pkg, rel
+
+pytestmark = pytest.mark.gpu
+
+SHIM = """
+#include <stddef.h>
+static int (*next)(void **, size_t);
+static size_t size;
+static int skip, refused;
+void shim_set(void *f, size_t bytes, int after) { next = (int (*)(void **, size_t))f; size = bytes; skip = after; }
+int shim_refused(void) { return refused; }
+int rsvdt_hip_malloc(void **p, size_t bytes)
+{
+    if (bytes == size && skip-- == 0) { refused++; *p = NULL; return 103; }
+    return next(p, bytes);
+}
+"""
+
+
+def operator(N, real, width=3):
+    import scipy.sparse as sp
+    rng = np.random.default_rng(N)
+    offs = range(-(width // 2), width - width // 2)
+    d = [rng.standard_normal(N - abs(o)) + (0 if real else 1j * rng.standard_normal(N - abs(o))) for o in offs]
+    return (sp.diags(d, list(offs), shape=(N, N)) - (1 + width) * sp.eye(N)).tocsr().astype(np.complex128)
+
+
+KW = dict(k=3, q=0, Nw=16, w=0.7, TL=1.0, dt=0.04)
+
+
+def refusing(shim, what, removal):
+    """Child process: one direct action with one allocation refused."""
+    import ctypes
+    S = ctypes.CDLL(shim, mode=ctypes.RTLD_GLOBAL)      # before the library, whose calls then bind to it
+    pkg = load_pkg()
+    L = pkg.lib()
+    S.shim_set.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+    real = ctypes.cast(L.rsvdt_hip_malloc, ctypes.c_void_p)
+    S.shim_set(real, 0, 0)
+    N = 301
+    A = operator(N, True)
+    out = {}
+    for fuse in (0, 1):
+        s = pkg.Session(A, transient_removal=removal, fuse_small=fuse, **KW)
+        if not fuse:
+            F = crandn(np.random.default_rng(0), N, s.k * s.Nw_eff)
+        s.set_sketch(F)
+        if fuse:        # the propagator, or the harmonic responses (as large as the forcing's two work blocks)
+            S.shim_set(real, N * N * 16 if what == "E" else N * s.k * s.Nw_eff * 16, 0)
+        s.direct()
+        out[fuse] = s.get_Y()
+        st = pkg.action_stats()
+        s.close()
+    assert S.shim_refused() == 1
+    assert st["chunk_steps"] != s.RR, "the action leapt"
+    assert rel(out[1], out[0]) < (1e-9 if removal else 1e-12)
+
+
+@pytest.mark.parametrize("what", ["E", "H"])
+@pytest.mark.parametrize("removal", [0, 1])
+def test_steps_without_room_to_leap(tmp_path, what, removal):
+    """When the propagator or the responses cannot be allocated the action steps
+    one by one, as before the forcing was folded in place."""
+    cc = shutil.which("gcc")
+    if cc is None:
+        pytest.skip("no C compiler")
+    (tmp_path / "shim.c").write_text(SHIM)
+    so = str(tmp_path / "shim.so")
+    subprocess.run([cc, "-shared", "-fPIC", "-O1", "-o", so, str(tmp_path / "shim.c")], check=True)
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), so, what, str(removal)], cwd=ROOT, timeout=100,
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+
+
+if __name__ == "__main__":
+    refusing(sys.argv[1], sys.argv[2], bool(int(sys.argv[3])))
