@@ -188,10 +188,14 @@ int rsvdt_hip_horner_fused_fits(int64_t nrows, int64_t nnz, int a_real, int prec
 int rsvdt_hip_horner_fused(const rsvdt_spmm_desc *d, int64_t nnz, int64_t maxrow, void *y, const void *g,
                            int64_t gstride, const double *coef, int64_t nsteps, double *snap, int64_t snap_stride,
                            int64_t i0, int64_t Nt, int64_t RR, int64_t Nstore, int dir, rsvdt_stream_t s);
-/* (column, block) pairs of rsvdt_hip_horner_fused that the GPU's 256 CUs hold
- * at once for this operator (0: it does not fit). */
+/* (column, block) pairs of rsvdt_hip_horner_fused that the GPU's CUs hold at once
+ * for this operator (0: it does not fit). */
 int64_t rsvdt_hip_horner_fused_resident(int64_t nrows, int64_t nnz, int64_t maxrow, int a_real, int prec);
-/* The same from y = 0 with harmonic forcing, FP64: the forcing of step j of
+/* About how many us a step of it takes for `cols` such pairs, FP64 (0: it does not
+ * fit), and one rsvdt_hip_dense_apply of `cols` columns, k nb. */
+double rsvdt_hip_horner_fused_us(int64_t nrows, int64_t nnz, int64_t maxrow, int a_real, int64_t cols);
+double rsvdt_hip_dense_apply_us(int64_t N, int64_t cols);
+/* rsvdt_hip_horner_fused from y = 0 with harmonic forcing, FP64: the forcing of step j of
  * block m (d->nb blocks) is G_m exp(+-i phase), the phase that entry
  * (m, sgn*2j mod nt2) of the iDFT table idft ([nt2][d->nb]) holds times 2/nt2;
  * y (d->nb blocks) receives the state after nsteps steps, 2(nsteps-1) < nt2. */

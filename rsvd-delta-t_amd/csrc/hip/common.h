@@ -71,6 +71,9 @@ __device__ __forceinline__ int xcd_block(int bx, int nb, int mode)
 static inline hipStream_t as_stream(rsvdt_stream_t s) { return (hipStream_t)s; }
 static inline unsigned ceil_div(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
+// CUs of the current device (256 on an MI355X; also where there is no device).
+int device_cus();
+
 // The Horner stage on the tiled operator form (rsvdt_spmm_desc variant 9),
 // in tile.hip.
 int horner_tile(const rsvdt_spmm_desc *d, const void *vin, const void *y, const double *ys, const void *g, double c,

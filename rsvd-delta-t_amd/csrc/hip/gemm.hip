@@ -1180,6 +1180,19 @@ extern "C" int rsvdt_hip_bapply_gram(int64_t nbatch, int64_t nrows, int64_t n, c
     return RSVDT_HIP_OK;
 }
 
+// Measured products, one after another on a stream (N = 32 .. 1860, 1 to 650
+// columns): 5 us up to 200 rows, a launch; then 4 rows a workgroup 6.8 us at 500,
+// 12.5 at 1000; 16 rows 8.1 us at 500, 14 at 1000, 24 at 1860 for each round of as
+// many workgroups as CUs, and 11, 19, 35 us with two column tiles.
+extern "C" double rsvdt_hip_dense_apply_us(int64_t N, int64_t cols)
+{
+    const double n = (double)N, least = 5.0;
+    if (cols <= 16 && N <= 1024) return n < 240 ? least : 2.5 + 0.0105 * n;
+    const int64_t ct = cols <= 256 ? 16 : 32, wg = ((N + 15) / 16) * ((cols + ct - 1) / ct), cus = device_cus();
+    const double one = cols <= 256 ? 2.0 + 0.012 * n : 2.0 + 0.018 * n;
+    return (one < least ? least : one) * (double)((wg + cus - 1) / cus);
+}
+
 extern "C" int rsvdt_hip_dense_apply(int64_t N, int64_t k, int64_t nb, const double *E, const double *X,
                                      const double *F, double *Out, rsvdt_stream_t s)
 {

@@ -1050,7 +1050,25 @@ extern "C" int64_t rsvdt_hip_horner_fused_resident(int64_t nrows, int64_t nnz, i
     const size_t lds = reg ? (size_t)3 * (size_t)nrows * (prec == 64 ? 16 : 8) : fused_layout(nrows, nnz, a_real, prec).total;
     const int64_t by_lds = (int64_t)(RSVDT_FUSED_LDS / (lds + 256)), by_waves = reg ? 4 : 8;
     const int64_t per = by_lds < by_waves ? by_lds : by_waves;
-    return 256 * (per < 1 ? 1 : per);
+    return device_cus() * (per < 1 ? 1 : per);
+}
+
+// Measured steps (N = 20 .. 1860, 1 to 27 nonzeros a row, real and complex, 1 to N
+// columns): registers 0.5 us at 32 rows to 1.4 us at 1000 for a real operator, 0.7
+// to 1.8 us for a complex one; otherwise 256 rows at a time of 1.0 us with one
+// nonzero a row, 2.1 with five, 8 with 27.  Columns beyond what is resident go in
+// rounds; in registers, four columns a CU slow each other (N = 700: 1.0 us with
+// 256 columns, 2.3 with 700).
+extern "C" double rsvdt_hip_horner_fused_us(int64_t nrows, int64_t nnz, int64_t maxrow, int a_real, int64_t cols)
+{
+    const int64_t res = rsvdt_hip_horner_fused_resident(nrows, nnz, maxrow, a_real, 64);
+    if (res <= 0) return 0;
+    const double N = (double)nrows, rounds = (double)((cols + res - 1) / res);
+    if (maxrow >= 0 && maxrow <= 4 && nrows <= 1024) {
+        const double shared = 0.8 * (double)cols / device_cus();
+        return (shared > rounds ? shared : rounds) * (a_real ? 0.45 + 0.001 * N : 0.7 + 0.0013 * N);
+    }
+    return rounds * (double)((nrows + 255) / 256) * (0.8 + 0.3 * (double)maxrow);
 }
 
 static int launch_fused(const rsvdt_spmm_desc *d, int64_t nnz, int64_t maxrow, void *y, const void *g, int64_t gstride,

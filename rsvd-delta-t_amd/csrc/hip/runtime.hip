@@ -76,6 +76,18 @@ void cache_release_locked() {
 }
 }  // namespace
 
+namespace rsvdt {
+int device_cus() {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) {
+        (void)hipGetLastError();
+        n = 256;
+    }
+    return n;
+}
+}  // namespace rsvdt
+
 extern "C" int rsvdt_hip_malloc(void **p, size_t bytes) {
     *p = nullptr;
     const size_t r = round_alloc(bytes ? bytes : 256);

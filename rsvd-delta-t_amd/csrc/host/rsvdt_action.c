@@ -683,30 +683,62 @@ static PetscErrorCode step_range(stepper *st, Mat A, RSVDt_vars *V, Mat Yall, Pe
  * same recursion, rounded in another order; the Nt % RR first steps run one
  * by one.
  *
- * It pays when the steps it needs, in rounds of resident columns, are well
- * below the steps of the state, counting a product as 5 steps (a step takes
- * 1.1 us, a product and its launch about 5): with N = 500, k = 10, Nw = 64,
- * RR = 64 an action's stepping takes 0.84 ms (H 0.17, 70 products 0.57, samples
- * 0.1) and E 0.11 ms once; step by step it took 5.1 ms. */
+ * It is taken when the steps it needs, in rounds of resident columns, are well
+ * below the steps of the state (a product counted as 5 steps), so that E and H
+ * stay small beside the action, and when, by the measured times of a step, a
+ * product and a forcing term, it is not the slower way: with few steps between
+ * snapshots (RR below about 10) on operators whose steps take 0.5 to 1.5 us, 64
+ * products of 5 to 13 us cost more than 64 RR steps.  Of 600 actions of random
+ * sizes (N = 20 to 1860, k to 128, RR = 3 to 100) and 300 picked near the line,
+ * timed both ways, 573 leap: one of these is 4 % slower (8 % in the operator's
+ * first action), the others at most 3 %; with the first condition alone six of
+ * them are, by up to 8 %.  E's build counts always, so that the
+ * first action of an operator and the later ones go the same way.  N = 500, k =
+ * 10, Nw = 64, RR = 64: an action's stepping takes 0.78 ms (H 0.17, 70 products
+ * 0.46, forcing terms 0.1) and E 0.11 ms once; step by step it took 5.1 ms. */
 static PetscInt fused_rounds(Mat A, int dir, PetscInt cols)
 {
     const int64_t res = rsvdt_hip_horner_fused_resident(A->rows, A->nnz, dir ? A->maxrow : A->maxrowH, A->is_real, 64);
     return res > 0 ? (PetscInt)((cols + res - 1) / res) : 0;
 }
 
+/* us of one step of cols columns */
+static double step_us(Mat A, int dir, PetscInt cols)
+{
+    return rsvdt_hip_horner_fused_us(A->rows, A->nnz, dir ? A->maxrow : A->maxrowH, A->is_real, cols);
+}
+
 static int leap_pays(Mat A, int dir, RSVDt_vars *V)
 {
-    const PetscInt Nw = V->RSVD.Nw, RR = V->TS.ResRatio, Nt = V->TS.Nt, k = V->RSVD.k;
+    const PetscInt Nw = V->RSVD.Nw, Nwe = V->RSVD.Nw_eff, RR = V->TS.ResRatio, Nt = V->TS.Nt, k = V->RSVD.k;
     if (g_rsvdt.opt.precision != 64 || g_rsvdt.opt.rk4_form || !g_rsvdt.opt.fuse_small || RR < 2 || Nt < 0 ||
         V->TS.Ns != Nw * RR || A->rows > 16384)
         return 0;
     const PetscInt rk = fused_rounds(A, dir, k);
     if (!rk) return 0;
-    const PetscInt nleap = Nt / RR + Nw + (V->TS.TransientRemoval ? 1 : 0);
-    const double one_by_one = (double)(nleap * RR + Nt % RR) * (double)rk;
-    const double leaps = (double)RR * (double)(fused_rounds(A, dir, A->rows) + fused_rounds(A, dir, V->RSVD.Nw_eff * k)) +
-                         (double)(Nt % RR) * (double)rk + 5.0 * (double)nleap;
-    return leaps < 0.7 * one_by_one;
+    const PetscInt nleap = Nt / RR + Nw + (V->TS.TransientRemoval ? 1 : 0), lead = Nt % RR, nstep = nleap * RR + lead;
+    const double one_by_one = (double)nstep * (double)rk;
+    const double leaps = (double)RR * (double)(fused_rounds(A, dir, A->rows) + fused_rounds(A, dir, Nwe * k)) +
+                         (double)lead * (double)rk + 5.0 * (double)nleap;
+    if (leaps >= 0.7 * one_by_one) return 0;
+    /* a forcing term: its bytes at 1.3 TB/s and 8 Nwe operations an entry at 40
+     * TFLOP/s; chunks of steps and their events 40 us; a step with harmonic
+     * forcing 1.3 times one without */
+    const double sk = step_us(A, dir, k), term = (double)A->rows * (double)k * (1.2e-5 + 2e-7 * (double)Nwe);
+    const double steps_us = 40.0 + (double)nstep * (sk + term);
+    const double leaps_us = (double)RR * (step_us(A, dir, A->rows) + 1.3 * step_us(A, dir, Nwe * k)) + (double)lead * sk +
+                            (double)nleap * (rsvdt_hip_dense_apply_us(A->rows, k) + term);
+    return leaps_us < steps_us;
+}
+
+/* e^{A dT} of cols basis columns as one product with E, where the action leaps:
+ * its work grows with N^2, that of the RR steps (and two transposes) with N.
+ * N = 500, RR = 64, 650 columns: 32 us, 140 us in steps; N = 1024, RR = 11, 2176
+ * columns: 0.35 ms, 0.2 ms in steps. */
+static int leap_basis_pays(Mat A, int dir, RSVDt_vars *V, PetscInt cols)
+{
+    return cols <= 65535 * 16 && leap_pays(A, dir, V) &&
+           rsvdt_hip_dense_apply_us(A->rows, cols) < 20.0 + 1.2 * (double)V->TS.ResRatio * step_us(A, dir, cols);
 }
 
 /* E of A (dir 1) or A^H: nsteps homogeneous steps of the identity.  *out is NULL
@@ -1286,7 +1318,8 @@ static PetscErrorCode mtilde_group(LNS_vars *LNS, RSVDt_vars *V, TS_removal_matr
     /* the operator's dense propagator (the stepping of the same action built it)
      * on the basis as it lies, N x Ns1 per test vector */
     const double *E = NULL;
-    if (leap_pays(LNS->A, dir, V)) RSVDT_CHK(leap_operator(LNS->A, dir, V->TS.dt, V->TS.ResRatio, &E));
+    if (leap_basis_pays(LNS->A, dir, V, Ns1 * g))
+        RSVDT_CHK(leap_operator(LNS->A, dir, V->TS.dt, V->TS.ResRatio, &E));
     if (E) {
         h = rsvdt_hip_dense_apply(N, Ns1, g, E, g_trg.V, NULL, MV, g_rsvdt.stream);
         trt_add(TRT_STEPS, t0);

@@ -82,5 +82,54 @@ def test_steps_without_room_to_leap(tmp_path, what, removal):
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
 
 
+def action(pkg, A, removal=False, fuse=1, F=None, **kw):
+    s = pkg.Session(A, transient_removal=removal, fuse_small=fuse, q=0, w=0.7, **kw)
+    if F is None:
+        F = crandn(np.random.default_rng(1), A.shape[0], s.k * s.Nw_eff)
+    s.set_sketch(F)
+    s.direct()
+    out, st = s.get_Y(), pkg.action_stats()
+    leapt = st["chunk_steps"] == s.RR and st["rk4_launches"] < st["steps"]
+    s.close()
+    return out, F, leapt
+
+
+def steps(n):
+    """The step size of n steps a period, at w = 0.7."""
+    return 2 * np.pi / 0.7 / n
+
+
+@pytest.mark.parametrize("N,real,k,Nw,RR,leaps", [
+    (64, True, 1, 64, 8, False),         # 64 products of 5 us, 512 steps of 0.5 us
+    (1024, True, 10, 64, 8, False),      # 13 us, 1.5 us
+    (600, True, 100, 16, 6, False),
+    (64, True, 1, 64, 24, True),
+    (500, False, 10, 64, 16, True),
+    (1100, False, 10, 16, 32, True),     # rows beyond the stepper's registers
+    (1300, True, 33, 32, 24, True),
+])
+def test_leap_rule(pkg, N, real, k, Nw, RR, leaps):
+    """Leaps where products cost less than steps, steps where they do not; both
+    give the stage kernels' result."""
+    A = operator(N, real)
+    kw = dict(k=k, Nw=Nw, TL=0.0, dt=steps(Nw * RR) * 1.0001)
+    out, F, leapt = action(pkg, A, **kw)
+    assert leapt == leaps
+    ref, _, _ = action(pkg, A, fuse=0, F=F, **kw)
+    assert rel(out, ref) < 1e-12
+
+
+@pytest.mark.parametrize("N,k,Nw,RR", [(1024, 64, 16, 12), (500, 10, 16, 32), (1100, 3, 16, 32)])
+def test_leap_rule_removal(pkg, N, k, Nw, RR):
+    """The removal's e^{A dT} of a leaping action: as products of the whole basis
+    (the second) or, where these cost more, as steps."""
+    A = operator(N, True)
+    kw = dict(k=k, Nw=Nw, TL=1.0, dt=steps(Nw * RR) * 1.0001)
+    out, F, leapt = action(pkg, A, removal=True, **kw)
+    assert leapt
+    ref, _, _ = action(pkg, A, removal=True, fuse=0, F=F, **kw)
+    assert rel(out, ref) < 1e-9
+
+
 if __name__ == "__main__":
     refusing(sys.argv[1], sys.argv[2], bool(int(sys.argv[3])))
