@@ -78,11 +78,18 @@ void cache_release_locked() {
 
 namespace rsvdt {
 int device_cus() {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) {
+    static thread_local int of = -1, n = 256;     // asked once a device: rules ask dozens of times an action
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) {
         (void)hipGetLastError();
-        n = 256;
+        return 256;
+    }
+    if (dev != of) {
+        of = dev;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) {
+            (void)hipGetLastError();
+            n = 256;
+        }
     }
     return n;
 }
