@@ -683,19 +683,20 @@ static PetscErrorCode step_range(stepper *st, Mat A, RSVDt_vars *V, Mat Yall, Pe
  * same recursion, rounded in another order; the Nt % RR first steps run one
  * by one.
  *
- * It is taken when the steps it needs, in rounds of resident columns, are well
- * below the steps of the state (a product counted as 5 steps), so that E and H
- * stay small beside the action, and when, by the measured times of a step, a
- * product and a forcing term, it is not the slower way: with few steps between
- * snapshots (RR below about 10) on operators whose steps take 0.5 to 1.5 us, 64
- * products of 5 to 13 us cost more than 64 RR steps.  Of 600 actions of random
- * sizes (N = 20 to 1860, k to 128, RR = 3 to 100) and 300 picked near the line,
- * timed both ways, 573 leap: one of these is 4 % slower (8 % in the operator's
- * first action), the others at most 3 %; with the first condition alone six of
- * them are, by up to 8 %.  E's build counts always, so that the
- * first action of an operator and the later ones go the same way.  N = 500, k =
- * 10, Nw = 64, RR = 64: an action's stepping takes 0.78 ms (H 0.17, 70 products
- * 0.46, forcing terms 0.1) and E 0.11 ms once; step by step it took 5.1 ms. */
+ * It is taken, unless the caller has set the steps of a chunk, when the steps
+ * it needs, in rounds of resident columns, are well below the steps of the
+ * state (a product counted as 5 steps), so that E and H stay small beside the
+ * action, and when, by the measured times of a step, a product and a forcing
+ * term, it is not the slower way: with few steps between snapshots (RR below
+ * about 10) on operators whose steps take 0.5 to 1.5 us, 64 products of 5 to 13
+ * us cost more than 64 RR steps.  Of 600 actions of random sizes (N = 20 to
+ * 1860, k to 128, RR = 3 to 100) and 300 picked near the line, timed both ways,
+ * 573 leap: one of these is 4 % slower (8 % in the operator's first action), the
+ * others at most 3 %; with the first condition alone six of them are, by up to
+ * 8 %.  E's build counts always, so that the first action of an operator and the
+ * later ones go the same way.  N = 500, k = 10, Nw = 64, RR = 64: an action's
+ * stepping takes 0.78 ms (H 0.17, 70 products 0.46, forcing terms 0.1) and E
+ * 0.11 ms once; step by step it took 5.1 ms. */
 static PetscInt fused_rounds(Mat A, int dir, PetscInt cols)
 {
     const int64_t res = rsvdt_hip_horner_fused_resident(A->rows, A->nnz, dir ? A->maxrow : A->maxrowH, A->is_real, 64);
@@ -711,8 +712,8 @@ static double step_us(Mat A, int dir, PetscInt cols)
 static int leap_pays(Mat A, int dir, RSVDt_vars *V)
 {
     const PetscInt Nw = V->RSVD.Nw, Nwe = V->RSVD.Nw_eff, RR = V->TS.ResRatio, Nt = V->TS.Nt, k = V->RSVD.k;
-    if (g_rsvdt.opt.precision != 64 || g_rsvdt.opt.rk4_form || !g_rsvdt.opt.fuse_small || RR < 2 || Nt < 0 ||
-        V->TS.Ns != Nw * RR || A->rows > 16384)
+    if (g_rsvdt.opt.precision != 64 || g_rsvdt.opt.rk4_form || !g_rsvdt.opt.fuse_small || g_rsvdt.opt.chunk_steps > 0 ||
+        RR < 2 || Nt < 0 || V->TS.Ns != Nw * RR || A->rows > 16384)
         return 0;
     const PetscInt rk = fused_rounds(A, dir, k);
     if (!rk) return 0;

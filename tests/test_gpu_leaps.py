@@ -131,5 +131,16 @@ def test_leap_rule_removal(pkg, N, k, Nw, RR):
     assert rel(out, ref) < 1e-9
 
 
+def test_chunk_option(pkg):
+    """Chunks of a size the caller sets are chunks of steps."""
+    A = operator(64, True)
+    kw = dict(k=3, Nw=16, TL=1.0, dt=0.04)
+    ref, F, leapt = action(pkg, A, **kw)
+    assert leapt
+    out, _, leapt = action(pkg, A, F=F, chunk_steps=7, **kw)
+    assert not leapt and pkg.action_stats()["chunk_steps"] == 7
+    assert rel(out, ref) < 1e-12
+
+
 if __name__ == "__main__":
     refusing(sys.argv[1], sys.argv[2], bool(int(sys.argv[3])))
