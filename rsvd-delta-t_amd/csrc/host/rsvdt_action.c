@@ -886,6 +886,11 @@ static PetscErrorCode time_stepping(Mat A, DFT_matrices *D, RSVDt_vars *V, Mat F
         g_rsvdt.stats.steps = rend;
         g_rsvdt.stats.rk4_launches = launches;
         g_rsvdt.stats.chunk_steps = (int)V->TS.ResRatio;
+        rsvdt_spmm_desc d;                   /* the stepper's shape, as for chunks of steps */
+        desc_for(&d, A, dir, 64, k, 1);
+        g_rsvdt.stats.spmm_lanes = d.lanes;
+        g_rsvdt.stats.spmm_variant = d.variant;
+        g_rsvdt.stats.spmm_xcd_remap = d.xcd_remap;
         return 0;
     }
     double *y64 = NULL;          /* the FP32 state at step Nt, widened */

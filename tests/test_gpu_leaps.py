@@ -142,5 +142,18 @@ def test_chunk_option(pkg):
     assert rel(out, ref) < 1e-12
 
 
+def test_stats_name_the_shape(pkg):
+    """The launch shape that the statistics name does not depend on the way."""
+    A = operator(64, True)
+    kw = dict(k=3, Nw=16, TL=1.0, dt=0.04)
+    shape = {}
+    for chunk in (0, 7):
+        _, _, leapt = action(pkg, A, chunk_steps=chunk, **kw)
+        assert leapt == (chunk == 0)
+        st = pkg.action_stats()
+        shape[chunk] = [st[f] for f in ("spmm_lanes", "spmm_variant", "spmm_xcd_remap", "rk4_form")]
+    assert shape[0] == shape[7] and shape[7][1:3] == [3, 1]
+
+
 if __name__ == "__main__":
     refusing(sys.argv[1], sys.argv[2], bool(int(sys.argv[3])))
