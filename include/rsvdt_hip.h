@@ -102,7 +102,8 @@ typedef struct {
     int lanes;            /* 0 = default choice */
     int xcd_remap;        /* workgroup -> rows map: 0 identity, 1 one contiguous row range per XCD,
                              2 / 3 chunks of 64 / 256 row blocks dealt round-robin to the XCDs
-                             (one block; with several the tiled forms choose by their tiles) */
+                             (as given for one block, or where a workgroup of the tiled form takes
+                             all blocks of its tile; else rsvdt_hip_tile_map chooses) */
     int variant;          /* 0: 16-nonzero gather batches; 1: + nontemporal row-local
                              streams; 2: 8-nonzero batches; 3: 8 + nontemporal; 4: 12-nonzero
                              batches; 5: 12 + nontemporal (variants 1-3 apply to the RK4 stage
@@ -161,6 +162,9 @@ int rsvdt_hip_rk4_stage(const rsvdt_spmm_desc *d, int stage,
  * the launch shape as for rsvdt_hip_rk4_stage. */
 int rsvdt_hip_horner_stage(const rsvdt_spmm_desc *d, const void *vin, const void *y, const double *yscale,
                            const void *g, double c, void *out, double *snap, rsvdt_stream_t s);
+/* The map (xcd_remap's values) that the tiled form takes for ntiles tiles of nb
+ * blocks, bpw of them a workgroup, when the descriptor asks for xcd_remap. */
+int rsvdt_hip_tile_map(int64_t nb, int64_t bpw, int64_t ntiles, int xcd_remap);
 /* As rsvdt_hip_horner_stage, with the snapshot destination read at run time:
  * when snap_slot is not NULL, the kernel reads the int *snap_slot and writes
  * the copy of out to snap + slot*snap_stride (complex entries) when slot >= 0,

@@ -243,14 +243,7 @@ static int launch_tile(const rsvdt_spmm_desc *d, const void *vin, const void *y,
     const int bpw = d->tile_bpw > 1 ? d->tile_bpw : 1;
     const unsigned gx = ceil_div(d->nrows, TR);
     const unsigned gy = ceil_div(d->nb, bpw);
-    int remap = (d->xcd_remap > 0 && d->xcd_remap <= 3 && gy == 1 && gx >= 8) ? d->xcd_remap : 0;
-    // Several blocks: bound by what the L2s miss.  With neighbouring tiles on
-    // eight XCDs every L2 reads the rows that tiles share (14.7 GB a stage,
-    // 7.2 TB/s, where 6.1 GB is needed: 65 blocks of 245,760 x 8 on the 3D
-    // operator).  Runs of 64 tiles per XCD: 15.6 -> 11.7 ms for 8 stages (runs
-    // of 256: 12.3, one run per XCD: 14.6); below 512 tiles, where such runs
-    // do not reach all XCDs, one run each.
-    if (d->nb > 1 && gx >= 64) remap = gx >= 512 ? 2 : 1;
+    const int remap = rsvdt_hip_tile_map(d->nb, bpw, gx, d->xcd_remap);
     hipLaunchKernelGGL((k_horner_tile<T, AREAL, KC, RPT, PF ? 6 : 8, PF>), dim3(gx, gy), dim3(256), lay.total, s,
                        (int)d->nrows, (int)d->k, (int)d->nb, bpw, d->tile_hmax, d->tile_emax, remap,
                        d->nrows * d->k, d->rowptr,
@@ -304,3 +297,17 @@ int horner_tile(const rsvdt_spmm_desc *d, const void *vin, const void *y, const 
 }
 
 }  // namespace rsvdt
+
+// Workgroup -> tile map.  The caller's where one workgroup forms all blocks of a
+// tile.  Otherwise, several blocks are bound by what the L2s miss: with
+// neighbouring tiles on eight XCDs every L2 reads the rows that tiles share (14.7
+// GB a stage, 7.2 TB/s, where 6.1 GB is needed: 65 blocks of 245,760 x 8 on the 3D
+// operator).  Runs of 64 tiles per XCD: 15.6 -> 11.7 ms for 8 stages (runs of 256:
+// 12.3, one run per XCD: 14.6); below 512 tiles, where such runs do not reach all
+// XCDs, one run each.
+extern "C" int rsvdt_hip_tile_map(int64_t nb, int64_t bpw, int64_t ntiles, int xcd_remap)
+{
+    if (xcd_remap > 0 && xcd_remap <= 3 && (nb <= 1 || bpw >= nb) && ntiles >= 8) return xcd_remap;
+    if (nb > 1 && ntiles >= 64) return ntiles >= 512 ? 2 : 1;
+    return 0;
+}
