@@ -155,5 +155,28 @@ def test_stats_name_the_shape(pkg):
     assert shape[0] == shape[7] and shape[7][1:3] == [3, 1]
 
 
+@pytest.mark.parametrize("direct", [True, False])
+def test_propagator_follows_the_steps(pkg, direct):
+    """One Mat stepped with one step size, another, another number of steps and the
+    first again: the kept propagator is the one of the call."""
+    A = operator(200, False)
+    first = pkg.Session(A, q=0, w=0.7, transient_removal=False, k=4, Nw=16, TL=1.0, dt=0.04)
+    for Nw, dt in ((16, 0.04), (16, 0.02), (8, 0.02), (16, 0.04)):
+        kw = dict(q=0, w=0.7, transient_removal=False, k=4, Nw=Nw, TL=1.0, dt=dt)
+        s = pkg.Session(A, **kw)
+        own, s.LNS.A = s.LNS.A, first.LNS.A
+        F = crandn(np.random.default_rng(Nw), 200, 4 * s.Nw_eff)
+        s.set_sketch(F)
+        s.direct() if direct else s.adjoint()
+        out = s.get_Y()
+        assert pkg.action_stats()["rk4_launches"] < s.Ns // 4
+        s.LNS.A = own
+        s.set_sketch(F)
+        s.direct() if direct else s.adjoint()
+        assert np.array_equal(out, s.get_Y())      # a Mat of its own: the same kernels, the same bits
+        s.close()
+    first.close()
+
+
 if __name__ == "__main__":
     refusing(sys.argv[1], sys.argv[2], bool(int(sys.argv[3])))

@@ -200,3 +200,115 @@ def test_spmm_blocks_wide(L, pkg, rows, k, nb):
         assert np.max(np.abs(got[b] - M @ x[b])) <= 4 * 7 * EPS * 36      # sums of 7 products of |.| < 6 each
         assert L.rsvdt_hip_spmm_blocks(rows, k, 1, *p, at(dx, b * rows * k * 16), rows * k, one.p, rows * k, None) == 0
         assert np.array_equal(got[b], one.get(np.complex128, (rows, k)))
+
+
+@pytest.mark.parametrize("rows,nb", [(4096, 8), (4096, 13), (4096, 33), (9000, 11), (70000, 17)])
+def test_spmm_blocks_groups(L, pkg, rows, nb):
+    """Two, three and eight blocks a workgroup, in groups of two and four that do
+    not fill, entries walked again for each group, and outputs beyond the
+    last-level cache (the last): every block the same bits as the block alone."""
+    k = 16
+    rng = np.random.default_rng(rows + nb)
+    cnt = rng.integers(0, 6, rows)
+    rp = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32)
+    ci = rng.integers(0, rows, rp[-1]).astype(np.int32)
+    v, x = crandn(rng, len(ci)), crandn(rng, nb, rows, k)
+    held = [Dev(pkg, a) for a in (rp, ci, v)]
+    dx, out, one = Dev(pkg, x), Dev(pkg, np.full((nb, rows, k), np.nan + 0j)), Dev(pkg, nbytes=rows * k * 16)
+    L.rsvdt_hip_spmm_blocks.argtypes = [I64] * 3 + [V, V, V, V, I64, V, I64, V]
+    p = [h.p for h in held]
+    assert L.rsvdt_hip_spmm_blocks(rows, k, nb, *p, dx.p, rows * k, out.p, rows * k, None) == 0
+    got = out.get(np.complex128, (nb, rows, k))
+    M = sp.csr_matrix((v, ci, rp), shape=(rows, rows))
+    for b in range(nb):
+        assert L.rsvdt_hip_spmm_blocks(rows, k, 1, *p, at(dx, b * rows * k * 16), rows * k, one.p, rows * k, None) == 0
+        assert np.array_equal(got[b], one.get(np.complex128, (rows, k)))
+    assert np.max(np.abs(got[-1] - M @ x[-1])) <= 4 * 5 * EPS * 36
+
+
+def test_transpose_beyond_cache(L, pkg):
+    """Nontemporal row transposes, 290 MB a side, both ways."""
+    N, n, kt, b0, kb = 35000, 65, 9, 1, 8
+    rng = np.random.default_rng(3)
+    src = rng.standard_normal((n, N, kt)) + 0j
+    dS, dD, dB = Dev(pkg, src), Dev(pkg, nbytes=kb * N * n * 16), Dev(pkg, np.zeros_like(src))
+    L.rsvdt_hip_transpose_rows.argtypes = [I64] * 5 + [V, V, ctypes.c_int, V]
+    assert L.rsvdt_hip_transpose_rows(N, n, kt, b0, kb, dS.p, dD.p, 0, None) == 0
+    assert np.array_equal(dD.get(np.complex128, (kb, N, n)), src[:, :, b0:].transpose(2, 1, 0))
+    assert L.rsvdt_hip_transpose_rows(N, n, kt, b0, kb, dD.p, dB.p, 1, None) == 0
+    src[:, :, 0] = 0
+    assert np.array_equal(dB.get(np.complex128, src.shape), src)
+
+
+@pytest.mark.parametrize("in_place", [False, True])
+def test_apply_gram_beyond_cache(L, pkg, in_place):
+    """Nontemporal rows of a CholeskyQR pass: 300 MB."""
+    nb, nr, n = 2, 290001, 33
+    rng = np.random.default_rng(4)
+    X, C = crandn(rng, nb, nr, n), np.triu(crandn(rng, nb, n, n)) / np.sqrt(n)
+    L.rsvdt_hip_bgram_work_bytes.restype = ctypes.c_size_t
+    L.rsvdt_hip_bgram_work_bytes.argtypes = [I64] * 4
+    L.rsvdt_hip_bapply_gram.argtypes = [I64] * 3 + [V, I64, I64, V, V, V, V, V]
+    dX, dC, dG = Dev(pkg, X), Dev(pkg, C), Dev(pkg, nbytes=C.nbytes)
+    dO = dX if in_place else Dev(pkg, nbytes=X.nbytes)
+    dw = Dev(pkg, nbytes=L.rsvdt_hip_bgram_work_bytes(nb, nr, n, n))
+    assert L.rsvdt_hip_bapply_gram(nb, nr, n, dX.p, nr * n, n, dC.p, dO.p, dG.p, dw.p, None) == 0
+    out, G, ref = dO.get(np.complex128, X.shape), dG.get(np.complex128, C.shape), X @ C
+    assert np.max(np.abs(out - ref)) <= 8 * EPS * n * np.abs(X).max() * np.abs(C).max()
+    assert np.max(np.abs(G - ref.conj().transpose(0, 2, 1) @ ref)) <= 16 * EPS * nr * np.abs(ref).max() ** 2
+
+
+class QrWork(ctypes.Structure):
+    _fields_ = [(f, V) for f in ("G", "R", "Ri", "Ra", "Rt", "work", "info")]
+
+
+@pytest.mark.parametrize("npass", [1, 2, 3])
+@pytest.mark.parametrize("n", [16, 33, 64, 65])
+def test_cholqr_from_another_array(L, pkg, n, npass):
+    """CholeskyQR passes that start from an array of their own and end in X after
+    odd and even numbers, with the product of their factors."""
+    nb, nr = 2, 700
+    rng = np.random.default_rng(n)
+    X0 = crandn(rng, nb, nr, n)
+    L.rsvdt_hip_bgram_work_bytes.restype = ctypes.c_size_t
+    L.rsvdt_hip_bgram_work_bytes.argtypes = [I64] * 4
+    mat = nb * n * n * 16
+    d0, dX, dT, dR = Dev(pkg, X0), Dev(pkg, nbytes=X0.nbytes), Dev(pkg, nbytes=X0.nbytes), Dev(pkg, nbytes=mat)
+    held = [Dev(pkg, nbytes=mat) for _ in range(5)] + [Dev(pkg, nbytes=L.rsvdt_hip_bgram_work_bytes(nb, nr, n, n)),
+                                                       Dev(pkg, nbytes=256)]
+    w = QrWork(*[h.p for h in held])
+    f = L.rsvdt_cholqr_bufs
+    f.argtypes = [I64] * 3 + [V, V, I64, I64, I64, V, ctypes.c_int, ctypes.c_int, ctypes.c_double, V, ctypes.c_size_t,
+                              V, V, ctypes.c_int]
+    assert f(nb, nr, n, d0.p, dX.p, nr * n, n, 1, dR.p, npass, 0, 0.0, dT.p, X0.nbytes, ctypes.byref(w), None, 0) == 0
+    Q, R = dX.get(np.complex128, X0.shape), dR.get(np.complex128, (nb, n, n))
+    assert np.array_equal(d0.get(np.complex128, X0.shape), X0)
+    cond = max(np.linalg.cond(X0[b]) for b in range(nb))
+    for b in range(nb):
+        # one pass of CholeskyQR loses cond^2, two are at rounding
+        assert np.max(np.abs(Q[b].conj().T @ Q[b] - np.eye(n))) <= 8 * n * EPS * (cond ** 2 if npass == 1 else 8)
+        assert np.max(np.abs(Q[b] @ R[b] - X0[b])) <= 8 * n * EPS * np.linalg.norm(X0[b], 2) * 4
+        assert np.all(np.tril(R[b], -1) == 0) and np.all(np.diag(R[b]).real > 0)
+
+
+@pytest.mark.parametrize("n,drop", [(17, 3), (33, 5), (64, 9), (65, 9)])
+def test_basis_of_dependent_columns(pkg, n, drop):
+    """QRDecomposition of dependent columns (the second level of the span basis):
+    orthonormal columns, zeros for what is left out, the span kept to rounding."""
+    nr = 900
+    rng = np.random.default_rng(n)
+    X = crandn(rng, nr, n)
+    where = rng.choice(n - 1, drop, replace=False) + 1
+    for c in where:
+        X[:, c] = X[:, :c] @ crandn(rng, c) / np.sqrt(c)
+    m = pkg.mat_from_dense(np.asfortranarray(X), n)
+    f = pkg.lib().QRDecomposition
+    f.argtypes = [V]
+    assert f(m) == 0
+    Q = pkg.mat_to_dense(m)
+    pkg.destroy(m)
+    G = Q.conj().T @ Q
+    live = np.diag(G).real > 0.5
+    assert n - drop <= live.sum() <= n
+    assert np.max(np.abs(G - np.diag(live.astype(float)))) <= 64 * n * EPS
+    assert np.linalg.norm(X - Q @ (Q.conj().T @ X)) <= 64 * n * EPS * np.linalg.norm(X)
