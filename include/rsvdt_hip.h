@@ -310,7 +310,7 @@ size_t rsvdt_qr_blocks_noalloc_bytes(int64_t nblocks, int64_t N, int64_t k);
 int rsvdt_qr_blocks_noalloc(double *Y, int64_t N, int64_t k, int64_t nblocks, rsvdt_stream_t s);
 
 /* ---- elementwise ------------------------------------------------------ */
-/* the n x n complex FP64 identity */
+/* the n x n complex FP64 identity, n < 65536 */
 int rsvdt_hip_identity(int64_t n, double *p, rsvdt_stream_t s);
 /* y = a*x (complex entries, FP64), n entries */
 int rsvdt_hip_zscale(int64_t n, double a, const double *x, double *y, rsvdt_stream_t s);

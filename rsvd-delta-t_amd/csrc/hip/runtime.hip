@@ -321,7 +321,7 @@ __global__ void k_identity(int64_t n, double2 *p) {
 }
 extern "C" int rsvdt_hip_identity(int64_t n, double *p, rsvdt_stream_t s) {
     if (n <= 0) return RSVDT_HIP_OK;
-    if (n > 65536) { set_error_msg("rsvdt_hip_identity: n <= 65536"); return RSVDT_HIP_ERR_ARG; }
+    if (n > 65535) { set_error_msg("rsvdt_hip_identity: n < 65536"); return RSVDT_HIP_ERR_ARG; }     // 2^32 threads
     hipLaunchKernelGGL(k_identity, dim3(ceil_div(n * n, 256)), dim3(256), 0, as_stream(s), n, (double2 *)p);
     RSVDT_LAUNCH_CHECK("rsvdt_hip_identity");
     return RSVDT_HIP_OK;

@@ -21,3 +21,11 @@ def test_tile_map(pkg, asked, nb, bpw, ntiles):
         assert got == (2 if ntiles >= 512 else 1)
     else:
         assert got == 0
+
+
+@pytest.mark.parametrize("n", [65536, 70000])
+def test_identity_beyond_one_launch(pkg, n):
+    """Refused before anything is launched: a launch has less than 2^32 threads."""
+    f = pkg.lib().rsvdt_hip_identity
+    f.argtypes = [I64, ctypes.c_void_p, ctypes.c_void_p]
+    assert f(n, None, None) == 102
