@@ -230,7 +230,8 @@ PetscErrorCode RSVDT_VecView(Vec v, const char *path);
 /* ---- engine controls (no counterpart in the reference) ------------------- */
 typedef struct {
     int precision;        /* 64: complex FP64 state (reference); 32: complex FP32 RK4 state and SpMM */
-    int chunk_steps;      /* RK4 steps per forcing chunk (0 = automatic) */
+    int chunk_steps;      /* RK4 steps per forcing chunk (0 = automatic: small operators may leap
+                             from snapshot to snapshot instead) */
     int spmm_lanes;       /* lanes per row in the SpMM (0 = automatic / autotuned) */
     int xcd_remap;        /* contiguous row ranges per XCD */
     int use_graph;        /* capture each forcing chunk's RK4 steps in a hipGraph */
@@ -254,8 +255,8 @@ typedef struct {
     double tr_ms;          /* transient removal total */
     double total_ms;       /* the whole action */
     int64_t steps;         /* RK4 steps taken */
-    int64_t rk4_launches;  /* RK4 stage launches */
-    int chunk_steps;       /* RK4 steps per forcing chunk */
+    int64_t rk4_launches;  /* launches that advance the state: stages, chunks or products */
+    int chunk_steps;       /* RK4 steps per forcing chunk, or per leap */
     int spmm_lanes, spmm_variant, spmm_xcd_remap;   /* SpMM launch shape used */
     int rk4_form;          /* stepping form used (RSVDT_Options.rk4_form) */
 } RSVDT_ActionStats;

@@ -63,8 +63,8 @@ __global__ __launch_bounds__(256) void k_coef_gemm(
     // streamed operand loaded PF steps ahead, across tile boundaries too; both
     // ends of the stream count steps and move pointers (finding a step's tile by
     // 64-bit division cost more vector instructions than all the rest).  Bound
-    // by the FP64 matrix cores: the 64 x 64 x 6.3M forcing chunk takes 3.78 ms
-    // (4.18 ms with divisions), 81 % of their cycles at the 2.05 GHz that this
+    // by the FP64 matrix cores: the 64 x 64 x 6.3M forcing chunk takes 3.6 to 3.8 ms
+    // (4.2 ms with divisions), 75 to 81 % of their cycles at the 2.05 GHz that this
     // load runs at; PF = 8, 12, 16: 3.87, 3.78, 3.82 ms.
     constexpr int PF = 12;
     const int nks = (int)(Kpad >> 2);
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(256) void k_bgram_reduce(int64_t nch, int na, int n
 //   * PF row steps are in flight per wave where the MFMAs of a step do not
 //     cover a load's latency; the loads are branch-free (clamped addresses,
 //     zeros selected afterwards).
-// 8 batches of 98,304 x 65 (V^H X of a removal): 508 us, 52 TFLOP/s (48 x 48
+// 8 batches of 98,304 x 65 (V^H X of a removal): 483 us, 55 TFLOP/s (48 x 48
 // tiles per wave, padded to 96 x 96: 1620 us).  16 batches of 393,216 x 16
 // (QR): 329 us, 4.9 TB/s, with nontemporal loads and 8 steps in flight; 351 us
 // without the hint, 377 us with one step in flight.  The launch bound keeps
@@ -569,9 +569,10 @@ __global__ __launch_bounds__(256) void k_bapply(
 // Out may alias X; Out may always alias Y (read and written by the same lane).
 // BORD: a last column beyond the 16-wide tiles (nc = 16 T + 1, the bases of
 // Nw + 1 snapshots) is a plain FMA sum on the operands the lanes hold.
-// Bound by memory and FP64 MFMA together at 32 columns (61 % of the cycles
-// hold an MFMA), by MFMA above.  8 batches of 98,304 x 65 times 65 x 32: 340 us,
-// with Y 372 us, 4.4 TB/s (413 and 520 us with one step in flight); PF = 8 is
+// Bound by memory and FP64 MFMA together at 32 columns (MFMAs busy in 51 to 55 % of
+// the cycles, 45 to 47 % with Y), by MFMA above.  8 batches of 98,304 x 65 times 65 x 32:
+// alone 340 us, with Y 372 us (413 and 520 us with one step in flight); in a
+// projection, after other kernels, 366 and 411 us, 3.3 and 3.9 TB/s.  PF = 8 is
 // slower (385 us), 16 x 16 chunks turned through LDS too (383 us).
 template <int TC, bool BORD>
 __global__ __launch_bounds__(256) void k_bapply_mfma(

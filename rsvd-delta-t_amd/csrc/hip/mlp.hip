@@ -145,7 +145,7 @@ __device__ __forceinline__ void gemm_put(__bf16 *__restrict__ S, const float (&v
 // part of both operands, are dealt to one XCD (f % 8), so that its L2 serves all
 // but the first: 16,000 x 256 x 256 read A four times over (64 MB; 96 MB for the
 // weight gradient).  Forward, weight and input gradients 19.6 + 19.4 + 21.9 ->
-// 16.5 + 17.4 + 19.9 us.  The groups past the last eight keep the plain order.
+// 16.2 + 16.9 + 18.8 us.  The groups past the last eight keep the plain order.
 struct gemm_tile {
     int m, n, s;
 };

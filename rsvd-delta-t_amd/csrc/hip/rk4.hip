@@ -1204,7 +1204,7 @@ extern "C" int rsvdt_hip_horner_stage(const rsvdt_spmm_desc *d, const void *vin,
 // or as many as there are), the row's first entries kept in registers over the
 // bpw blocks a workgroup forms.
 // 393,216 x 16, 8 blocks, 1 to 5 entries a row: 591 us one block and entry at
-// a time, 557 with six entries of one block in flight, 345 as here (4.8 TB/s;
+// a time, 557 with six entries of one block in flight, 325 as here (5.0 TB/s;
 // four blocks x three entries, two x three, eight x three: 1 %, 6 %, 18 % more).
 namespace rsvdt {
 template <bool NT, int BB>

@@ -303,8 +303,8 @@ int horner_tile(const rsvdt_spmm_desc *d, const void *vin, const void *y, const 
 // neighbouring tiles on eight XCDs every L2 reads the rows that tiles share (14.7
 // GB a stage, 7.2 TB/s, where 6.1 GB is needed: 65 blocks of 245,760 x 8 on the 3D
 // operator).  Runs of 64 tiles per XCD: 15.6 -> 11.7 ms for 8 stages (runs of 256:
-// 12.3, one run per XCD: 14.6); below 512 tiles, where such runs do not reach all
-// XCDs, one run each.
+// 12.3, one run per XCD: 14.6), the tiles past the last 512 as they come; below
+// 512, where such runs do not reach all XCDs, one run each.
 extern "C" int rsvdt_hip_tile_map(int64_t nb, int64_t bpw, int64_t ntiles, int xcd_remap)
 {
     if (xcd_remap > 0 && xcd_remap <= 3 && (nb <= 1 || bpw >= nb) && ntiles >= 8) return xcd_remap;

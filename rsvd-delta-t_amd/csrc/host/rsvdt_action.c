@@ -695,7 +695,7 @@ static PetscErrorCode step_range(stepper *st, Mat A, RSVDt_vars *V, Mat Yall, Pe
  * others at most 3 %; with the first condition alone six of them are, by up to
  * 8 %.  E's build counts always, so that the first action of an operator and the
  * later ones go the same way.  N = 500, k = 10, Nw = 64, RR = 64: an action's
- * stepping takes 0.78 ms (H 0.17, 70 products 0.46, forcing terms 0.1) and E
+ * stepping takes 0.8 ms (H 0.17, 70 products 0.49, forcing terms 0.1) and E
  * 0.11 ms once; step by step it took 5.1 ms. */
 static PetscInt fused_rounds(Mat A, int dir, PetscInt cols)
 {
