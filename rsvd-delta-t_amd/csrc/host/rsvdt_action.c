@@ -742,9 +742,10 @@ static int leap_basis_pays(Mat A, int dir, RSVDt_vars *V, PetscInt cols)
            rsvdt_hip_dense_apply_us(A->rows, cols) < 20.0 + 1.2 * (double)V->TS.ResRatio * step_us(A, dir, cols);
 }
 
-/* E of A (dir 1) or A^H: nsteps homogeneous steps of the identity.  *out is NULL
- * when there is no room for it: the caller steps one by one. */
-static PetscErrorCode leap_operator(Mat A, int dir, double h, PetscInt nsteps, const double **out)
+/* E of A (dir 1) or A^H: nsteps homogeneous steps of the identity, timed by t (may
+ * be NULL) where they are taken.  *out is NULL when there is no room for it: the
+ * caller steps one by one. */
+static PetscErrorCode leap_operator(Mat A, int dir, double h, PetscInt nsteps, phase_timer *t, const double **out)
 {
     const int q = dir ? 0 : 1;
     const PetscInt N = A->rows;
@@ -755,9 +756,11 @@ static PetscErrorCode leap_operator(Mat A, int dir, double h, PetscInt nsteps, c
         rsvdt_spmm_desc d;
         desc_for(&d, A, dir, 64, N, 1);
         const double cf[4] = {h / 4, h / 3, h / 2, h};
+        if (t) pt_begin(t);
         RSVDT_HIPCHK("TSActionRK4", rsvdt_hip_identity(N, A->leap[q].d, g_rsvdt.stream));
         RSVDT_HIPCHK("TSActionRK4", rsvdt_hip_horner_fused(&d, A->nnz, dir ? A->maxrow : A->maxrowH, A->leap[q].d, NULL, 0,
                                                            cf, nsteps, NULL, 0, 0, 0, 1, 1, dir, g_rsvdt.stream));
+        if (t) pt_end(t);
         A->leap[q].h = h;
         A->leap[q].steps = nsteps;
     }
@@ -781,11 +784,7 @@ static PetscErrorCode leap_reserve(Mat A, RSVDt_vars *V, leap_bufs *b, phase_tim
     b->y0 = b->H ? rsvdt_scratch(SCR_Y, blk) : NULL;
     b->y1 = b->y0 ? rsvdt_scratch(SCR_U1, blk) : NULL;
     b->f = b->y1 ? rsvdt_scratch(SCR_FBUF, blk * (size_t)(most < LEAP_CHUNK ? most : LEAP_CHUNK)) : NULL;
-    if (b->f) {
-        if (t_frc) pt_begin(t_frc);
-        RSVDT_CHK(leap_operator(A, V->TS.DirAdj ? 1 : 0, V->TS.dt, RR, &b->E));
-        if (t_frc) pt_end(t_frc);
-    }
+    if (b->f) RSVDT_CHK(leap_operator(A, V->TS.DirAdj ? 1 : 0, V->TS.dt, RR, t_frc, &b->E));
     if (!b->E) {
         rsvdt_scratch_release(SCR_H);
         rsvdt_scratch_release(SCR_FBUF);
@@ -1325,7 +1324,7 @@ static PetscErrorCode mtilde_group(LNS_vars *LNS, RSVDt_vars *V, TS_removal_matr
      * on the basis as it lies, N x Ns1 per test vector */
     const double *E = NULL;
     if (leap_basis_pays(LNS->A, dir, V, Ns1 * g))
-        RSVDT_CHK(leap_operator(LNS->A, dir, V->TS.dt, V->TS.ResRatio, &E));
+        RSVDT_CHK(leap_operator(LNS->A, dir, V->TS.dt, V->TS.ResRatio, NULL, &E));
     if (E) {
         h = rsvdt_hip_dense_apply(N, Ns1, g, E, g_trg.V, NULL, MV, g_rsvdt.stream);
         trt_add(TRT_STEPS, t0);
